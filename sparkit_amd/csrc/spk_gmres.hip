@@ -5,13 +5,13 @@
 //   r0 = b - A x (SpMV epilogue); GMRES: V0 = M_L r0; beta = |V0|
 //   Arnoldi step j:  Z_j = M_R V_j (GMRES) / M V_j (FGMRES)
 //                    V_{j+1} = M_L A Z_j (GMRES) / A Z_j (FGMRES)
-//                    modified Gram-Schmidt: j+1 fused kernels, kernel i
-//                    applies the update of V_{i-1} and reduces <V_i, V_{j+1}>
-//                    (so each MGS sweep streams V_{j+1} once per basis
-//                    vector, in the reference's order)
-//                    last kernel: update with V_j and |V_{j+1}|^2; its last
-//                    block runs the Givens rotations and the convergence test
-//                    on the device (FP64), then V_{j+1} is normalised
+//                    modified Gram-Schmidt and the normalisation: one
+//                    persistent kernel (mgs_step_kernel) up to 3.2M rows;
+//                    beyond, j+1 fused kernels, kernel i applies the update
+//                    of V_{i-1} and reduces <V_i, V_{j+1}>, a last one
+//                    updates with V_j and sums |V_{j+1}|^2, its finisher
+//                    runs the Givens rotations and the convergence test on
+//                    the device (FP64), then V_{j+1} is normalised
 //   form_solution:   back-substitution (one thread) and x += Z y
 // Optional orthogonalization SPK_ORTHO_CGS2 (classical Gram-Schmidt applied
 // twice): per step two passes of {all j+1 dot products in one launch (a
@@ -22,6 +22,7 @@
 // The host reads the state once per cycle.  Vectors may be FP32
 // (precision = SPK_F32); H, the rotations, g, y, every dot product and the
 // Gram-Schmidt updates are computed in FP64 and the basis is stored in T.
+#include "spk_link.hpp"
 #include "spk_solver_common.hpp"
 
 namespace spk {
@@ -36,6 +37,7 @@ struct GmState {
   int32_t collect;
   int32_t j_final;
   int32_t flexible;
+  int32_t expired;    // a grid exchange's bounded wait ended without its value
   double* history;
   double* H;  // (m+1) x m, column-major, leading dimension m+1
   double* cs;
@@ -45,16 +47,15 @@ struct GmState {
   int64_t m;
 };
 
-// apply_givens_rotations + residual record + convergence check
-// (gmres.hpp:283-326, 193-205; fgmres.hpp:286-356), thread 0 of the last
-// block of the final Gram-Schmidt kernel of step j.
-__device__ void arnoldi_finish(GmState* st, int j, double h) {
-  const int64_t ld = st->m + 1;
-  double* col = st->H + (int64_t)j * ld;
-  double* cs = st->cs;
-  double* sn = st->sn;
+// apply_givens_rotations + residual record + convergence check of step j
+// (gmres.hpp:283-326, 193-205; fgmres.hpp:286-356), one thread.  col[0..j]:
+// the new column, cs / sn: the earlier rotations (in LDS, or st's own
+// arrays); h = |V_{j+1}| before its normalisation.  The rotated column goes
+// to st->H.
+__device__ void arnoldi_finish(GmState* st, int j, double h, const double* col,
+                               const double* cs, const double* sn) {
+  double* H = st->H + (int64_t)j * (st->m + 1);
   double* g = st->g;
-  col[j + 1] = h;
   st->hnorm = h;
   // the earlier rotations in the reference's order; only the rotated
   // entry carries from one to the next, so each batch of eight loads its
@@ -75,36 +76,183 @@ __device__ void arnoldi_finish(GmState* st, int j, double h) {
       if (u < nb) {
         const double temp = c8[u] * ci + s8[u] * h8[u];
         ci = -s8[u] * ci + c8[u] * h8[u];
-        col[i0 + u] = temp;
+        H[i0 + u] = temp;
       }
   }
-  if (j > 0) col[j] = ci;
-  double a = col[j], b = col[j + 1];
-  if (b == 0.0) {
-    cs[j] = 1.0;
-    sn[j] = 0.0;
-  } else if (a == 0.0) {
-    cs[j] = 0.0;
-    sn[j] = 1.0;
+  double c, s;
+  if (h == 0.0) {
+    c = 1.0;
+    s = 0.0;
+  } else if (ci == 0.0) {
+    c = 0.0;
+    s = 1.0;
   } else {
-    double r = sqrt(a * a + b * b);
-    cs[j] = a / r;
-    sn[j] = b / r;
+    const double r = sqrt(ci * ci + h * h);
+    c = ci / r;
+    s = h / r;
   }
-  col[j] = cs[j] * col[j] + sn[j] * col[j + 1];
-  col[j + 1] = 0.0;
-  double temp = cs[j] * g[j] + sn[j] * g[j + 1];
-  g[j + 1] = -sn[j] * g[j] + cs[j] * g[j + 1];
-  g[j] = temp;
+  st->cs[j] = c;
+  st->sn[j] = s;
+  H[j] = c * ci + s * h;
+  H[j + 1] = 0.0;
+  const double gj = g[j], gn = g[j + 1];
+  const double next = -s * gj + c * gn;
+  g[j] = c * gj + s * gn;
+  g[j + 1] = next;
   st->iters += 1;
   st->j_final = j;
-  double absres = fabs(g[j + 1]);
+  const double absres = fabs(next);
   st->resnorm = absres;
   if (st->collect) st->history[st->iters - 1] = absres;
   if (absres / st->bnorm < st->tol) {
     st->converged = 1;
     st->stop = 1;
   }
+}
+
+// The one-launch modified Gram-Schmidt step.  448 threads with data and the
+// link's wavefront make two wavefronts a SIMD: 256 registers each, which the
+// three vectors of 28 FP64 elements fit (512 + 64 threads leave 168: the
+// 3.6M-row step spilled and took 611 us instead of 309).
+constexpr int kMgsBlock = 448;
+constexpr int kMgsMaxCols = 512;  // restart dimension the LDS columns hold
+constexpr int kMgsMaxElems = 28;  // elements a thread holds
+// Up to here one block, whose exchanges stay in LDS: 8,000 rows took 35.6 us
+// a GMRES(30) step against 45.9 with 16 blocks; 14,616 rows do not fit one
+// block's registers without loss (74 us against 39 with 8 blocks).
+constexpr int kMgsSolo = 16 * kMgsBlock;
+// Elements a block, at least: 512 / 1024 / 2048 / 4096 took 71.6 / 78.8 /
+// 54.7 / 57.5 us a step at 110,592 rows and 92.8 / 92.8 / 63.4 / 65.5 at
+// 262,144 (more blocks: more slots for every block to read).
+constexpr int kMgsGrain = 4 * kMgsBlock;
+
+inline int mgs_blocks() { return std::min(kLinkBlocks, ctx().num_cus); }
+inline bool mgs_fits(int64_t n, int64_t m) {
+  return m <= kMgsMaxCols && n <= (int64_t)mgs_blocks() * kMgsBlock * kMgsMaxElems;
+}
+
+// One modified Gram-Schmidt step in one launch (gmres.hpp:258-280): w =
+// V_{j+1} stays in registers, E elements a thread; for every basis vector in
+// turn the blocks exchange their parts of <V_i, w> and subtract, then |w|,
+// the Givens update and the normalisation.  V_{i+1} is loaded while the
+// exchange of V_i is under way.  w comes from w0, scaled by a Jacobi left
+// preconditioner's diagonal dl (may be null); with a Jacobi right one (dr)
+// the next step's Z_{j+1} = M V_{j+1} is written too.  The arithmetic is that
+// of the kernels gmres_solve queues otherwise; only the dot products'
+// summation order differs.
+// Bound: each exchange's round trip through memory (about 1.9 us; 0.7 us
+// within one block) up to some 300,000 rows, the basis' bytes beyond (2.1M
+// rows FP64: V is read at 4.3 TB/s).  A GMRES(30) step with Jacobi, the
+// sequence of kernels -> this: 4,096 rows 108.0 -> 28.0 us, 32,768 rows
+// 109.2 -> 46.6, 262,144 rows 126.1 -> 62.5, 2,097,152 rows 329.4 -> 148.3
+// (FP32 203.2 -> 114.4).
+template <typename T, int E>
+__global__ __launch_bounds__(kMgsBlock + 64) void mgs_step_kernel(
+    unsigned n, const T* __restrict__ V, size_t ldv, const T* __restrict__ w0,
+    const T* __restrict__ dl, T* __restrict__ w, const T* __restrict__ dr,
+    T* __restrict__ z, int j, GmState* st, GridLink link) {
+  __shared__ double red[link_lds(kMgsBlock)];
+  __shared__ double hc[kMgsMaxCols + 1], cs[kMgsMaxCols], sn[kMgsMaxCols];
+  if (st->stop) return;  // written only after every block has been here
+  unsigned tag = *link.tag;
+  // the link's wavefront holds no elements
+  const unsigned i0 =
+      threadIdx.x < kMgsBlock ? blockIdx.x * (kMgsBlock * E) + threadIdx.x : n;
+  if (blockIdx.x == 0)
+    for (int k = threadIdx.x; k < j; k += kMgsBlock + 64) {
+      cs[k] = st->cs[k];
+      sn[k] = st->sn[k];
+    }
+  T x[E], v[E], next[E];
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const unsigned e = i0 + u * kMgsBlock;
+    x[u] = e < n ? w0[e] : T(0);
+    v[u] = e < n ? V[e] : T(0);
+  }
+  if (dl) {
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const unsigned e = i0 + u * kMgsBlock;
+      if (e < n) x[u] = dl[e] * x[u];
+    }
+  }
+  bool ok = true;
+  for (int i = 0; i <= j; ++i) {
+    if (i < j) {
+      const T* vn = V + (size_t)(i + 1) * ldv;
+#pragma unroll
+      for (int u = 0; u < E; ++u) {
+        const unsigned e = i0 + u * kMgsBlock;
+        next[u] = e < n ? vn[e] : T(0);
+      }
+    }
+    double s[1] = {0.0};
+#pragma unroll
+    for (int u = 0; u < E; ++u) s[0] += (double)v[u] * (double)x[u];
+    ok = ok && link_sum<1, kMgsBlock>(link, ++tag, s, red);
+#pragma unroll
+    for (int u = 0; u < E; ++u) x[u] = (T)((double)x[u] - s[0] * (double)v[u]);
+    if (threadIdx.x == 0) hc[i] = s[0];
+#pragma unroll
+    for (int u = 0; u < E; ++u) v[u] = next[u];
+  }
+  double s[1] = {0.0};
+#pragma unroll
+  for (int u = 0; u < E; ++u) s[0] += (double)x[u] * (double)x[u];
+  ok = ok && link_sum<1, kMgsBlock>(link, ++tag, s, red);
+  const double hn = sqrt(s[0]);
+  // normalise V_{j+1} if h > 0 (gmres.hpp:276-280 divides, fgmres.hpp:283
+  // multiplies by the reciprocal)
+  const double inv = 1.0 / hn;
+  const bool flexible = st->flexible != 0;
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    const unsigned e = i0 + u * kMgsBlock;
+    T t = x[u];
+    if (hn > 0.0) t = flexible ? (T)((double)t * inv) : (T)((double)t / hn);
+    x[u] = t;
+    if (e < n) w[e] = t;
+  }
+  if (dr) {
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      const unsigned e = i0 + u * kMgsBlock;
+      if (e < n) z[e] = dr[e] * x[u];
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (gridDim.x > 1) *link.tag = tag;
+    if (ok) arnoldi_finish(st, j, hn, hc, cs, sn);
+    else st->stop = 1;  // the host reports it
+  }
+}
+
+// One block while n fits it (its sums stay in LDS), else about kMgsGrain
+// elements a block while there are blocks left; E: the smallest that holds a
+// block's share.
+template <typename T>
+void launch_mgs_step(int64_t n, const T* V, size_t ldv, const T* w0, const T* dl, T* w,
+                     const T* dr, T* z, int j, GmState* st, const GridLink& link) {
+  const int64_t share =
+      n <= kMgsSolo ? n : std::max<int64_t>(kMgsGrain, (n + mgs_blocks() - 1) / mgs_blocks());
+  const int64_t e = (share + kMgsBlock - 1) / kMgsBlock;
+  auto run = [&](auto size) {
+    constexpr int E = decltype(size)::value;
+    const int g = (int)((n + kMgsBlock * E - 1) / (kMgsBlock * E));
+    hipLaunchKernelGGL((mgs_step_kernel<T, E>), dim3(g), dim3(kMgsBlock + 64), 0,
+                       stream(), (unsigned)n, V, ldv, w0, dl, w, dr, z, j, st, link);
+    SPK_HIP_TRY(hipGetLastError());
+  };
+  if (e <= 1) run(std::integral_constant<int, 1>{});
+  else if (e <= 2) run(std::integral_constant<int, 2>{});
+  else if (e <= 4) run(std::integral_constant<int, 4>{});
+  else if (e <= 8) run(std::integral_constant<int, 8>{});
+  else if (e <= 12) run(std::integral_constant<int, 12>{});
+  else if (e <= 16) run(std::integral_constant<int, 16>{});
+  else if (e <= 20) run(std::integral_constant<int, 20>{});
+  else if (e <= 24) run(std::integral_constant<int, 24>{});
+  else run(std::integral_constant<int, kMgsMaxElems>{});
 }
 
 constexpr int kDotChunk = 4096;  // elements per (chunk, vector) block
@@ -249,6 +397,10 @@ void gmres_solve(bool flexible, spk_csr_s* A, spk_precond_s* ML,
     parts = reduce_partials(std::max<size_t>((size_t)(m + 1) * nch,
                                              (size_t)vec_grid(n)));
   }
+  // modified Gram-Schmidt with V_{j+1} in registers, one launch a step
+  const bool mgs_one = !cgs2 && mgs_fits(n, m);
+  GridLink link{};
+  if (mgs_one) link = grid_link();
   DevState<GmState> st(kWsGmres + 5);
   GmState h{};
   h.tol = cfg->tolerance;
@@ -294,9 +446,8 @@ void gmres_solve(bool flexible, spk_csr_s* A, spk_precond_s* ML,
       acc[0] += (double)V[i] * (double)V[i];
     }, [=] __device__(const double* t) {
       double beta = sqrt(t[0]);
+      // H and the rotations are written column by column before they are read
       for (int64_t k = 0; k <= S->m; ++k) S->g[k] = 0.0;
-      for (int64_t k = 0; k < (S->m + 1) * S->m; ++k) S->H[k] = 0.0;
-      for (int64_t k = 0; k < S->m; ++k) S->cs[k] = S->sn[k] = 0.0;
       S->g[0] = beta;
       S->hnorm = beta;
       S->j_final = 0;
@@ -327,12 +478,22 @@ void gmres_solve(bool flexible, spk_csr_s* A, spk_precond_s* ML,
       T* vj = V + (size_t)j * nn;
       T* vj1 = V + (size_t)(j + 1) * nn;
       T* zj = right_id ? vj : Z + (size_t)j * nn;
-      if (!right_id) right->apply((const T*)vj, zj);
+      // with the one-launch step a Jacobi preconditioner is applied there
+      if (!right_id && !(mgs_one && is_jacobi(right) && j > 0))
+        right->apply((const T*)vj, zj);
       if (is_identity(left)) {
         launch_spmv(*A, (const T*)zj, EpiStore<T>{vj1, stop}, s);
       } else {
         launch_spmv(*A, (const T*)zj, EpiStore<T>{r0, stop}, s);
-        left->apply((const T*)r0, vj1);
+        if (!(mgs_one && is_jacobi(left))) left->apply((const T*)r0, vj1);
+      }
+      if (mgs_one) {
+        const bool dl = is_jacobi(left), dr = is_jacobi(right) && j + 1 < m_eff;
+        launch_mgs_step(n, (const T*)V, nn, dl ? (const T*)r0 : (const T*)vj1,
+                        dl ? diag_of<T>(left) : nullptr, vj1,
+                        dr ? diag_of<T>(right) : nullptr, dr ? zj + nn : nullptr,
+                        (int)j, S, link);
+        continue;  // V_{j+1} is normalised
       }
       if (cgs2) {
         double* hcol = small + j * ld;
@@ -357,7 +518,7 @@ void gmres_solve(bool flexible, spk_csr_s* A, spk_precond_s* ML,
                                stop);
             const int jj = (int)j;
             launch_finish<1>(parts, g, [=] __device__(const double* t) {
-              arnoldi_finish(S, jj, sqrt(t[0]));
+              arnoldi_finish(S, jj, sqrt(t[0]), hcol, S->cs, S->sn);
             }, stop);
           }
           SPK_HIP_TRY(hipGetLastError());
@@ -386,7 +547,7 @@ void gmres_solve(bool flexible, spk_csr_s* A, spk_precond_s* ML,
           vj1[e] = w;
           acc[0] += (double)w * (double)w;
         }, [=] __device__(const double* t) {
-          arnoldi_finish(S, jj, sqrt(t[0]));
+          arnoldi_finish(S, jj, sqrt(t[0]), hcol, S->cs, S->sn);
         }, stop);
       }
       }  // MGS
@@ -414,10 +575,13 @@ void gmres_solve(bool flexible, spk_csr_s* A, spk_precond_s* ML,
       x[e] = (T)((double)x[e] + sum);
     }, done);
     // close the cycle: a converged cycle finishes the solve
+    const int* expired = link.expired;
     launch_map(1, [=] __device__(int64_t) {
       if (S->converged) S->done = 1;
-    }, done);
+      if (expired) S->expired = *expired;
+    });
     h = st.download();
+    if (h.expired) check_link(link);
     iters = h.iters;
     if (monitor && !h.converged && !h.done && !(*monitor)(iters, h.resnorm))
       break;

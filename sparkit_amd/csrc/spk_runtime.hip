@@ -1,6 +1,6 @@
 // spk_runtime.hip -- device selection, the library stream, device memory,
 // timers, the workspace pool and the reduction scratch.
-#include "spk_internal.hpp"
+#include "spk_link.hpp"
 
 #include <cstring>
 #include <memory>
@@ -26,6 +26,7 @@ struct Arena {
   size_t slot_bytes[kArenaSlots] = {};
   double* partials = nullptr;
   size_t partials_count = 0;
+  GridLink link{};
 };
 Arena* g_arena = nullptr;
 
@@ -48,6 +49,21 @@ hipStream_t g_user_stream = nullptr;
 hipEvent_t g_ev0 = nullptr, g_ev1 = nullptr;
 std::unique_ptr<Workspace> g_ws;
 DevBuf<double>* g_partials = nullptr;
+DevBuf<unsigned long long>* g_link = nullptr;
+
+__global__ void link_clear_kernel(unsigned long long* w, int n) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) w[k] = 0;
+}
+
+// a link over kLinkWords words at w, cleared
+GridLink make_link(unsigned long long* w) {
+  const int n = (int)kLinkWords;
+  hipLaunchKernelGGL(link_clear_kernel, dim3((n + 255) / 256), dim3(256), 0, stream(),
+                     w, n);
+  SPK_HIP_TRY(hipGetLastError());
+  return GridLink{w, (unsigned*)(w + kLinkSlotWords), (int*)(w + kLinkSlotWords + 1)};
+}
 
 void init_device(int device) {
   int count = 0;
@@ -147,6 +163,33 @@ double* reduce_partials(size_t count) {
   return g_partials->p;
 }
 
+GridLink grid_link() {
+  ctx();
+  if (g_arena) {
+    Arena& a = *g_arena;
+    if (!a.link.slots)
+      a.link = make_link((unsigned long long*)arena_carve(
+          a, kLinkWords * sizeof(unsigned long long)));
+    return a.link;
+  }
+  static GridLink link;  // of g_link's memory
+  if (!g_link) {
+    g_link = new DevBuf<unsigned long long>(kLinkWords);
+    link = make_link(g_link->p);
+  }
+  return link;
+}
+
+void check_link(const GridLink& l) {
+  int h = 0;
+  SPK_HIP_TRY(hipMemcpyAsync(&h, l.expired, sizeof(int), hipMemcpyDeviceToHost, stream()));
+  SPK_HIP_TRY(hipStreamSynchronize(stream()));
+  if (!h) return;
+  (void)make_link(l.slots);  // flag and slots cleared
+  SPK_HIP_TRY(hipStreamSynchronize(stream()));
+  SPK_REQUIRE(false, SPK_HIP_ERROR,
+              "grid exchange: a bounded wait expired (results invalid)");
+}
 
 }  // namespace spk
 
@@ -172,6 +215,8 @@ spk_status spk_finalize(void) {
     g_ws.reset();
     delete g_partials;
     g_partials = nullptr;
+    delete g_link;
+    g_link = nullptr;
     (void)hipEventDestroy(g_ev0);
     (void)hipEventDestroy(g_ev1);
     (void)hipStreamDestroy(g_ctx.stream);
