@@ -264,16 +264,17 @@ spk_status spk_convert(int64_t n, int dtype_src, const void* d_src,
  * SPK_INVALID_ARGUMENT on an exact zero diagonal entry. */
 spk_status spk_precond_create_jacobi(spk_csr A, spk_precond* out);
 /* ilu0(A) / milu0(A) (ilu.hpp:35-168): factors on A's pattern, computed on
- * the device by level-scheduled IKJ rows; L has its unit diagonal last,
+ * the device by IKJ rows in dependency order; L has its unit diagonal last,
  * U its diagonal first (ilu.hpp:123-141).  SPK_INVALID_ARGUMENT for a
  * non-square matrix or a missing diagonal. */
 spk_status spk_precond_create_ilu0(spk_csr A, int modified, spk_precond* out);
 /* Schedule of the ILU(0) triangular sweeps (no reference counterpart; the
- * arithmetic, and so the result, is the same for both): SPK_ILU_AUTO (0,
- * the default: per-level launches for at least 65536 rows and at most 4096
- * levels, else sync-free), SPK_ILU_LEVELS (1: one launch per dependency
- * level), SPK_ILU_SYNC_FREE (2: one launch per sweep, rows wait for their
- * dependencies' published values). */
+ * arithmetic, and so the result, is the same for all): SPK_ILU_AUTO (0, the
+ * default) and SPK_ILU_SYNC_FREE (2) run one launch per sweep, in which rows
+ * wait for their dependencies' published values; SPK_ILU_LEVELS (1) runs one
+ * launch per dependency level.  Under AUTO get_schedule names the factors'
+ * shape, not the launches: LEVELS for at least 65536 rows and at most 4096
+ * levels, else SYNC_FREE. */
 #define SPK_ILU_AUTO 0
 #define SPK_ILU_LEVELS 1
 #define SPK_ILU_SYNC_FREE 2

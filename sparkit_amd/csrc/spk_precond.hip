@@ -2,7 +2,9 @@
 #include "spk_precond.hpp"
 
 #include <algorithm>
+#include <cstring>
 #include <type_traits>
+#include <utility>
 
 #include "spk_vec.hpp"
 
@@ -69,169 +71,92 @@ __global__ void ilu_factor_level_kernel(const int32_t* __restrict__ rows,
   if (modified) w[diag_pos[i]] = w[diag_pos[i]] - dropped;
 }
 
-// Split the factored values into L (unit diagonal last) and U (diagonal
+// Split the factored rows into L (unit diagonal last) and U (diagonal
 // first): ilu.hpp:123-141.
-__global__ void ilu_split_kernel(int64_t n, const int32_t* __restrict__ rp,
-                                 const int32_t* __restrict__ ci,
-                                 const double* __restrict__ w,
+__global__ void ilu_split_kernel(TriPattern P, const double* __restrict__ w,
                                  const int32_t* __restrict__ lrp,
-                                 double* __restrict__ lv,
+                                 int32_t* __restrict__ lci, double* __restrict__ lv,
                                  const int32_t* __restrict__ urp,
-                                 double* __restrict__ uv) {
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
+                                 int32_t* __restrict__ uci, double* __restrict__ uv) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= P.n) return;
+  const int dp = P.dpos[i];
   int lk = lrp[i], uk = urp[i];
-  for (int p = rp[i]; p < rp[i + 1]; ++p) {
-    if (ci[p] < i) lv[lk++] = w[p];
-    else uv[uk++] = w[p];
+  for (int p = P.rp[i]; p < dp; ++p, ++lk) {
+    lci[lk] = P.ci[p];
+    lv[lk] = w[p];
   }
+  lci[lk] = (int32_t)i;
   lv[lk] = 1.0;
+  for (int p = dp; p < P.rp[i + 1]; ++p, ++uk) {
+    uci[uk] = P.ci[p];
+    uv[uk] = w[p];
+  }
 }
 
-// Triangular sweeps in ONE launch ("sync-free").  Rows are laid out in
-// dependency-level order, one thread per row, and every level is padded to a
-// multiple of the wavefront size, so the rows of one wavefront never depend
-// on each other: a lane only ever waits for rows of EARLIER wavefronts.
-// (Without the padding a wavefront straddling two levels deadlocks: the
-// compiler may sink the final store below the wait loop, where it runs only
-// after every lane of the wavefront has left the loop.)  Every value of the
-// output doubles as its own ready flag: the output starts filled with a NaN
-// sentinel that arithmetic never produces, a finished row stores its value
-// with one agent-scope atomic store, and a row waiting on a dependency spins
-// on an agent-scope atomic load of it.  Workgroups are dispatched in order,
-// so the earliest unfinished wavefront always has its dependencies resident
-// or finished.  A bounded spin sets an error flag and ends the row, so every
-// wavefront exits whatever happens.
-template <typename T>
-struct Sentinel;
-template <>
-struct Sentinel<double> {
-  typedef unsigned long long U;
-  static constexpr U bits = 0xFFF8DEADBEEFCAFEull;
-};
-template <>
-struct Sentinel<float> {
-  typedef unsigned int U;
-  static constexpr U bits = 0xFFC0DEADu;
-};
-
-template <typename T>
-__device__ __forceinline__ bool load_ready(const T* p, T* out) {
-  typedef typename Sentinel<T>::U U;
-  U u = __hip_atomic_load(reinterpret_cast<const U*>(p), __ATOMIC_RELAXED,
-                          __HIP_MEMORY_SCOPE_AGENT);
-  T v;
-  __builtin_memcpy(&v, &u, sizeof(T));
-  *out = v;
-  return u != Sentinel<T>::bits;
+// Each row's diagonal position (ilu.hpp:54-66); out[0] |= 1 a missing
+// diagonal, 2 columns that do not ascend, 4 a repeated diagonal, 8 another
+// repeated column; out[1] the longest row; out[4] the most entries on one
+// side of the diagonal; *lower: the strictly lower entries.
+__global__ void ilu_rows_kernel(int64_t n, const int32_t* __restrict__ rp,
+                                const int32_t* __restrict__ ci, int32_t* __restrict__ dpos,
+                                int* out, unsigned long long* lower) {
+  __shared__ unsigned long long red[256 / 64];
+  unsigned long long below = 0;
+  int bad = 0, len = 0, side = 0;
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * 256) {
+    const int p0 = rp[i], pe = rp[i + 1];
+    int d = -1, last = -1;
+    for (int p = p0; p < pe; ++p) {
+      const int c = ci[p];
+      if (c < last) bad |= 2;
+      if (c == last && c != i) bad |= 8;
+      if (c == i) {
+        if (d >= 0) bad |= 4;
+        else d = p;
+      }
+      last = c;
+    }
+    if (d < 0) {
+      bad |= 1;
+      d = p0;
+    }
+    dpos[i] = d;
+    below += (unsigned long long)(d - p0);
+    len = pe - p0 > len ? pe - p0 : len;
+    side = d - p0 > side ? d - p0 : side;
+    side = pe - d - 1 > side ? pe - d - 1 : side;
+  }
+  below = block_reduce_sum<unsigned long long, 256>(below, red);
+  for (int o = 32; o > 0; o >>= 1) {
+    const int other = __shfl_xor(len, o, 64);
+    len = other > len ? other : len;
+    const int os = __shfl_xor(side, o, 64);
+    side = os > side ? os : side;
+    bad |= __shfl_xor(bad, o, 64);
+  }
+  if (threadIdx.x == 0) atomicAdd(lower, below);
+  if ((threadIdx.x & 63) == 0) {
+    if (bad) atomicOr(out, bad);
+    atomicMax(out + 1, len);
+    atomicMax(out + 4, side);
+  }
 }
 
-template <typename T>
-__device__ __forceinline__ void store_ready(T* p, T v) {
-  typedef typename Sentinel<T>::U U;
-  U u;
-  __builtin_memcpy(&u, &v, sizeof(T));
-  // a NaN result carrying the sentinel's payload (propagated from a NaN
-  // input) must not read as "not ready": publish it with another payload
-  if (u == Sentinel<T>::bits) u ^= (U)1;
-  __hip_atomic_store(reinterpret_cast<U*>(p), u, __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
+__global__ void clear_words_kernel(int* p, int n) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) p[k] = 0;
 }
 
-template <typename T>
-__device__ __forceinline__ T sentinel_value() {
-  typedef typename Sentinel<T>::U U;
-  U u = Sentinel<T>::bits;
-  T v;
-  __builtin_memcpy(&v, &u, sizeof(T));
-  return v;
-}
-
-constexpr unsigned kSpinLimit = 1u << 22;
-constexpr int kSweepBatch = 4;  // dependencies a sweep row loads together
 constexpr int kErrorWords = 64;  // sweep status word + guard words
-// sweep schedule thresholds (see spk_precond_s::level_launch)
+// the reported schedule's thresholds (see spk_precond_s::level_launch)
 constexpr int64_t kLevelLaunchRows = 65536;
 constexpr int64_t kLevelLaunchMaxLevels = 4096;
 
-// LOWER: forward_solve (triangular_solve.hpp:42-53), the diagonal is the
-// row's last entry; otherwise backward_solve (:82-96), the diagonal is the
-// first.  x[c] -= v * x[c'] in storage order, multiply-adds not contracted:
-// bit-identical to the sequential reference.  Optionally resets b[i] to the
-// sentinel after reading it (b is the previous sweep's output) and marks
-// mark[i] with the sentinel (the next sweep's output).
-template <typename T, bool LOWER>
-__global__ __launch_bounds__(256) void sweep_kernel(
-    const int32_t* __restrict__ rows, int n, const int32_t* __restrict__ rp,
-    const int32_t* __restrict__ ci, const T* __restrict__ v, T* b, T* x,
-    bool reset_b, T* mark, int* error) {
-#pragma clang fp contract(off)
-  // A small persistent grid walks the sweep order: each thread takes the
-  // rows t, t + W, t + 2W, ... (W = grid threads), so only a window of W
-  // rows -- a few levels -- waits at any time.  A wavefront always holds 64
-  // consecutive positions of one (padded) level, i.e. independent rows, and
-  // every row waits only for earlier positions, so the earliest unfinished
-  // row can always proceed.
-  const int W = gridDim.x * blockDim.x;
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += W) {
-    const int i = rows[t];
-    if (i < 0) continue;  // level padding
-    const int p0 = rp[i], p1 = rp[i + 1];
-    const int q1 = LOWER ? p1 - 1 : p1;
-    const int pd = LOWER ? p1 - 1 : p0;
-    T s = b[i];
-    if (reset_b) b[i] = sentinel_value<T>();
-    if (mark) mark[i] = sentinel_value<T>();
-    // The dependencies are polled kSweepBatch at a time: all of a batch's
-    // loads are issued together (one round trip instead of one per
-    // dependency), and the batch is consumed in storage order once every
-    // value in it is ready -- the reference's arithmetic, unchanged.
-    int p = LOWER ? p0 : p0 + 1;
-    unsigned spins = 0;
-    while (p < q1) {
-      const int cnt = q1 - p < kSweepBatch ? q1 - p : kSweepBatch;
-      int c[kSweepBatch];
-      T xv[kSweepBatch];
-      bool ok[kSweepBatch];
-#pragma unroll
-      for (int k = 0; k < kSweepBatch; ++k) {
-        ok[k] = k >= cnt;
-        c[k] = k < cnt ? ci[p + k] : 0;
-      }
-      bool all = false;
-      while (!all) {
-        all = true;
-#pragma unroll
-        for (int k = 0; k < kSweepBatch; ++k) {
-          if (!ok[k]) ok[k] = load_ready(x + c[k], &xv[k]);
-          all = all && ok[k];
-        }
-        if (!all) {
-          if (++spins > kSpinLimit) {
-            atomicOr(error, LOWER ? 1 : 2);
-            break;
-          }
-          __builtin_amdgcn_s_sleep(2);  // back off: fewer polls in flight
-        }
-      }
-      if (!all) {  // expired wait: publish what there is (reported)
-        p = q1;
-        break;
-      }
-#pragma unroll
-      for (int k = 0; k < kSweepBatch; ++k)
-        if (k < cnt) s = s - v[p + k] * xv[k];
-      p += cnt;
-    }
-    store_ready(x + i, s / v[pd]);
-    // keep this row's publication ahead of the next row's waits
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  }
-}
-
 // One dependency level of a triangular sweep: every row of the level reads
 // only rows of earlier levels (final, previous launches), so plain loads
-// suffice.  Same operation order as sweep_kernel.
+// suffice.  Same operation order as the sweeps in tiles.
 template <typename T, bool LOWER>
 __global__ __launch_bounds__(256) void level_sweep_kernel(
     const int32_t* __restrict__ rows, int count, const int32_t* __restrict__ rp,
@@ -254,18 +179,6 @@ __global__ void fill_sentinel_kernel(T* x, int64_t n) {
   if (i < n) x[i] = sentinel_value<T>();
 }
 
-// rows grouped by level, each level padded with -1 to a multiple of 64
-std::vector<int32_t> pad_levels(const std::vector<int32_t>& rows,
-                                const std::vector<int32_t>& ptr) {
-  std::vector<int32_t> out;
-  out.reserve(rows.size() + 64 * (ptr.size() - 1));
-  for (size_t l = 0; l + 1 < ptr.size(); ++l) {
-    for (int32_t k = ptr[l]; k < ptr[l + 1]; ++k) out.push_back(rows[k]);
-    while (out.size() % 64) out.push_back(-1);
-  }
-  return out;
-}
-
 // group rows by level (counting sort); returns level pointer array
 std::vector<int32_t> group_levels(const std::vector<int32_t>& lvl,
                                   std::vector<int32_t>& rows_out) {
@@ -280,18 +193,20 @@ std::vector<int32_t> group_levels(const std::vector<int32_t>& lvl,
   return ptr;
 }
 
-spk_csr_s* make_store(int64_t n, std::vector<int32_t>&& rp,
-                      const std::vector<int32_t>& ci) {
+// an n x n store with the given row offsets, columns and values not set
+spk_csr_s* make_store(int64_t n, std::vector<int32_t>&& rp) {
   auto* S = new spk_csr_s();
-  S->allocate(n, n, rp[n]);
-  hipStream_t s = stream();
-  SPK_HIP_TRY(hipMemcpyAsync(S->rp.p, rp.data(), rp.size() * 4,
-                             hipMemcpyHostToDevice, s));
-  SPK_HIP_TRY(hipMemcpyAsync(S->ci.p, ci.data(), ci.size() * 4,
-                             hipMemcpyHostToDevice, s));
-  SPK_HIP_TRY(hipStreamSynchronize(s));
-  S->h_rp = std::move(rp);
-  upload_plan(*S, build_spmv_plan(S->h_rp.data(), n, &S->nlong));
+  try {
+    S->allocate(n, n, rp[(size_t)n]);
+    SPK_HIP_TRY(hipMemcpyAsync(S->rp.p, rp.data(), rp.size() * 4, hipMemcpyHostToDevice,
+                               stream()));
+    SPK_HIP_TRY(hipStreamSynchronize(stream()));
+    S->h_rp = std::move(rp);
+    upload_plan(*S, build_spmv_plan(S->h_rp.data(), n, &S->nlong));
+  } catch (...) {
+    delete S;
+    throw;
+  }
   return S;
 }
 
@@ -319,6 +234,104 @@ const float* spk_precond_s::inv_diag32() {
     has32 = true;
   }
   return inv_d32.p;
+}
+
+bool spk_precond_s::wide_levels() const {
+  return n >= kLevelLaunchRows && std::max(levels_l, levels_u) <= kLevelLaunchMaxLevels;
+}
+
+// ilu0_impl (ilu.hpp:35-141): the pattern, both triangles' layouts and the
+// numeric factorization, all on the device; the host reads back a few
+// counters in between.
+void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
+  hipStream_t s = stream();
+  n = A.nrows;
+  nnz = A.nnz;
+  rp.alloc((size_t)n + 1);
+  ci.alloc((size_t)nnz);
+  w.alloc((size_t)nnz);
+  dpos.alloc((size_t)n);
+  sweep_error.alloc(kErrorWords);
+  ticket.alloc(10);  // two sweeps' tickets; counters of the construction
+  SPK_HIP_TRY(hipMemcpyAsync(rp.p, A.rp.p, (n + 1) * 4, hipMemcpyDeviceToDevice, s));
+  if (nnz) SPK_HIP_TRY(hipMemcpyAsync(ci.p, A.ci.p, nnz * 4, hipMemcpyDeviceToDevice, s));
+  DevBuf<double> ordered;  // the values, where the rows had to be sorted
+  hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, s, sweep_error.p, kErrorWords);
+  int h[5];
+  for (bool sorted = false;;) {
+    hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, s, ticket.p, 10);
+    hipLaunchKernelGGL(ilu_rows_kernel, dim3(std::min(blocks_for(n), 1024u)), dim3(256), 0, s, n,
+                       (const int32_t*)rp.p, (const int32_t*)ci.p, dpos.p, ticket.p + 4,
+                       (unsigned long long*)(ticket.p + 6));
+    SPK_HIP_TRY(hipGetLastError());
+    SPK_HIP_TRY(hipMemcpyAsync(h, ticket.p + 4, sizeof(h), hipMemcpyDeviceToHost, s));
+    SPK_HIP_TRY(hipStreamSynchronize(s));
+    SPK_REQUIRE((h[0] & 1) == 0, SPK_INVALID_ARGUMENT, "ilu0: missing diagonal entry");
+    SPK_REQUIRE((h[0] & 4) == 0, SPK_INVALID_ARGUMENT, "ilu0: repeated diagonal entry");
+    if ((h[0] & 2) == 0 || sorted) break;
+    sort_rows(A, ordered);  // a caller's CSR rows in another order than ascending
+    sorted = true;
+  }
+  unsigned long long below;
+  std::memcpy(&below, h + 2, sizeof(below));
+  nnz_l = (int64_t)below + n;
+  nnz_u = nnz - (int64_t)below;
+  const TriPattern P = pattern();
+  {
+    DevBuf<int32_t> lvl;
+    int count[2];
+    tri_levels(P, lvl, count);
+    levels_l = lower.levels = count[0];
+    levels_u = upper.levels = count[1];
+    tri_layout(P, true, lvl.p, lower);
+    tri_layout(P, false, lvl.p + n, upper);
+  }
+  level_launch = wide_levels();
+  per_level = n >= kMaxTileSweepRows;
+  const double* in = ordered.p ? ordered.p : A.v64.p;
+  if (h[1] <= kTriFactorLen && (h[0] & 8) == 0) {
+    tri_factor(P, lower, in, w, modified, h[1], h[4], ticket.p, sweep_error.p);
+  } else {
+    // long rows, or a column twice: one launch per dependency level, a
+    // thread per row
+    SPK_HIP_TRY(hipMemcpyAsync(w.p, in, nnz * 8, hipMemcpyDeviceToDevice, s));
+    build_levels();
+    for (size_t l = 0; l + 1 < lvl_ptr_l.size(); ++l) {
+      const int cnt = lvl_ptr_l[l + 1] - lvl_ptr_l[l];
+      hipLaunchKernelGGL(ilu_factor_level_kernel, dim3(blocks_for(cnt)), dim3(256), 0, s,
+                         lvl_rows_l.p + lvl_ptr_l[l], cnt, rp.p, ci.p, dpos.p, w.p,
+                         modified ? 1 : 0);
+    }
+    SPK_HIP_TRY(hipGetLastError());
+  }
+  tri_values(P, true, w.p, lower);
+  tri_values(P, false, w.p, upper);
+  check_sweeps();
+}
+
+void spk_precond_s::sort_rows(const spk_csr_s& A, DevBuf<double>& values) {
+  hipStream_t s = stream();
+  std::vector<int32_t> c((size_t)nnz);
+  std::vector<double> v((size_t)nnz);
+  SPK_HIP_TRY(hipMemcpyAsync(c.data(), ci.p, nnz * 4, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipMemcpyAsync(v.data(), A.v64.p, nnz * 8, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipStreamSynchronize(s));
+  std::vector<std::pair<int32_t, double>> row;
+  for (int64_t i = 0; i < n; ++i) {
+    const size_t a = (size_t)A.h_rp[(size_t)i], b = (size_t)A.h_rp[(size_t)i + 1];
+    row.clear();
+    for (size_t k = a; k < b; ++k) row.emplace_back(c[k], v[k]);
+    std::stable_sort(row.begin(), row.end(),
+                     [](const auto& x, const auto& y) { return x.first < y.first; });
+    for (size_t k = a; k < b; ++k) {
+      c[k] = row[k - a].first;
+      v[k] = row[k - a].second;
+    }
+  }
+  SPK_HIP_TRY(hipMemcpyAsync(ci.p, c.data(), nnz * 4, hipMemcpyHostToDevice, s));
+  values.alloc((size_t)nnz);
+  SPK_HIP_TRY(hipMemcpyAsync(values.p, v.data(), nnz * 8, hipMemcpyHostToDevice, s));
+  SPK_HIP_TRY(hipStreamSynchronize(s));
 }
 
 template <typename T>
@@ -353,7 +366,8 @@ void spk_precond_s::reset_sentinels() {
 
 void spk_precond_s::check_sweeps() {
   if (kind != kIlu) return;
-  // word 0: 1 = a forward, 2 = a backward sweep's bounded wait expired;
+  // word 0: 1 = a forward, 2 = a backward sweep's bounded wait expired, 4 =
+  // the factorization's;
   // words 1..kErrorWords-1 must stay zero (a guard against stray writes)
   int h[kErrorWords];
   SPK_HIP_TRY(hipMemcpyAsync(h, sweep_error.p, sizeof(h), hipMemcpyDeviceToHost,
@@ -366,6 +380,8 @@ void spk_precond_s::check_sweeps() {
   SPK_HIP_TRY(hipStreamSynchronize(stream()));
   SPK_REQUIRE(guard_ok, SPK_HIP_ERROR,
               "ILU sweep status words overwritten (a stray device write)");
+  SPK_REQUIRE((h[0] & 4) == 0, SPK_HIP_ERROR,
+              "ilu0: bounded wait expired in the factorization");
   SPK_REQUIRE(false, SPK_HIP_ERROR,
               std::string("ILU triangular sweep: bounded wait expired in the ") +
                   (h[0] & 1 ? "forward" : "") + (h[0] == 3 ? " and " : "") +
@@ -375,6 +391,8 @@ void spk_precond_s::check_sweeps() {
 template <typename T, bool LOWER>
 void spk_precond_s::level_sweep(const T* b, T* x) {
   hipStream_t s = stream();
+  build_factors();
+  build_levels();
   CsrView<T> v = (LOWER ? L : U)->view<T>();
   const std::vector<int32_t>& ptr = LOWER ? lvl_ptr_l : lvl_ptr_u;
   const int32_t* rows = LOWER ? lvl_rows_l.p : lvl_rows_u.p;
@@ -388,34 +406,72 @@ void spk_precond_s::level_sweep(const T* b, T* x) {
 
 template <typename T>
 void spk_precond_s::forward(const T* b, T* x) {
-  if (level_launch) {
+  if (per_level) {
     level_sweep<T, true>(b, x);
     return;
   }
   hipStream_t s = stream();
-  CsrView<T> v = L->view<T>();
-  hipLaunchKernelGGL((fill_sentinel_kernel<T>), dim3(blocks_for(n)),
-                     dim3(256), 0, s, x, n);
-  hipLaunchKernelGGL((sweep_kernel<T, true>), dim3(sweep_grid_l),
-                     dim3(256), 0, s, sweep_rows_l.p, (int)sweep_len_l, v.rp,
-                     v.ci, v.v, (T*)b, x, false, (T*)nullptr, sweep_error.p);
+  hipLaunchKernelGGL((fill_sentinel_kernel<T>), dim3(blocks_for(n)), dim3(256), 0, s, x, n);
   SPK_HIP_TRY(hipGetLastError());
+  tri_sweep<T, true>(lower, (T*)b, x, false, (T*)nullptr, ticket.p, sweep_error.p, s);
 }
 
 template <typename T>
 void spk_precond_s::backward(const T* b, T* x) {
-  if (level_launch) {
+  if (per_level) {
     level_sweep<T, false>(b, x);
     return;
   }
   hipStream_t s = stream();
-  CsrView<T> v = U->view<T>();
-  hipLaunchKernelGGL((fill_sentinel_kernel<T>), dim3(blocks_for(n)),
-                     dim3(256), 0, s, x, n);
-  hipLaunchKernelGGL((sweep_kernel<T, false>), dim3(sweep_grid_u),
-                     dim3(256), 0, s, sweep_rows_u.p, (int)sweep_len_u, v.rp,
-                     v.ci, v.v, (T*)b, x, false, (T*)nullptr, sweep_error.p);
+  hipLaunchKernelGGL((fill_sentinel_kernel<T>), dim3(blocks_for(n)), dim3(256), 0, s, x, n);
   SPK_HIP_TRY(hipGetLastError());
+  tri_sweep<T, false>(upper, (T*)b, x, false, (T*)nullptr, ticket.p + 2, sweep_error.p, s);
+}
+
+void spk_precond_s::build_factors() {
+  if (L) return;
+  hipStream_t s = stream();
+  std::vector<int32_t> hrp((size_t)n + 1), hd((size_t)n), lrp((size_t)n + 1),
+      urp((size_t)n + 1);
+  SPK_HIP_TRY(hipMemcpyAsync(hrp.data(), rp.p, (n + 1) * 4, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipMemcpyAsync(hd.data(), dpos.p, n * 4, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipStreamSynchronize(s));
+  for (size_t i = 0; i < (size_t)n; ++i) {
+    lrp[i + 1] = lrp[i] + hd[i] - hrp[i] + 1;
+    urp[i + 1] = urp[i] + hrp[i + 1] - hd[i];
+  }
+  spk_csr_s* l = make_store(n, std::move(lrp));
+  try {
+    U = make_store(n, std::move(urp));
+  } catch (...) {
+    delete l;
+    throw;
+  }
+  L = l;
+  hipLaunchKernelGGL(ilu_split_kernel, dim3(blocks_for(n)), dim3(256), 0, s, pattern(),
+                     (const double*)w.p, (const int32_t*)L->rp.p, L->ci.p, L->v64.p,
+                     (const int32_t*)U->rp.p, U->ci.p, U->v64.p);
+  SPK_HIP_TRY(hipGetLastError());
+}
+
+void spk_precond_s::build_levels() {
+  if (lvl_rows_l.p) return;
+  hipStream_t s = stream();
+  DevBuf<int32_t> lvl;
+  int count[2];
+  tri_levels(pattern(), lvl, count);
+  std::vector<int32_t> h((size_t)(2 * n));
+  SPK_HIP_TRY(hipMemcpyAsync(h.data(), lvl.p, 8 * n, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipStreamSynchronize(s));
+  std::vector<int32_t> rows_l, rows_u;
+  lvl_ptr_l = group_levels({h.begin(), h.begin() + n}, rows_l);
+  lvl_ptr_u = group_levels({h.begin() + n, h.end()}, rows_u);
+  DevBuf<int32_t> l((size_t)n), u((size_t)n);
+  SPK_HIP_TRY(hipMemcpyAsync(l.p, rows_l.data(), n * 4, hipMemcpyHostToDevice, s));
+  SPK_HIP_TRY(hipMemcpyAsync(u.p, rows_u.data(), n * 4, hipMemcpyHostToDevice, s));
+  SPK_HIP_TRY(hipStreamSynchronize(s));
+  lvl_rows_l = std::move(l);
+  lvl_rows_u = std::move(u);
 }
 
 // strict part of one factor row: L drops its last entry (the unit
@@ -439,6 +495,7 @@ __global__ void strict_copy_kernel(int64_t n, const int32_t* __restrict__ rp,
 
 void spk_precond_s::build_strict() {
   if (Ls) return;
+  build_factors();
   hipStream_t s = stream();
   du64.alloc((size_t)(n > 0 ? n : 1));
   for (int f = 0; f < 2; ++f) {
@@ -597,22 +654,14 @@ void spk_precond_s::apply(const T* in, T* out) {
         break;
       }
       T* y = tmp<T>();
-      if (level_launch) {  // wide levels: one launch per level, no waiting
+      if (per_level) {  // one launch per level, no waiting
         level_sweep<T, true>(in, y);
         level_sweep<T, false>((const T*)y, out);
         break;
       }
-      hipStream_t s = stream();
-      CsrView<T> lv = L->view<T>(), uv = U->view<T>();
-      hipLaunchKernelGGL((sweep_kernel<T, true>), dim3(sweep_grid_l),
-                         dim3(256), 0, s, sweep_rows_l.p, (int)sweep_len_l,
-                         lv.rp, lv.ci, lv.v, (T*)in, y, false, out,
-                         sweep_error.p);
-      hipLaunchKernelGGL((sweep_kernel<T, false>), dim3(sweep_grid_u),
-                         dim3(256), 0, s, sweep_rows_u.p, (int)sweep_len_u,
-                         uv.rp, uv.ci, uv.v, y, out, true, (T*)nullptr,
-                         sweep_error.p);
-      SPK_HIP_TRY(hipGetLastError());
+      tri_sweep<T, true>(lower, (T*)in, y, false, out, ticket.p, sweep_error.p, stream());
+      tri_sweep<T, false>(upper, y, out, true, (T*)nullptr, ticket.p + 2, sweep_error.p,
+                          stream());
       break;
     }
     case kSpmv:
@@ -767,17 +816,11 @@ spk_status spk_ilu0_set_schedule(spk_precond M, int schedule) {
     SPK_REQUIRE(schedule >= 0 && schedule <= 2, SPK_INVALID_ARGUMENT,
                 "bad schedule");
     SPK_HIP_TRY(hipStreamSynchronize(stream()));
-    if (schedule == 0) {
-      const int64_t nl = (int64_t)M->lvl_ptr_l.size() - 1;
-      const int64_t nu = (int64_t)M->lvl_ptr_u.size() - 1;
-      M->level_launch = M->n >= kLevelLaunchRows &&
-                        std::max(nl, nu) <= kLevelLaunchMaxLevels;
-    } else {
-      M->level_launch = schedule == 1;
-    }
+    M->per_level = schedule == 1 || M->n >= kMaxTileSweepRows;
+    M->level_launch = schedule == 0 ? M->wide_levels() : schedule == 1;
     // the per-level schedule leaves ordinary values in the scratch vector;
-    // the sync-free one needs it filled with the ready sentinel
-    if (!M->level_launch) M->reset_sentinels();
+    // the sweeps in tiles need it filled with the ready sentinel
+    if (!M->per_level) M->reset_sentinels();
   });
 }
 
@@ -917,114 +960,10 @@ spk_status spk_precond_create_ilu0(spk_csr A, int modified, spk_precond* out) {
     SPK_REQUIRE(A && out, SPK_INVALID_ARGUMENT, "null argument");
     SPK_REQUIRE(A->nrows == A->ncols, SPK_INVALID_ARGUMENT,
                 "ilu0 requires a square matrix");
-    const int64_t n = A->nrows;
-    hipStream_t s = stream();
-    std::vector<int32_t> ci((size_t)A->nnz);
-    if (A->nnz)
-      SPK_HIP_TRY(hipMemcpyAsync(ci.data(), A->ci.p, A->nnz * 4,
-                                 hipMemcpyDeviceToHost, s));
-    SPK_HIP_TRY(hipStreamSynchronize(s));
-    const std::vector<int32_t>& rp = A->h_rp;
-    // diagonal positions (ilu.hpp:54-66) and factor patterns
-    std::vector<int32_t> diag_pos((size_t)n);
-    std::vector<int32_t> lrp((size_t)n + 1), urp((size_t)n + 1);
-    lrp[0] = urp[0] = 0;
-    for (int64_t i = 0; i < n; ++i) {
-      int32_t dp = -1, nl = 0;
-      for (int32_t p = rp[i]; p < rp[i + 1]; ++p) {
-        if (ci[p] == i && dp < 0) dp = p;
-        if (ci[p] < i) ++nl;
-      }
-      SPK_REQUIRE(dp >= 0, SPK_INVALID_ARGUMENT, "ilu0: missing diagonal entry");
-      diag_pos[i] = dp;
-      lrp[i + 1] = lrp[i] + nl + 1;
-      urp[i + 1] = urp[i] + (rp[i + 1] - rp[i] - nl);
-    }
-    std::vector<int32_t> lci((size_t)lrp[n]), uci((size_t)urp[n]);
-    std::vector<int32_t> lvl_l((size_t)n), lvl_u((size_t)n);
-    for (int64_t i = 0; i < n; ++i) {
-      int32_t lk = lrp[i], uk = urp[i], lv = 0;
-      for (int32_t p = rp[i]; p < rp[i + 1]; ++p) {
-        if (ci[p] < i) {
-          lci[lk++] = ci[p];
-          lv = std::max(lv, lvl_l[ci[p]] + 1);
-        } else {
-          uci[uk++] = ci[p];
-        }
-      }
-      lci[lk] = (int32_t)i;
-      lvl_l[i] = lv;
-    }
-    for (int64_t i = n - 1; i >= 0; --i) {
-      int32_t lv = 0;
-      for (int32_t p = rp[i]; p < rp[i + 1]; ++p)
-        if (ci[p] > i) lv = std::max(lv, lvl_u[ci[p]] + 1);
-      lvl_u[i] = lv;
-    }
     auto* M = new spk_precond_s();
     try {
       M->kind = spk_precond_s::kIlu;
-      M->n = n;
-      M->sweep_error.alloc(kErrorWords);
-      SPK_HIP_TRY(hipMemsetAsync(M->sweep_error.p, 0, sizeof(int) * kErrorWords, s));
-      std::vector<int32_t> rows_l, rows_u;
-      M->lvl_ptr_l = group_levels(lvl_l, rows_l);
-      M->lvl_ptr_u = group_levels(lvl_u, rows_u);
-      M->lvl_rows_l.alloc((size_t)n);
-      M->lvl_rows_u.alloc((size_t)n);
-      std::vector<int32_t> pad_l = pad_levels(rows_l, M->lvl_ptr_l);
-      std::vector<int32_t> pad_u = pad_levels(rows_u, M->lvl_ptr_u);
-      SPK_REQUIRE(pad_l.size() < (size_t)INT32_MAX && pad_u.size() < (size_t)INT32_MAX,
-                  SPK_INVALID_ARGUMENT, "too many rows for the sweep order");
-      M->sweep_len_l = (int64_t)pad_l.size();
-      M->sweep_len_u = (int64_t)pad_u.size();
-      {
-        const int64_t nl = (int64_t)M->lvl_ptr_l.size() - 1;
-        const int64_t nu = (int64_t)M->lvl_ptr_u.size() - 1;
-        M->level_launch = n >= kLevelLaunchRows &&
-                          std::max(nl, nu) <= kLevelLaunchMaxLevels;
-        // sync-free window: about four padded levels of threads
-        auto grid = [&](int64_t len, int64_t levels) {
-          const int64_t w = levels > 0 ? len / levels : 64;
-          int64_t g = (4 * w + 255) / 256;
-          const int64_t cap = std::max<int64_t>(4, 4 * ctx().num_cus);
-          g = std::max<int64_t>(4, std::min(g, cap));
-          return (unsigned)std::min<int64_t>(g, blocks_for(std::max<int64_t>(len, 1)));
-        };
-        M->sweep_grid_l = grid(M->sweep_len_l, nl);
-        M->sweep_grid_u = grid(M->sweep_len_u, nu);
-      }
-      M->sweep_rows_l.alloc(pad_l.size());
-      M->sweep_rows_u.alloc(pad_u.size());
-      SPK_HIP_TRY(hipMemcpyAsync(M->sweep_rows_l.p, pad_l.data(), pad_l.size() * 4,
-                                 hipMemcpyHostToDevice, s));
-      SPK_HIP_TRY(hipMemcpyAsync(M->sweep_rows_u.p, pad_u.data(), pad_u.size() * 4,
-                                 hipMemcpyHostToDevice, s));
-      SPK_HIP_TRY(hipMemcpyAsync(M->lvl_rows_l.p, rows_l.data(), n * 4,
-                                 hipMemcpyHostToDevice, s));
-      SPK_HIP_TRY(hipMemcpyAsync(M->lvl_rows_u.p, rows_u.data(), n * 4,
-                                 hipMemcpyHostToDevice, s));
-      M->L = make_store(n, std::move(lrp), lci);
-      M->U = make_store(n, std::move(urp), uci);
-      // numeric factorization on a copy of A's values
-      DevBuf<double> w((size_t)A->nnz);
-      DevBuf<int32_t> dpos((size_t)n);
-      SPK_HIP_TRY(hipMemcpyAsync(w.p, A->v64.p, A->nnz * 8,
-                                 hipMemcpyDeviceToDevice, s));
-      SPK_HIP_TRY(hipMemcpyAsync(dpos.p, diag_pos.data(), n * 4,
-                                 hipMemcpyHostToDevice, s));
-      for (size_t l = 0; l + 1 < M->lvl_ptr_l.size(); ++l) {
-        int cnt = M->lvl_ptr_l[l + 1] - M->lvl_ptr_l[l];
-        hipLaunchKernelGGL(ilu_factor_level_kernel, dim3(blocks_for(cnt)),
-                           dim3(256), 0, s, M->lvl_rows_l.p + M->lvl_ptr_l[l],
-                           cnt, A->rp.p, A->ci.p, dpos.p, w.p, modified);
-      }
-      if (n > 0)
-        hipLaunchKernelGGL(ilu_split_kernel, dim3(blocks_for(n)), dim3(256), 0,
-                           s, n, A->rp.p, A->ci.p, w.p, M->L->rp.p,
-                           M->L->v64.p, M->U->rp.p, M->U->v64.p);
-      SPK_HIP_TRY(hipGetLastError());
-      SPK_HIP_TRY(hipStreamSynchronize(s));
+      M->factor(*A, modified != 0);
     } catch (...) {
       delete M;
       throw;
@@ -1056,8 +995,8 @@ spk_status spk_ilu0_factor_nnz(spk_precond M, int64_t* nnz_l, int64_t* nnz_u) {
   return guarded([&] {
     SPK_REQUIRE(M && M->kind == spk_precond_s::kIlu, SPK_INVALID_ARGUMENT,
                 "not an ILU preconditioner");
-    if (nnz_l) *nnz_l = M->L->nnz;
-    if (nnz_u) *nnz_u = M->U->nnz;
+    if (nnz_l) *nnz_l = M->nnz_l;
+    if (nnz_u) *nnz_u = M->nnz_u;
   });
 }
 
@@ -1070,6 +1009,8 @@ spk_status spk_ilu0_download(spk_precond M, int64_t* l_row_ptr,
     set_error("not an ILU preconditioner");
     return SPK_INVALID_ARGUMENT;
   }
+  st = guarded([&] { M->build_factors(); });
+  if (st) return st;
   st = spk_csr_download(M->L, l_row_ptr, l_col_ind, l_vals);
   if (st) return st;
   return spk_csr_download(M->U, u_row_ptr, u_col_ind, u_vals);
@@ -1080,8 +1021,8 @@ spk_status spk_ilu0_levels(spk_precond M, int64_t* levels_l,
   return guarded([&] {
     SPK_REQUIRE(M && M->kind == spk_precond_s::kIlu, SPK_INVALID_ARGUMENT,
                 "not an ILU preconditioner");
-    if (levels_l) *levels_l = (int64_t)M->lvl_ptr_l.size() - 1;
-    if (levels_u) *levels_u = (int64_t)M->lvl_ptr_u.size() - 1;
+    if (levels_l) *levels_l = M->levels_l;
+    if (levels_u) *levels_u = M->levels_u;
   });
 }
 

@@ -1,20 +1,24 @@
 // spk_precond.hpp -- device preconditioners: identity, Jacobi, ILU(0)/MILU(0)
 // and "apply an explicit sparse approximate inverse" (one SpMV).
 //
-// ILU(0) layout in HBM:
-//   L store: strictly-lower entries of A's pattern + unit diagonal LAST in
-//            each row; U store: diagonal FIRST + upper entries (the
-//            reference's layout, ilu.hpp:123-141), int32 indices.
-//   lvl_rows_l / lvl_ptr_l: rows of the forward sweep (and of the numeric
-//            factorization) grouped by dependency level;
-//   lvl_rows_u / lvl_ptr_u: the same for the backward sweep.
-// A level is one launch; rows in a level are independent.  The numeric
-// factorization runs the reference's IKJ loop (ilu.hpp:72-115) for every row
-// of a level in one thread, with contraction of multiply-adds disabled, so
-// the factors are bit-identical to the sequential reference.
+// ILU(0) in HBM:
+//   rp, ci, dpos, w: A's pattern (columns ascending), each row's diagonal
+//            position and the factored values (L below the diagonal, U from
+//            it on);
+//   lower, upper: the two triangles in the sweeps' tile layout (spk_tri.hpp).
+// Made when something asks for them:
+//   L store: strictly-lower entries + unit diagonal LAST in each row; U
+//            store: diagonal FIRST + upper entries (the reference's layout,
+//            ilu.hpp:123-141), int32 indices;
+//   lvl_rows_l / lvl_ptr_l, lvl_rows_u / lvl_ptr_u: the rows grouped by
+//            dependency level, for the per-level schedule.
+// The numeric factorization runs the reference's IKJ loop (ilu.hpp:72-115),
+// a row per lane, with contraction of multiply-adds disabled, so the factors
+// are bit-identical to the sequential reference.
 #pragma once
 
 #include "spk_csr.hpp"
+#include "spk_tri.hpp"
 
 struct spk_precond_s {
   enum Kind { kIdentity, kJacobi, kIlu, kSpmv, kInnerCg, kInnerIr } kind = kIdentity;
@@ -24,24 +28,32 @@ struct spk_precond_s {
   spk::DevBuf<float> inv_d32;
   bool has32 = false;
   // ILU(0)
+  spk::DevBuf<int32_t> rp, ci, dpos;
+  spk::DevBuf<double> w;
+  int64_t nnz = 0, nnz_l = 0, nnz_u = 0;
+  int levels_l = 0, levels_u = 0;
+  spk::TriTiles lower, upper;
+  spk::DevBuf<int> ticket;  // of the forward and of the backward sweep
   spk_csr_s* L = nullptr;
   spk_csr_s* U = nullptr;
   spk::DevBuf<int32_t> lvl_rows_l, lvl_rows_u;
   std::vector<int32_t> lvl_ptr_l, lvl_ptr_u;
-  // the same orders with every level padded by -1 entries to a multiple of
-  // the wavefront size (the sweeps' thread -> row map)
-  spk::DevBuf<int32_t> sweep_rows_l, sweep_rows_u;
-  int64_t sweep_len_l = 0, sweep_len_u = 0;
-  unsigned sweep_grid_l = 1, sweep_grid_u = 1;  // persistent sweep grids
   spk::DevBuf<double> tmp64;  // between the sweeps; kept filled with the
   spk::DevBuf<float> tmp32;   // ready sentinel between applications
   spk::DevBuf<int> sweep_error;  // set if a sweep's bounded wait expired
-  // Sweep schedule, chosen when the factors are made: one launch per
-  // dependency level when the levels are wide (average at least
-  // kLevelLaunchWidth rows: thousands of waiting wavefronts would flood the
-  // memory system with readiness polls), the sync-free sweep otherwise
-  // (long chains of narrow levels, where launches would dominate).
+  // The schedule asked for: per-level launches only when the caller chose
+  // them; level_launch is the reported schedule, which under AUTO names the
+  // factors' shape (at least kLevelLaunchRows rows, at most
+  // kLevelLaunchMaxLevels levels) whatever runs.
+  bool per_level = false;
   bool level_launch = false;
+  spk::TriPattern pattern() const { return {n, rp.p, ci.p, dpos.p}; }
+  bool wide_levels() const;
+  void factor(const spk_csr_s& A, bool modified);
+  void sort_rows(const spk_csr_s& A, spk::DevBuf<double>& values);
+  // the L and U stores, the level lists
+  void build_factors();
+  void build_levels();
   // Approximate apply (jac_sweeps > 0): each triangular solve is replaced
   // by jac_sweeps Jacobi iterations from the diagonal-scaled right-hand
   // side, y <- r - L_s y and z <- (y - U_s z) / d_U, with L_s, U_s the

@@ -1,0 +1,135 @@
+"""ILU(0) factorization and triangular sweeps in tiles, bit for bit against
+the oracle where the layout can go wrong: sizes around a tile (2,048 rows)
+and a block (4 tiles), chains inside a tile and across tiles, rows wider than
+a batch of four entries, rows too long for the short and for the tiled
+factorization, rows of very different lengths in one level, rows given in
+another order than ascending."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def O():
+    from oracle import oracle
+    return oracle
+
+
+@pytest.fixture(scope="module")
+def spk():
+    import sparkit_amd
+    sparkit_amd.init(0)
+    return sparkit_amd
+
+
+def _banded(O, n, offsets, seed=1):
+    """Diagonally dominant, entries at the given column offsets."""
+    rng = np.random.default_rng(seed)
+    r, c, v = [np.arange(n)], [np.arange(n)], [np.full(n, 2.0 * len(offsets) + 2)]
+    for o in offsets:
+        i = np.arange(max(0, -o), min(n, n - o))
+        r.append(i)
+        c.append(i + o)
+        v.append(rng.uniform(-1, 1, len(i)))
+    return O.make_matrix(n, n, np.concatenate(r), np.concatenate(c), np.concatenate(v))
+
+
+def _arrow(O, n, width):
+    """Two rows and columns of `width` entries among rows of three."""
+    rng = np.random.default_rng(3)
+    rows, cols = [np.arange(n), np.arange(1, n), np.arange(n - 1)], \
+                 [np.arange(n), np.arange(n - 1), np.arange(1, n)]
+    far = rng.choice(n - 2, width, replace=False)
+    for i in (n // 2, n - 1):
+        rows += [np.full(width, i), far]
+        cols += [far, np.full(width, i)]
+    r, c = np.concatenate(rows), np.concatenate(cols)
+    v = np.where(r == c, 4.0 * width, rng.uniform(-1, 1, len(r)))
+    return O.make_matrix(n, n, r, c, v)
+
+
+def _check(O, spk, A, modified=False):
+    Lr, Ur = O.ilu0(A, modified)
+    Ad = spk.CsrMatrix.from_oracle(A)
+    F = (spk.milu0 if modified else spk.ilu0)(Ad)
+    r = O.uniform_pm1(5, A.nrows)
+    rd = spk.DeviceVector.from_numpy(r)
+    y, z = spk.DeviceVector.zeros(A.nrows), spk.DeviceVector.zeros(A.nrows)
+    y_ref = O.forward_solve(Lr, r)
+    z_ref = O.backward_solve(Ur, y_ref)
+    for _ in range(2):  # the second application finds the first one's scratch
+        spk.ilu_apply(F, rd, z)
+        assert np.array_equal(z.numpy(), z_ref)
+    F.forward(rd, y)
+    assert np.array_equal(y.numpy(), y_ref)
+    F.backward(y, z)
+    assert np.array_equal(z.numpy(), z_ref)
+    zz = spk.DeviceVector.from_numpy(r)  # in place
+    F.apply(zz, zz)
+    assert np.array_equal(zz.numpy(), z_ref)
+    z32 = spk.DeviceVector.zeros(A.nrows, np.float32)
+    F.apply(spk.DeviceVector.from_numpy(r, np.float32), z32)
+    # FP32 factors and vector: a few roundings of 2^-24 per entry; the
+    # matrices are diagonally dominant, so errors do not grow
+    assert np.linalg.norm(z32.numpy() - z_ref) <= 1e-5 * np.linalg.norm(z_ref)
+    (lrp, lci, lv), (urp, uci, uv) = F.factors()
+    assert np.array_equal(lci, Lr.col_ind) and np.array_equal(lv, Lr.vals)
+    assert np.array_equal(uci, Ur.col_ind) and np.array_equal(uv, Ur.vals)
+
+
+@pytest.mark.parametrize("n", [2, 3, 64, 65, 2047, 2048, 2049, 8191, 8192, 8193, 20000])
+def test_chain(O, spk, n):
+    """One row a level: every step a single lane."""
+    print("chain", n, flush=True)
+    _check(O, spk, _banded(O, n, (-1, 1)))
+
+
+@pytest.mark.parametrize("offsets", [(-2049, 2049), (-8192, -1, 1, 8192), (-100, 3),
+                                     (-9000, -5000, -2000, -1, 1, 2000, 5000, 9000)])
+def test_dependencies_across_tiles(O, spk, offsets):
+    print("offsets", offsets, flush=True)
+    for modified in (False, True):
+        _check(O, spk, _banded(O, 18001, offsets), modified)
+
+
+@pytest.mark.parametrize("side", [4, 5, 8, 15, 16])
+def test_wide_rows(O, spk, side):
+    """4: the short factorization's widest rows; 15: the tiled one's (31
+    entries); 16: a launch per level."""
+    print("side", side, flush=True)
+    near = [k * k + k - 1 for k in range(1, side + 1)]
+    _check(O, spk, _banded(O, 5000, [-k for k in near] + near))
+
+
+@pytest.mark.parametrize("width", [10, 300])
+def test_mixed_lengths(O, spk, width):
+    print("arrow", width, flush=True)
+    _check(O, spk, _arrow(O, 4500, width))
+
+
+def test_ragged_grids(O, spk):
+    for dims in ((13, 11, 9), (45, 3, 31), (100, 37, 3)):
+        print("grid", dims, flush=True)
+        for modified in (False, True):
+            _check(O, spk, O.convdiff_3d(*dims, 1.0, 0.3, 0.2, 0.1), modified)
+
+
+def test_diagonal_matrix(O, spk):
+    """No dependencies: one level."""
+    _check(O, spk, _banded(O, 5000, ()))
+
+
+def test_rows_in_another_order(O, spk):
+    """A store whose rows list their columns descending: the factors are
+    those of the ascending one."""
+    A = O.convdiff_3d(9, 8, 7, 1.0, 0.3, 0.2, 0.1)
+    ci, v = np.array(A.col_ind), np.array(A.vals)
+    for i in range(A.nrows):
+        s = slice(A.row_ptr[i], A.row_ptr[i + 1])
+        ci[s], v[s] = ci[s][::-1], v[s][::-1]
+    F = spk.ilu0(spk.CsrMatrix.from_host(A.nrows, A.ncols, A.row_ptr, ci, v))
+    G = spk.ilu0(spk.CsrMatrix.from_oracle(A))
+    for a, b in zip(F.factors(), G.factors()):
+        for p, q in zip(a, b):
+            assert np.array_equal(p, q)
