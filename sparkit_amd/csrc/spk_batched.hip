@@ -536,7 +536,20 @@ struct spk_batch_s {
   DevBuf<double> ell_v64;
   DevBuf<int32_t> iters, outer, conv;
   DevBuf<double> relres;
-  spk_batch_tuning tuning{256, 2, 0, 0};
+  spk_batch_tuning tuning{512, 2, kSmallSystem, 0};
+  // The launch shape until a caller sets or tunes another, by the largest
+  // system: a pass over its rows is a few loads per lane at 512 threads up to
+  // kSmallSystem rows, two workgroups a CU; the largest system's solve is the
+  // whole solve's tail, so beyond that it gets 1,024 threads.  p sits in LDS
+  // in both.  (512, 2) / (1024, 1) / 256 threads and p in HBM, ms: 256
+  // systems of 12^2-30^2 0.42 / 0.51 / 0.56, 4,096 of 12^2-40^2 3.4 / 5.9 /
+  // 4.3, 256 of 32^2-96^2 6.4 / 4.75 / 12.9, 256 of 96^2-200^2 79 / 59 / 138;
+  // FP64, 256 of 32^2-96^2: 12.0 / 8.3 / 15.7.
+  static constexpr int kSmallSystem = 2048;
+  static spk_batch_tuning default_tuning(int64_t max_rows) {
+    if (max_rows <= kSmallSystem) return {512, 2, kSmallSystem, 0};
+    return {1024, 1, 16384, 0};
+  }
   // captured graphs, keyed by (b, x, config, tuning, precision)
   struct Key {
     const void* b;
@@ -566,6 +579,7 @@ struct spk_batch_s {
       max_rows = std::max(max_rows, h_row[(size_t)k + 1] - h_row[(size_t)k]);
     SPK_REQUIRE(max_rows < ((int64_t)1 << 29), SPK_INVALID_ARGUMENT,
                 "a system of the batch holds 2^29 rows or more");
+    tuning = default_tuning(max_rows);
     sys_row.alloc((size_t)K + 1);
     SPK_HIP_TRY(hipMemcpyAsync(sys_row.p, h_row.data(), (K + 1) * 8,
                                hipMemcpyHostToDevice, s));
