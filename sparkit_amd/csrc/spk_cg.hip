@@ -36,6 +36,10 @@
 // step parity, as the kernel that reads rz_k writes rz_{k+1}.  Jacobi-PCG
 // with more SpMV row blocks than that keeps K1's finisher (alpha from the
 // parity slot) and hands off from K2 on.
+// Matrices whose rows fit the chip's registers (up to nine entries a row and
+// some 340,000-460,000 rows) run many steps in one launch instead
+// (spk_cgstep.hpp), with M_L Jacobi or the identity.
+#include "spk_cgstep.hpp"
 #include "spk_solver_common.hpp"
 
 namespace spk {
@@ -44,13 +48,37 @@ namespace {
 struct CgState {
   double bnorm, rz, alpha, beta, resnorm, tol;
   int64_t iters;
-  int32_t done, converged, collect, pad;
+  int32_t done, converged, collect;
+  int32_t expired;  // a grid exchange's bounded wait ended without its value
   double* history;
   // one-kernel hand-off path: rz by step parity (a kernel reads one and
   // writes the other), the step whose residual update ran
   double rzb[2];
   int64_t k2_step;
 };
+
+// many steps in one launch (spk_cgstep.hpp): is_converged() and the
+// bookkeeping of compute_new_residual, conjugate_gradient.hpp:248-276
+struct CgCtl {
+  CgState* st;
+  __device__ bool skip() const { return st->done != 0; }
+  __device__ double rz() const { return st->rz; }
+  __device__ bool ends(double rr) const { return sqrt(rr) / st->bnorm < st->tol; }
+  __device__ void record(int step, double rr) const {
+    if (st->collect) st->history[st->iters + step] = sqrt(rr);
+  }
+  __device__ void finish(int steps, double rr, double, double rz, bool ended,
+                         bool ok) const {
+    st->iters += steps;
+    st->resnorm = sqrt(rr);
+    st->rz = rz;
+    if (ended && ok) st->converged = 1;
+    if (ended) st->done = 1;
+  }
+};
+constexpr int kCgSteps = 4096;  // steps of one launch, at most
+constexpr int kCgQueue = 8;     // launches between two looks at the state,
+constexpr int kCgLook = 256;    // unless they hold this many steps
 
 // launch gates of the one-kernel hand-off path
 struct GateNotDone {
@@ -214,14 +242,15 @@ void cg_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
   const int* done = &S->done;
   // the one-kernel hand-off needs few partials: every block of the next
   // kernel reads all of them
-  const bool handoff = right_id && (jac || spmv_left) &&
+  const bool steps_fit = right_id && (jac || is_identity(ML)) && cg_steps_fit<T>(*A);
+  const bool handoff = !steps_fit && right_id && (jac || spmv_left) &&
                        spmv_partials_count(*A) <= kProMaxPartials &&
                        (!spmv_left || spmv_partials_count(*ML->M) <= kProMaxPartials) &&
                        pro_grid(n) <= kProMaxPartials;
   // Jacobi-PCG whose SpMV has too many row blocks for a prologue: the SpMV
   // keeps its finisher (alpha), the r update hands its partials to the
   // x / p pass
-  const bool mixed = !handoff && right_id && jac && pro_grid(n) <= kProMaxPartials;
+  const bool mixed = !steps_fit && !handoff && right_id && jac && pro_grid(n) <= kProMaxPartials;
   double* part1 = nullptr;
   double* part2 = nullptr;
   double* part3 = nullptr;
@@ -232,25 +261,26 @@ void cg_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
     part3 = (double*)ws.get(kWsCg + 9, pb);
   }
 
-  auto issue = [&](int64_t k) {
-    if (k % cfg->restart == 0) {  // reorthogonalize(), :216-230
-      if (jac) {
-        launch_spmv(*A, (const T*)x,
-                    EpiCgRestartJacobi<T>{b, invd, r, p, S, done, (int)(k & 1)}, s);
-      } else {
-        launch_spmv(*A, (const T*)x, EpiCgResidual<T>{b, r, done}, s);
-        apply_precond(ML, n, (const T*)r, z);
-        const int par = (int)(k & 1);
-        launch_reduce<1>(n, [=] __device__(int64_t i, double* acc) {
-          T zi = z[i];
-          p[i] = zi;
-          acc[0] += (double)r[i] * (double)zi;
-        }, [=] __device__(const double* t) {
-          S->rz = t[0];
-          S->rzb[par] = t[0];
-        }, done);
-      }
+  auto restart = [&](int64_t k) {  // reorthogonalize(), :216-230
+    if (jac) {
+      launch_spmv(*A, (const T*)x,
+                  EpiCgRestartJacobi<T>{b, invd, r, p, S, done, (int)(k & 1)}, s);
+    } else {
+      launch_spmv(*A, (const T*)x, EpiCgResidual<T>{b, r, done}, s);
+      apply_precond(ML, n, (const T*)r, z);
+      const int par = (int)(k & 1);
+      launch_reduce<1>(n, [=] __device__(int64_t i, double* acc) {
+        T zi = z[i];
+        p[i] = zi;
+        acc[0] += (double)r[i] * (double)zi;
+      }, [=] __device__(const double* t) {
+        S->rz = t[0];
+        S->rzb[par] = t[0];
+      }, done);
     }
+  };
+  auto issue = [&](int64_t k) {
+    if (k % cfg->restart == 0) restart(k);
     if (handoff || mixed) {
       // One-kernel hand-off: no finisher kernels.  K1 q = A p (partials
       // <p,q>); K2 sums them itself -> alpha, r -= alpha q, partials;
@@ -422,9 +452,29 @@ void cg_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
     }
   };
   auto is_done = [&]() { return st.download().done != 0; };
-  chunked_loop(cfg->max_iterations, issue, is_done);
+  if (steps_fit) {
+    const GridLink link = grid_link();
+    const int* expired = link.expired;
+    for (int64_t k = 0; k < cfg->max_iterations;) {
+      // short restart intervals: several launches between two looks
+      int64_t queued = 0;
+      for (int j = 0; j < kCgQueue && queued < kCgLook && k < cfg->max_iterations; ++j) {
+        if (k % cfg->restart == 0) restart(k);
+        const int64_t m = std::min<int64_t>(
+            kCgSteps, std::min(cfg->restart - k % cfg->restart, cfg->max_iterations - k));
+        launch_cg_steps(*A, invd, x, r, p, z, (int)m, CgCtl{S}, link);
+        k += m;
+        queued += m;
+      }
+      launch_map(1, [=] __device__(int64_t) { S->expired = *expired; });
+      if (is_done()) break;
+    }
+  } else {
+    chunked_loop(cfg->max_iterations, issue, is_done);
+  }
 
   h = st.download();
+  if (h.expired) check_link(grid_link());
   out->residual_norm = h.resnorm;
   out->computed_iterations = h.iters;
   out->converged = h.converged;
@@ -540,7 +590,8 @@ extern "C" spk_status spk_cg_solve_noalloc(spk_csr A, spk_precond M_left,
     const size_t vb = arena_round((size_t)(n > 0 ? n : 1) * (fp32 ? 4 : 8));
     const size_t partials =
         std::max(blocks, (size_t)2 * (size_t)vec_grid(n > 0 ? n : 1));
-    size_t need = 5 * vb + arena_round(sizeof(double) * partials) +
+    size_t need = 5 * vb + arena_round(kLinkWords * sizeof(unsigned long long)) +
+                  arena_round(sizeof(double) * partials) +
                   3 * arena_round(sizeof(double) * 2 * (size_t)kProMaxPartials) +
                   arena_round(1024);
     if (cfg->collect_residuals)

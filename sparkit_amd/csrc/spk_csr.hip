@@ -131,6 +131,9 @@ void upload_plan(spk_csr_s& A, const std::vector<int32_t>& blocks) {
   for (size_t b = 0; b < blocks.size(); ++b)
     plan[b] = make_int2(blocks[b], A.h_rp[blocks[b]]);
   A.nblocks = (int)blocks.size() - 1;
+  A.max_len = 0;
+  for (size_t i = 0; i + 1 < A.h_rp.size(); ++i)
+    A.max_len = std::max(A.max_len, (int)(A.h_rp[i + 1] - A.h_rp[i]));
   A.plan.alloc(plan.size());
   SPK_HIP_TRY(hipMemcpyAsync(A.plan.p, plan.data(), plan.size() * sizeof(int2),
                              hipMemcpyHostToDevice, stream()));

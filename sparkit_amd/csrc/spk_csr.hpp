@@ -78,6 +78,7 @@ struct spk_csr_s {
   bool short_idx = false;
   const int16_t* short_cols() const { return short_idx ? c16.p : nullptr; }
   int nblocks = 0, nlong = 0;
+  int max_len = 0;  // entries of the longest row
   std::vector<int32_t> h_rp;  // host copy of the row offsets
   // Column panels (empty: none).  Panel p holds the entries with columns in
   // [p W, (p+1) W) as a store of its own; an SpMV runs the panels in column

@@ -10,6 +10,7 @@
 // The FP64 work per refinement step is one SpMV, one norm and one update;
 // everything inside the inner solve streams FP32 values (8 bytes per
 // nonzero instead of 12).
+#include "spk_cgstep.hpp"
 #include "spk_solver_common.hpp"
 
 namespace spk {
@@ -51,12 +52,32 @@ struct EpiResidualNorm {  // r = b - A x, partial |r|^2
 struct RcgState {
   double bnorm, rnorm, rupd, rz, alpha, beta, tol, delta;
   int64_t iters, updates;
-  int32_t hold, converged, pad0, pad1;
+  int32_t hold, converged, pad;
+  int32_t expired;  // a grid exchange's bounded wait ended without its value
   // one-kernel hand-off: rz by step parity, and the step whose second
   // kernel ran (gates the third)
   double rzb[2];
   int64_t k2_step;
 };
+
+// many FP32 steps in one launch (spk_cgstep.hpp): rcg_due's test
+struct RcgCtl {
+  RcgState* st;
+  __device__ bool skip() const { return st->hold != 0; }
+  __device__ double rz() const { return st->rz; }
+  __device__ bool ends(double rr) const {
+    const double rn = sqrt(rr);
+    return rn <= st->delta * st->rupd || rn / st->bnorm < st->tol;
+  }
+  __device__ void record(int, double) const {}
+  __device__ void finish(int steps, double, double rz0, double rz, bool ended,
+                         bool) const {
+    st->iters += steps;
+    st->rz = ended ? rz0 : rz;  // the update's beta divides by the last step's
+    if (ended) st->hold = 1;
+  }
+};
+constexpr int kRcgSteps = 4096;  // steps of one launch, at most
 
 struct RcgGateRun {
   const int* hold;
@@ -152,7 +173,9 @@ void cg_reliable(spk_csr_s* A, spk_precond_s* M, const spk_ir_config* cfg,
   const float* invd = jac ? M->inv_diag<float>() : nullptr;
   // the one-kernel hand-off (every block of the next kernel sums the
   // previous partials) when the partials are few
-  const bool handoff = (jac || ident || spai) &&
+  const bool steps_fit = (jac || ident) && cg_steps_fit<float>(*A);
+  const GridLink link = steps_fit ? grid_link() : GridLink{};
+  const bool handoff = !steps_fit && (jac || ident || spai) &&
                        spmv_partials_count(*A) <= kProMaxPartials &&
                        pro_grid(n) <= kProMaxPartials &&
                        (!spai || spmv_partials_count(*M->M) <= kProMaxPartials);
@@ -353,6 +376,18 @@ void cg_reliable(spk_csr_s* A, spk_precond_s* M, const spk_ir_config* cfg,
     {
       TraceRange steps_("reliable CG: FP32 steps");
       while (ran < cfg->max_inner) {
+        if (steps_fit) {
+          launch_cg_steps(*A, invd, xi, r32, p, z,
+                          (int)std::min<int64_t>(cfg->max_inner - ran, kRcgSteps),
+                          RcgCtl{S}, link);
+          const int* expired = link.expired;
+          launch_map(1, [=] __device__(int64_t) { S->expired = *expired; });
+          h = st.download();
+          if (h.expired) check_link(link);
+          ran = h.iters;
+          if (h.hold) break;
+          continue;
+        }
         const int64_t e = std::min(cfg->max_inner - ran, chunk);
         for (int64_t j = 0; j < e; ++j, ++issued) step();
         h = st.download();

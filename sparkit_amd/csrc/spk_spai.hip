@@ -804,6 +804,7 @@ spk_csr_s* clone_pattern(const spk_csr_s& A) {
                                hipMemcpyDeviceToDevice, s));
     M->nblocks = A.nblocks;
     M->nlong = A.nlong;
+    M->max_len = A.max_len;
   } catch (...) {
     delete M;
     throw;
