@@ -153,7 +153,7 @@ void bicgstab_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
   //       partials |r|^2, <r^, r> for the next K1
   // A step's |r| test runs in the next step's K1, or in a tail kernel
   // after the last step.
-  const bool handoff = spmv_partials_count(*A) <= kProMaxPartials &&
+  const bool handoff = spmv_partials_count<T>(*A) <= kProMaxPartials &&
                        pro_grid(n) <= kProMaxPartials;
   double* pq[4] = {nullptr, nullptr, nullptr, nullptr};
   int c_v = 0, c_s = 0, c_t = 0, c_r = 0;

@@ -244,8 +244,8 @@ void cg_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
   // kernel reads all of them
   const bool steps_fit = right_id && (jac || is_identity(ML)) && cg_steps_fit<T>(*A);
   const bool handoff = !steps_fit && right_id && (jac || spmv_left) &&
-                       spmv_partials_count(*A) <= kProMaxPartials &&
-                       (!spmv_left || spmv_partials_count(*ML->M) <= kProMaxPartials) &&
+                       spmv_partials_count<T>(*A) <= kProMaxPartials &&
+                       (!spmv_left || spmv_partials_count<T>(*ML->M) <= kProMaxPartials) &&
                        pro_grid(n) <= kProMaxPartials;
   // Jacobi-PCG whose SpMV has too many row blocks for a prologue: the SpMV
   // keeps its finisher (alpha), the r update hands its partials to the

@@ -161,7 +161,7 @@ void cgs_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
   // test; partials rho_new = <r^, r>); pass 3 (beta; u, p).  Block 0 records
   // state no block of the same kernel reads (rho by step parity); a block
   // 0 that ends the solve makes every block of its kernel skip its pass.
-  const bool handoff = spmv_partials_count(*A) <= kProMaxPartials &&
+  const bool handoff = spmv_partials_count<T>(*A) <= kProMaxPartials &&
                        pro_grid(n) <= kProMaxPartials;
   double* pq[3] = {nullptr, nullptr, nullptr};
   if (handoff) {

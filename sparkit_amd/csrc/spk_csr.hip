@@ -99,6 +99,109 @@ int grid_for(int64_t n, int block = 256) {
   return (int)std::min<int64_t>(std::max<int64_t>(g, 1), 65536);
 }
 
+// ---- row patterns: distinct rows go into a small open-addressed table by a
+// hash of their (column - row, value bits) list
+constexpr int kPatSlots = 1024;
+struct PatTable {
+  unsigned long long key[kPatSlots];  // 0: free
+  int rep[kPatSlots];                 // a row with that hash
+  int id[kPatSlots];
+  int count, fail;
+};
+
+__device__ __forceinline__ unsigned long long pat_hash(const int32_t* rp, const int32_t* ci,
+                                                       const double* v, int r) {
+  const int a = rp[r], len = rp[r + 1] - a;
+  unsigned long long h = 0x9E3779B97F4A7C15ull + (unsigned)len;
+  for (int k = 0; k < len; ++k) {
+    h ^= (unsigned)(ci[a + k] - r);
+    h *= 0xBF58476D1CE4E5B9ull;
+    h ^= h >> 29;
+    h ^= (unsigned long long)__double_as_longlong(v[a + k]);
+    h *= 0x94D049BB133111EBull;
+    h ^= h >> 32;
+  }
+  return h | 1;
+}
+
+__global__ void pat_clear_kernel(PatTable* t) {
+  for (int k = threadIdx.x; k < kPatSlots; k += blockDim.x) t->key[k] = 0;
+  if (threadIdx.x == 0) t->count = t->fail = 0;
+}
+
+__global__ __launch_bounds__(256) void pat_insert_kernel(int64_t n,
+                                                         const int32_t* __restrict__ rp,
+                                                         const int32_t* __restrict__ ci,
+                                                         const double* __restrict__ v,
+                                                         PatTable* t) {
+  for (int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x; r < n;
+       r += (int64_t)gridDim.x * 256) {
+    if (__hip_atomic_load(&t->fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+    const unsigned long long h = pat_hash(rp, ci, v, (int)r);
+    int slot = (int)(h >> 20) & (kPatSlots - 1);
+    for (int probe = 0; probe < kPatSlots; ++probe, slot = (slot + 1) & (kPatSlots - 1)) {
+      unsigned long long k =
+          __hip_atomic_load(&t->key[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (k == 0) {
+        k = atomicCAS(&t->key[slot], 0ull, h);
+        if (k == 0) {
+          t->rep[slot] = (int)r;
+          if (atomicAdd(&t->count, 1) >= kPatMax) atomicOr(&t->fail, 1);
+          break;
+        }
+      }
+      if (k == h) break;
+    }
+  }
+}
+
+// ids and lists of the table's rows; one block
+__global__ __launch_bounds__(256) void pat_lists_kernel(const int32_t* __restrict__ rp,
+                                                        const int32_t* __restrict__ ci,
+                                                        const double* __restrict__ v,
+                                                        PatTable* t, int width,
+                                                        int32_t* __restrict__ off,
+                                                        int32_t* __restrict__ len,
+                                                        double* __restrict__ v64,
+                                                        float* __restrict__ v32) {
+  __shared__ int next;
+  if (threadIdx.x == 0) next = 0;
+  __syncthreads();
+  for (int s = threadIdx.x; s < kPatSlots; s += 256) {
+    if (t->key[s] == 0) continue;
+    const int id = atomicAdd(&next, 1);
+    t->id[s] = id;
+    const int r = t->rep[s], a = rp[r], n = rp[r + 1] - a;
+    len[id] = n;
+    for (int k = 0; k < width; ++k) {
+      off[id * width + k] = k < n ? ci[a + k] - r : 0;
+      v64[id * width + k] = k < n ? v[a + k] : 0.0;
+      v32[id * width + k] = k < n ? (float)v[a + k] : 0.0f;
+    }
+  }
+}
+
+// every row's list, compared entry by entry: two rows with one hash and
+// different lists fail the whole store
+__global__ __launch_bounds__(256) void pat_assign_kernel(
+    int64_t n, const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
+    const double* __restrict__ v, PatTable* t, int width, const int32_t* __restrict__ off,
+    const int32_t* __restrict__ len, const double* __restrict__ v64,
+    uint8_t* __restrict__ out) {
+  const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (r >= n) return;
+  const unsigned long long h = pat_hash(rp, ci, v, (int)r);
+  int slot = (int)(h >> 20) & (kPatSlots - 1);
+  while (t->key[slot] != h && t->key[slot] != 0) slot = (slot + 1) & (kPatSlots - 1);
+  const int id = t->id[slot], a = rp[r], m = rp[r + 1] - a;
+  bool same = t->key[slot] == h && len[id] == m;
+  for (int k = 0; same && k < m; ++k)
+    same = off[id * width + k] == ci[a + k] - (int)r &&
+           __double_as_longlong(v64[id * width + k]) == __double_as_longlong(v[a + k]);
+  if (!same) atomicOr(&t->fail, 2);
+  out[r] = (uint8_t)id;
+}
+
 }  // namespace
 
 void finish_store(spk_csr_s& A, bool validate_cols) {
@@ -110,9 +213,14 @@ void finish_store(spk_csr_s& A, bool validate_cols) {
   SPK_HIP_TRY(hipStreamSynchronize(s));
   SPK_REQUIRE(A.h_rp[0] == 0 && A.h_rp[A.nrows] == A.nnz, SPK_INVALID_ARGUMENT,
               "row_ptr must start at 0 and end at nnz");
-  for (int64_t r = 0; r < A.nrows; ++r)
-    SPK_REQUIRE(A.h_rp[r] <= A.h_rp[r + 1], SPK_INVALID_ARGUMENT,
-                "row_ptr must be non-decreasing");
+  int lo = 0, hi = 0;  // shortest (negative: decreasing) and longest row
+  for (int64_t r = 0; r < A.nrows; ++r) {
+    const int len = A.h_rp[(size_t)r + 1] - A.h_rp[(size_t)r];
+    lo = len < lo ? len : lo;
+    hi = len > hi ? len : hi;
+  }
+  SPK_REQUIRE(lo >= 0, SPK_INVALID_ARGUMENT, "row_ptr must be non-decreasing");
+  A.max_len = hi;
   if (validate_cols && A.nnz > 0) {
     DevBuf<int> bad(1);
     SPK_HIP_TRY(hipMemsetAsync(bad.p, 0, sizeof(int), s));
@@ -124,6 +232,47 @@ void finish_store(spk_csr_s& A, bool validate_cols) {
     SPK_REQUIRE(!hbad, SPK_INVALID_ARGUMENT, "column index out of range");
   }
   upload_plan(A, build_spmv_plan(A.h_rp.data(), A.nrows, &A.nlong));
+  build_patterns(A);
+}
+
+void build_patterns(spk_csr_s& A) {
+  A.pat_count = 0;
+  if (A.nrows < kPatMinRows || A.nrows != A.ncols || A.max_len < 1 ||
+      A.max_len > kPatMaxLen)
+    return;
+  hipStream_t s = stream();
+  DevBuf<PatTable> t(1);
+  struct { int count, fail; } h;
+  auto look = [&] {
+    SPK_HIP_TRY(hipMemcpyAsync(&h, &t.p->count, sizeof(h), hipMemcpyDeviceToHost, s));
+    SPK_HIP_TRY(hipStreamSynchronize(s));
+  };
+  const int n256 = grid_for(A.nrows);
+  hipLaunchKernelGGL(pat_clear_kernel, dim3(1), dim3(256), 0, s, t.p);
+  hipLaunchKernelGGL(pat_insert_kernel, dim3(std::min(n256, 2048)), dim3(256), 0, s, A.nrows,
+                     (const int32_t*)A.rp.p, (const int32_t*)A.ci.p,
+                     (const double*)A.v64.p, t.p);
+  SPK_HIP_TRY(hipGetLastError());
+  look();
+  const size_t entries = (size_t)h.count * (size_t)A.max_len;
+  if (h.fail || h.count > kPatMax || entries > (size_t)kPatMaxEntries) return;
+  A.pat_id.alloc((size_t)A.nrows);
+  A.pat_off.alloc(entries);
+  A.pat_len.alloc((size_t)h.count);
+  A.pat_v64.alloc(entries);
+  A.pat_v32.alloc(entries);
+  hipLaunchKernelGGL(pat_lists_kernel, dim3(1), dim3(256), 0, s, (const int32_t*)A.rp.p,
+                     (const int32_t*)A.ci.p, (const double*)A.v64.p, t.p, A.max_len,
+                     A.pat_off.p, A.pat_len.p, A.pat_v64.p, A.pat_v32.p);
+  hipLaunchKernelGGL(pat_assign_kernel, dim3((unsigned)((A.nrows + 255) / 256)), dim3(256), 0,
+                     s, A.nrows, (const int32_t*)A.rp.p, (const int32_t*)A.ci.p,
+                     (const double*)A.v64.p, t.p, A.max_len, (const int32_t*)A.pat_off.p,
+                     (const int32_t*)A.pat_len.p, (const double*)A.pat_v64.p, A.pat_id.p);
+  SPK_HIP_TRY(hipGetLastError());
+  const int count = h.count;
+  look();
+  if (h.fail) return;
+  A.pat_count = count;
 }
 
 void upload_plan(spk_csr_s& A, const std::vector<int32_t>& blocks) {
@@ -131,9 +280,6 @@ void upload_plan(spk_csr_s& A, const std::vector<int32_t>& blocks) {
   for (size_t b = 0; b < blocks.size(); ++b)
     plan[b] = make_int2(blocks[b], A.h_rp[blocks[b]]);
   A.nblocks = (int)blocks.size() - 1;
-  A.max_len = 0;
-  for (size_t i = 0; i + 1 < A.h_rp.size(); ++i)
-    A.max_len = std::max(A.max_len, (int)(A.h_rp[i + 1] - A.h_rp[i]));
   A.plan.alloc(plan.size());
   SPK_HIP_TRY(hipMemcpyAsync(A.plan.p, plan.data(), plan.size() * sizeof(int2),
                              hipMemcpyHostToDevice, stream()));

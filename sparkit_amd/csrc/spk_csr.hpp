@@ -79,6 +79,22 @@ struct spk_csr_s {
   const int16_t* short_cols() const { return short_idx ? c16.p : nullptr; }
   int nblocks = 0, nlong = 0;
   int max_len = 0;  // entries of the longest row
+  // Row patterns (pat_count == 0: none): a store whose rows repeat a few
+  // lists of (column - row, value), as a constant-coefficient stencil's do,
+  // keeps a byte per row that names the list, and the lists.  The plain
+  // layout's SpMV then reads a byte a row instead of 12 (FP32: 8) an entry.
+  // The lists are found and every row is compared with its own when the
+  // store is made; ci and v64 stay for everything else.
+  int pat_count = 0;
+  spk::DevBuf<uint8_t> pat_id;   // [nrows]
+  spk::DevBuf<int32_t> pat_off;  // [pat_count][max_len]
+  spk::DevBuf<int32_t> pat_len;  // [pat_count]
+  spk::DevBuf<double> pat_v64;   // [pat_count][max_len]
+  spk::DevBuf<float> pat_v32;
+  template <typename T>
+  bool patterned() const {
+    return pat_count > 0 && !(std::is_same<T, float>::value && half32);
+  }
   std::vector<int32_t> h_rp;  // host copy of the row offsets
   // Column panels (empty: none).  Panel p holds the entries with columns in
   // [p W, (p+1) W) as a store of its own; an SpMV runs the panels in column
@@ -177,6 +193,8 @@ namespace spk {
 // Build the row-block plan from host row offsets: row-block boundaries.
 std::vector<int32_t> build_spmv_plan(const int32_t* rp, int64_t nrows,
                                      int* nlong);
+// Row patterns of a finished square store, if its rows repeat few enough.
+void build_patterns(spk_csr_s& A);
 // Upload a plan ({first row, first nonzero} per boundary) into A.plan.
 void upload_plan(spk_csr_s& A, const std::vector<int32_t>& blocks);
 // Finish a store whose rp/ci/v64 are filled on the device: copies rp back,
@@ -536,6 +554,133 @@ __global__ __launch_bounds__(kXtThreads) void xtile_spmv_kernel(
   }
 }
 
+// ------------------------------------------------------------- row patterns
+
+constexpr int kPatBlock = 512;
+constexpr int kPatMaxLen = 15;    // entries a row: the row kernel sums such
+                                  // rows with one lane, in storage order too
+constexpr int kPatMax = 255;      // lists a store may have
+constexpr int kPatMaxEntries = 1024;  // and their entries: 12 KB of LDS
+// Below, the row kernel is as fast (its launch and load chain, not its bytes,
+// take the time: 134,784 rows 7-point 4.9 us here with four rows a thread,
+// 5.1 there).
+constexpr int64_t kPatMinRows = 1 << 17;
+constexpr int kXcds = 8;
+// Rows a thread: two (262,144 rows 7-point 3.6 us against 5.1 with four,
+// 2.1M rows 12.3 / 12.6), four beyond 4.2M rows, where two would leave more
+// block sums than the next kernel's prologue reads (192^3: 34.5 / 35.8 us
+// alone, 47.4 / 46.4 with the sum); eight were slower everywhere (49.7).
+inline int pattern_rows(int64_t n) { return n <= (int64_t)4096 * kPatBlock * 2 ? 2 : 4; }
+
+template <typename T>
+struct PatView {
+  const uint8_t* __restrict__ id;
+  const int32_t* __restrict__ off;
+  const int32_t* __restrict__ len;
+  const T* __restrict__ v;
+  int n, count, width;  // width: entries a list is padded to
+};
+
+// A thread sums R rows: the lists are in LDS, so a row's gathers
+// depend on its one byte alone and all of a thread's are in flight together;
+// the products are rounded and added in storage order (the row kernel's and
+// sparse_blas.hpp:26-31's arithmetic, bit for bit).  K: entries a row may
+// have.
+// Bound: x and y from HBM and the gathers' reads through the caches.  FP64,
+// row kernel -> this: 192^3 7-point 133 -> 36 us (17 bytes a row: 3.4 TB/s;
+// as B_spmv 20 TB/s), 128^3 41 -> 12, 2000^2 5-point 54 -> 17; FP32 192^3 96
+// -> 19.
+template <typename T, int K, int R, typename Epi>
+__global__ __launch_bounds__(kPatBlock) void pattern_spmv_kernel(
+    PatView<T> A, const T* __restrict__ x, Epi epi, double* partials) {
+#pragma clang fp contract(off)
+  __shared__ int off[kPatMaxEntries];
+  __shared__ T val[kPatMaxEntries];
+  __shared__ int len[kPatMax + 1];
+  __shared__ double red[kPatBlock / 64];
+  if (epi.done && *epi.done) return;
+  // consecutive blocks go to the XCDs in turn: an XCD takes a contiguous range
+  // of the rows, so that its neighbours' x stays in its own L2 (192^3 38.3 ->
+  // 35.8 us, 2000^2 20.8 -> 17.4)
+  const int b = (int)(blockIdx.x % kXcds) * (int)(gridDim.x / kXcds) + (int)(blockIdx.x / kXcds);
+  if (b * (kPatBlock * R) >= A.n) return;
+  const int r0 = b * (kPatBlock * R) + threadIdx.x;
+  int id[R];
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int r = r0 + u * kPatBlock;
+    id[u] = r < A.n ? A.id[r] : 0;
+  }
+  for (int k = threadIdx.x; k < A.count * A.width; k += kPatBlock) {
+    off[k] = A.off[k];
+    val[k] = A.v[k];
+  }
+  for (int k = threadIdx.x; k < A.count; k += kPatBlock) len[k] = A.len[k];
+  __syncthreads();
+  T g[R][K];
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int r = r0 + u * kPatBlock;
+    const int base = id[u] * A.width;
+    const int rr = r < A.n ? r : A.n - 1;
+#pragma unroll
+    for (int k = 0; k < K; ++k)  // absent entries: the row's own column
+      g[u][k] = x[rr + (k < A.width && r < A.n ? off[base + k] : 0)];
+  }
+  double acc = 0.0;
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int r = r0 + u * kPatBlock;
+    const int base = id[u] * A.width, l = len[id[u]];
+    T s = T(0);
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (k < A.width) {
+        const T t = s + val[base + k] * g[u][k];
+        s = k < l ? t : s;
+      }
+    if (r < A.n) acc += epi.row(r, s);
+  }
+  if constexpr (Epi::kReduce) {
+    const double t = block_sum_to_thread0<kPatBlock>(acc, red);
+    if (threadIdx.x == 0) partials[b] = t;
+  }
+}
+
+inline int pattern_blocks(const spk_csr_s& A) {
+  const int rows = kPatBlock * pattern_rows(A.nrows);
+  return (int)((A.nrows + rows - 1) / rows);
+}
+
+template <typename T, typename Epi>
+void launch_patterns(spk_csr_s& A, const T* x, const Epi& epi, double* parts,
+                     hipStream_t s) {
+  PatView<T> v{A.pat_id.p, A.pat_off.p, A.pat_len.p, nullptr, (int)A.nrows, A.pat_count,
+               A.max_len};
+  if constexpr (std::is_same<T, float>::value) v.v = A.pat_v32.p;
+  else v.v = A.pat_v64.p;
+  const dim3 grid((pattern_blocks(A) + kXcds - 1) / kXcds * kXcds), block(kPatBlock);
+  auto run = [&](auto k, auto r) {
+    hipLaunchKernelGGL((pattern_spmv_kernel<T, decltype(k)::value, decltype(r)::value, Epi>),
+                       grid, block, 0, s, v, x, epi, parts);
+    SPK_HIP_TRY(hipGetLastError());
+  };
+  auto pick = [&](auto k) {
+    if (pattern_rows(A.nrows) == 2) run(k, std::integral_constant<int, 2>{});
+    else run(k, std::integral_constant<int, 4>{});
+  };
+  if (A.max_len <= 5) pick(std::integral_constant<int, 5>{});
+  else if (A.max_len <= 7) pick(std::integral_constant<int, 7>{});
+  else if (A.max_len <= 9) pick(std::integral_constant<int, 9>{});
+  else pick(std::integral_constant<int, kPatMaxLen>{});
+}
+
+// blocks (and partials) of a plain-layout SpMV over a store
+template <typename T>
+int plain_blocks(const spk_csr_s& A) {
+  return A.patterned<T>() ? pattern_blocks(A) : A.nblocks;
+}
+
 // the number of partials a tiled SpMV writes: one per group, then the long
 // rows' blocks
 inline int xtile_partials_count(const spk_csr_s& A) {
@@ -567,11 +712,15 @@ void launch_xtiles(spk_csr_s& A, const T* x, const Epi& epi, double* parts,
   }
 }
 
-// the row kernel over one store: FP32 SpMVs of a store with half32 set
-// read its FP16 values
+// the plain layout over one store: the row patterns where it has them;
+// FP32 SpMVs of a store with half32 set read its FP16 values
 template <typename T, typename Epi>
 void launch_row_kernel(spk_csr_s& A, const T* x, const Epi& epi, double* parts,
                        const T* init, hipStream_t s) {
+  if (A.patterned<T>() && init == nullptr) {
+    launch_patterns(A, x, epi, parts, s);
+    return;
+  }
   if constexpr (std::is_same<T, float>::value) {
     if (A.half32) {
       hipLaunchKernelGGL((spmv_kernel<float, Epi, _Float16>), dim3(A.nblocks),
@@ -588,7 +737,7 @@ void launch_row_kernel(spk_csr_s& A, const T* x, const Epi& epi, double* parts,
 template <typename T, typename Epi>
 void launch_spmv_one(spk_csr_s& A, const T* x, const Epi& epi, const T* init,
                      hipStream_t s) {
-  const int nparts = A.xt_groups ? xtile_partials_count(A) : A.nblocks;
+  const int nparts = A.xt_groups ? xtile_partials_count(A) : plain_blocks<T>(A);
   double* parts = Epi::kReduce ? reduce_partials(nparts) : nullptr;
   if (A.xt_groups) launch_xtiles(A, x, epi, parts, s);
   else launch_row_kernel(A, x, epi, parts, init, s);
@@ -636,13 +785,14 @@ int launch_spmv_partials(spk_csr_s& A, const T* x, const Epi& epi, double* parts
   const T* init = nullptr;
   if (!A.panels.empty()) init = launch_panels(A, x, epi.done, s);
   launch_row_kernel(last, x, epi, parts, init, s);
-  return last.nblocks;
+  return plain_blocks<T>(last);
 }
 
 // the number of partials launch_spmv_partials writes
+template <typename T>
 inline int spmv_partials_count(const spk_csr_s& A) {
   if (A.xt_groups) return xtile_partials_count(A);
-  return A.panels.empty() ? A.nblocks : A.panels.back()->nblocks;
+  return A.panels.empty() ? plain_blocks<T>(A) : A.panels.back()->nblocks;
 }
 
 template <typename T, typename Epi>

@@ -176,9 +176,9 @@ void cg_reliable(spk_csr_s* A, spk_precond_s* M, const spk_ir_config* cfg,
   const bool steps_fit = (jac || ident) && cg_steps_fit<float>(*A);
   const GridLink link = steps_fit ? grid_link() : GridLink{};
   const bool handoff = !steps_fit && (jac || ident || spai) &&
-                       spmv_partials_count(*A) <= kProMaxPartials &&
+                       spmv_partials_count<float>(*A) <= kProMaxPartials &&
                        pro_grid(n) <= kProMaxPartials &&
-                       (!spai || spmv_partials_count(*M->M) <= kProMaxPartials);
+                       (!spai || spmv_partials_count<float>(*M->M) <= kProMaxPartials);
   double* part1 = nullptr;
   double* part2 = nullptr;
   double* part3 = nullptr;

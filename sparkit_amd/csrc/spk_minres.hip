@@ -228,7 +228,7 @@ void minres_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
     // partials <w, u>; the update pass sums those, and every block derives
     // the rotations from the previous step's state (block 0 records the new
     // state in the other parity slot).
-    const bool handoff = diag && spmv_partials_count(*A) <= kProMaxPartials &&
+    const bool handoff = diag && spmv_partials_count<T>(*A) <= kProMaxPartials &&
                          pro_grid(n) <= kProMaxPartials;
     double* pq[2] = {nullptr, nullptr};
     if (handoff) {

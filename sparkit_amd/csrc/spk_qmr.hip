@@ -267,8 +267,8 @@ void qmr_solve(spk_csr_s* A, spk_csr_s* At, spk_precond_s* ML, spk_precond_s* MR
   // next delta).  The smoothing state alternates between two slots by
   // step parity; K6 is gated on K4's step stamp, as its block 0 may end
   // the solve.
-  const bool handoff = diag && spmv_partials_count(*A) <= kProMaxPartials &&
-                       spmv_partials_count(*At) <= kProMaxPartials &&
+  const bool handoff = diag && spmv_partials_count<T>(*A) <= kProMaxPartials &&
+                       spmv_partials_count<T>(*At) <= kProMaxPartials &&
                        pro_grid(n) <= kProMaxPartials;
   double* pq[4] = {nullptr, nullptr, nullptr, nullptr};
   int c_delta = 0;
