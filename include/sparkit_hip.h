@@ -60,6 +60,11 @@ void* spk_get_stream(void);
 spk_status spk_synchronize(void);
 spk_status spk_device_info(int* num_cus, char* name, size_t name_len);
 
+/* Device memory from a pool of at most 2 GiB of freed blocks, given back by
+ * spk_finalize and when an allocation would fail.  Freed memory is handed out
+ * again only after all work on the device queued before the spk_free has
+ * ended, on any stream; spk_free itself does not wait.  spk_free also takes
+ * memory from hipMalloc (and then waits as hipFree does). */
 spk_status spk_malloc(void** dptr, size_t bytes);
 spk_status spk_free(void* dptr);
 spk_status spk_memcpy_htod(void* dst, const void* src, size_t bytes);

@@ -72,6 +72,13 @@ spk_status guarded(F&& body) {
 
 // ------------------------------------------------------------- device
 
+// Device memory from the library's pool (spk_runtime.hip): hipMalloc's and
+// hipFree's contract -- freed memory is handed out again only after all work
+// on the device that was queued before has ended, on whatever stream -- at a
+// fraction of their time.  pool_malloc returns hipMalloc's error.
+hipError_t pool_malloc(void** p, size_t bytes);
+void pool_free(void* p);
+
 // Device memory owned by the library (RAII, move-only).
 template <typename T>
 struct DevBuf {
@@ -90,7 +97,7 @@ struct DevBuf {
   void alloc(size_t count) {
     release();
     if (count == 0) count = 1;
-    hipError_t e = hipMalloc(&p, count * sizeof(T));
+    hipError_t e = pool_malloc((void**)&p, count * sizeof(T));
     if (e != hipSuccess) {
       p = nullptr;
       throw Error{SPK_OUT_OF_MEMORY, "hipMalloc of " +
@@ -100,7 +107,7 @@ struct DevBuf {
   }
   // grow-only reallocation (contents are not preserved)
   void reserve(size_t count) { if (count > n || p == nullptr) alloc(count); }
-  void release() { if (p) (void)hipFree(p); p = nullptr; n = 0; }
+  void release() { if (p) pool_free(p); p = nullptr; n = 0; }
   T* get() const { return p; }
 };
 

@@ -3,8 +3,10 @@
 #include "spk_link.hpp"
 
 #include <cstring>
+#include <map>
 #include <memory>
 #include <mutex>
+#include <unordered_map>
 
 namespace spk {
 
@@ -65,6 +67,129 @@ GridLink make_link(unsigned long long* w) {
   return GridLink{w, (unsigned*)(w + kLinkSlotWords), (int*)(w + kLinkSlotWords + 1)};
 }
 
+// ---- the device memory pool
+//
+// A block freed waits in `idle` of its size until something of that size is
+// wanted and no block is `ready`; then the device is waited for once, and
+// every block that was idle by then is ready.  So a block's next owner starts
+// after all work queued before the free, on any stream of any thread, as with
+// hipFree (which waits too, each time).  Small sizes keep several blocks, so
+// that a loop that makes and drops a vector waits once in many rounds.
+// Measured on y = multiply(A, x), 4,096 rows: hipMalloc and hipFree took 13
+// of the call's 16.5 us.
+class Pool {
+ public:
+  hipError_t get(void** p, size_t bytes) {
+    const size_t size = rounded(bytes);
+    std::lock_guard<std::mutex> lk(m_);
+    if (!open()) return hipMalloc(p, bytes);
+    Size& c = sizes_[size];
+    if (c.ready.empty() && c.idle.size() >= idle_limit(size)) {
+      if (hipDeviceSynchronize() == hipSuccess) {
+        for (auto& s : sizes_) {
+          s.second.ready.insert(s.second.ready.end(), s.second.idle.begin(),
+                                s.second.idle.end());
+          s.second.idle.clear();
+        }
+      } else {
+        (void)hipGetLastError();
+      }
+    }
+    if (!c.ready.empty()) {
+      *p = c.ready.back();
+      c.ready.pop_back();
+      kept_ -= size;
+      --blocks_;
+      own(*p, size);
+      return hipSuccess;
+    }
+    hipError_t e = hipMalloc(p, size);
+    if (e != hipSuccess && kept_ > 0) {
+      (void)hipGetLastError();
+      give_back();
+      e = hipMalloc(p, size);
+    }
+    if (e == hipSuccess) own(*p, size);
+    return e;
+  }
+  // false: not a block of this pool
+  bool put(void* p) {
+    std::lock_guard<std::mutex> lk(m_);
+    auto it = owned_.find(p);
+    if (it == owned_.end()) return false;
+    const size_t size = it->second;
+    owned_.erase(it);
+    if (!open()) return false;
+    if (size > kLargest || kept_ + size > kMost || blocks_ >= kMostBlocks) {
+      (void)hipFree(p);
+      return true;
+    }
+    sizes_[size].idle.push_back(p);
+    kept_ += size;
+    ++blocks_;
+    return true;
+  }
+  void drain() {
+    std::lock_guard<std::mutex> lk(m_);
+    give_back();
+  }
+
+ private:
+  struct Size {
+    std::vector<void*> ready, idle;
+  };
+  static constexpr size_t kMost = size_t(2) << 30;      // bytes kept, at most
+  static constexpr size_t kLargest = size_t(256) << 20;  // a kept block's size
+  static constexpr size_t kMostBlocks = 512;
+  // sizes an eighth of a power of two apart, few enough to meet again; what
+  // is never kept is not rounded
+  static size_t rounded(size_t bytes) {
+    if (bytes > kLargest) return bytes;
+    size_t step = 512;
+    while (bytes > 8 * step) step *= 2;
+    return bytes == 0 ? step : (bytes + step - 1) / step * step;
+  }
+  static size_t idle_limit(size_t size) {
+    return size <= (64 << 10) ? 16 : size <= (1 << 20) ? 4 : 1;
+  }
+  // The pool keeps out of captures, of other devices and of the time after
+  // spk_finalize: hipMalloc and hipFree then decide, as without a pool.
+  static bool open() {
+    int dev = -1;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (g_ctx.device < 0) return false;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipStreamIsCapturing(g_user_stream ? g_user_stream : g_ctx.stream, &st) !=
+            hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    return dev == g_ctx.device && st == hipStreamCaptureStatusNone;
+  }
+  void own(void* p, size_t size) {
+    try {
+      owned_[p] = size;
+    } catch (const std::bad_alloc&) {  // then it goes back by hipFree
+    }
+  }
+  void give_back() {  // hipFree waits for the device itself
+    for (auto& s : sizes_) {
+      for (void* p : s.second.ready) (void)hipFree(p);
+      for (void* p : s.second.idle) (void)hipFree(p);
+    }
+    sizes_.clear();
+    kept_ = blocks_ = 0;
+  }
+  std::mutex m_;
+  std::map<size_t, Size> sizes_;
+  std::unordered_map<void*, size_t> owned_;
+  size_t kept_ = 0, blocks_ = 0;
+};
+Pool& pool() {
+  static Pool* p = new Pool();  // outlives the objects that free into it
+  return *p;
+}
+
 void init_device(int device) {
   int count = 0;
   if (hipGetDeviceCount(&count) != hipSuccess || count == 0)
@@ -91,6 +216,16 @@ void init_device(int device) {
 }  // namespace
 
 void set_error(const std::string& msg) { g_last_error = msg; }
+
+hipError_t pool_malloc(void** p, size_t bytes) { return pool().get(p, bytes); }
+void pool_free(void* p) {
+  bool kept = false;
+  try {
+    kept = pool().put(p);
+  } catch (const std::bad_alloc&) {  // called by destructors
+  }
+  if (!kept) (void)hipFree(p);
+}
 
 Context& ctx() {
   if (g_ctx.device < 0) {
@@ -217,6 +352,7 @@ spk_status spk_finalize(void) {
     g_partials = nullptr;
     delete g_link;
     g_link = nullptr;
+    pool().drain();
     (void)hipEventDestroy(g_ev0);
     (void)hipEventDestroy(g_ev1);
     (void)hipStreamDestroy(g_ctx.stream);
@@ -257,7 +393,7 @@ spk_status spk_malloc(void** dptr, size_t bytes) {
   return guarded([&] {
     ctx();
     SPK_REQUIRE(dptr, SPK_INVALID_ARGUMENT, "null output pointer");
-    hipError_t e = hipMalloc(dptr, bytes ? bytes : 1);
+    hipError_t e = pool_malloc(dptr, bytes ? bytes : 1);
     if (e != hipSuccess)
       throw Error{SPK_OUT_OF_MEMORY, "hipMalloc failed: " +
                   std::string(hipGetErrorString(e))};
@@ -267,6 +403,7 @@ spk_status spk_malloc(void** dptr, size_t bytes) {
 spk_status spk_free(void* dptr) {
   return guarded([&] {
     ctx();
+    if (!dptr || pool().put(dptr)) return;
     SPK_HIP_TRY(hipStreamSynchronize(stream()));
     SPK_HIP_TRY(hipFree(dptr));
   });

@@ -1,0 +1,98 @@
+"""Device memory from the pool: sizes around its classes and beyond what it
+keeps, blocks that come back, threads, and a block freed while work on it is
+still queued."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def spk():
+    import sparkit_amd
+    sparkit_amd.init(0)
+    return sparkit_amd
+
+
+@pytest.mark.parametrize("n", [0, 1, 511, 512, 513, 4096, 4097, 8191, 8193, 131072, 131073,
+                               1 << 20, (1 << 20) + 1, (1 << 25) + 3])
+def test_sizes(spk, n):
+    print("pool", n, flush=True)
+    rng = np.random.default_rng(n)
+    keep = [rng.integers(0, 1 << 30, n).astype(np.float64) for _ in range(2)]
+    for _ in range(3):
+        a, b = (spk.DeviceVector.from_numpy(k) for k in keep)
+        assert a.n == 0 or a.ptr.value != b.ptr.value
+        assert np.array_equal(a.numpy(), keep[0]) and np.array_equal(b.numpy(), keep[1])
+        del a, b
+
+
+def test_freed_while_in_use(spk):
+    """multiply's result is dropped and made again while the products are
+    queued: each kept one holds its own product."""
+    A = spk.poisson_2d(300)
+    xs = [spk.uniform_pm1(k, A.nrows) for k in range(40)]
+    ref = []
+    for x in xs:
+        y = spk.multiply(A, x)
+        spk.synchronize()
+        ref.append(y.numpy())
+    kept = []
+    for k, x in enumerate(xs):
+        for _ in range(5):
+            y = spk.multiply(A, xs[(k * 7) % 40])  # dropped at once
+        kept.append(spk.multiply(A, x))
+    for y, r in zip(kept, ref):
+        assert np.array_equal(y.numpy(), r)
+
+
+def test_threads(spk):
+    """Allocation and release from several threads (the calls that queue work
+    take turns, as the library asks)."""
+    lock, bad = threading.Lock(), []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        for _ in range(60):
+            h = rng.uniform(-1, 1, int(rng.integers(1, 40000)))
+            with lock:
+                v = spk.DeviceVector.from_numpy(h)
+                w = spk.DeviceVector(v.n)
+                w.copy_from(v)
+            with lock:
+                if not np.array_equal(w.numpy(), h):
+                    bad.append(seed)
+            del v, w  # outside the lock
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
+
+
+def test_finalize_gives_the_pool_back():
+    """Vectors that outlive spk_finalize, and a library started again."""
+    import subprocess
+    import sys
+    code = """
+import numpy as np, sparkit_amd as spk
+spk.init(0)
+for k in range(40):
+    v = spk.DeviceVector.from_numpy(np.arange(5000.0))
+late = spk.DeviceVector(77)
+from sparkit_amd import _lib
+_lib.call("spk_finalize")
+spk.init(0)
+w = spk.DeviceVector.from_numpy(np.arange(5000.0))
+del late
+for k in range(40):
+    v = spk.DeviceVector.from_numpy(np.arange(77.0) + k)
+assert np.array_equal(w.numpy(), np.arange(5000.0))
+print("ok")
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.stdout.strip().endswith("ok"), r.stderr
