@@ -18,20 +18,38 @@
 // fp32.  M_i,slot = (delta_{slot,4} + y_slot) / a_ii: zero output weights
 // give the Jacobi preconditioner.
 //
-// Kernel layout.  One workgroup = 4 wavefronts; each wavefront owns a tile
-// of 64 rows at a time (lane = row for the per-row work) and a 32 KB LDS
-// region for the tile's operands; the bf16 weights sit in LDS once per
-// workgroup.  Every GEMM is a sequence of v_mfma_f32_16x16x32_bf16 on 16x16
-// output tiles whose A/B fragments are read from LDS:
-//   forward   H1 = relu(X W1 + b1), H2 = relu(H1 W2 + b2), Y = H2 W3 + b3
-//   per row   m from Y, (M A)_i by a merge of the slot rows, dL/dy
-//   backward  dW3 += H2^T dY; dH2 = dY W3^T * [H2 > 0]; dW2 += H1^T dH2;
+// Kernel layout.  The matrices of a batch go through each pass together, up
+// to kGroupMats matrices or kGroupRows rows at a time (a larger matrix goes
+// alone):
+//   prepare   a row per thread: diagonal and row sum
+//   features  a row per thread: the row's 24 features in bfloat16
+//   forward   a wavefront per 64 rows: Y = H2 W3 + b3, H2 = relu(H1 W2 + b2),
+//             H1 = relu(X W1 + b1)
+//   rows      a row per thread: m from Y, (M A)_i by a merge of the slot
+//             rows, the row's loss and dL/dy
+//   backward  one workgroup of 4 wavefronts a compute unit, 64 rows per
+//             wavefront at a time: H1 and H2 again, then dW3 += H2^T dY;
+//             dH2 = dY W3^T * [H2 > 0]; dW2 += H1^T dH2;
 //             dH1 = dH2 W2^T * [H1 > 0]; dW1 += X^T dH1
-// Weight gradients stay in the MFMA accumulators across a wavefront's
-// tiles, are summed over the workgroup's wavefronts in LDS in a fixed order
-// and written as one partial per workgroup; the update kernel sums the
-// partials in workgroup order (deterministic) and applies Adam to the fp32
-// master weights, then refreshes the bf16 copy.
+// The per-row passes wait for dependent loads and run at the occupancy their
+// registers allow; only the two passes of products need LDS.  Every product
+// is a sequence of v_mfma_f32_16x16x32_bf16 on 16x16 output tiles.  The
+// weights' fragments stay in registers; an activation or delta is kept in
+// LDS by rows where its columns are summed over and by columns where its
+// rows are, so that every fragment is one 16-byte read (rows of 72 elements:
+// no bank conflicts).  Weight gradients stay in the MFMA accumulators across
+// a wavefront's tiles of a matrix, are summed over the workgroup's
+// wavefronts in LDS in a fixed order and added to one partial per workgroup;
+// the update kernel sums the partials in workgroup order (deterministic) and
+// applies Adam to the fp32 master weights, then refreshes the bf16 copy.
+//
+// Measured on a batch of 4 matrices of 65,536 9-point rows: prepare 20 us,
+// features 13, forward 14, rows 57 (issue bound: about 25 columns a row, nine
+// lists compared for each), backward 57 (one wavefront per SIMD, bound by
+// what its LDS holds; 14 us a matrix, 5 of them the workgroup's sums), update
+// 8.  One fused kernel for all of it, a matrix at a time, took 105 us a
+// matrix and the update 74 us: its per-row parts ran at one wavefront per
+// SIMD, and its fragments were read from LDS two bytes at a time.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -46,6 +64,7 @@ namespace spk {
 namespace {
 
 typedef __bf16 bf16;
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
@@ -64,111 +83,217 @@ constexpr int gW1 = 0, gW2 = gW1 + kFp * kH, gW3 = gW2 + kH * kH,
               kGradLen = gB3 + kOn;
 constexpr int kTile = 64;   // rows per wavefront tile
 constexpr int kWaves = 4;   // wavefronts per workgroup
-// per-wavefront LDS region, in bf16 elements
-constexpr int oX = 0, oH1 = oX + kTile * kFp, oH2 = oH1 + kTile * kH,
-              oYD = oH2 + kTile * kH, oD = oYD + kTile * kOk,
-              kPool = oD + kTile * kH;
+// LDS row length, in bf16 elements, of 64-wide operands and of dY by rows
+constexpr int kLd = 72, kLdY = 24;
+// what a training launch takes together, at most (or one larger matrix)
+constexpr int kGroupMats = 16;
+constexpr int64_t kGroupRows = 1 << 20;
+constexpr int kRowBlock = 256;
 
-struct Packed {  // what the tile kernel reads: bf16 weights, fp32 biases
-  bf16 w1[kFp * kH];
+// bf16 weights, those a product reads by columns in a transposed copy, and
+// fp32 biases
+struct Packed {
+  bf16 w1t[kH * kFp];  // [hidden][feature]
   bf16 w2[kH * kH];
+  bf16 w2t[kH * kH];
   bf16 w3[kH * kOk];
+  bf16 w3t[kOn * kH];
   float b1[kH], b2[kH], b3[kOn];
 };
 
-__host__ __device__ inline uint16_t bf16_bits(float x) {
-  uint32_t u = __builtin_bit_cast(uint32_t, x);
-  if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (uint16_t)(u >> 16);  // NaN
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-__device__ __forceinline__ bf16 to_bf16(float x) {
-  return __builtin_bit_cast(bf16, bf16_bits(x));
-}
-__device__ __forceinline__ float from_bf16(bf16 h) {
-  return __builtin_bit_cast(float, (uint32_t)__builtin_bit_cast(uint16_t, h)
-                                       << 16);
+// round to nearest even: v_cvt_pk_bf16_f32
+__device__ __forceinline__ bf16 to_bf16(float x) { return (bf16)x; }
+// of a value that relu gave (not negative, but -0 may be)
+__device__ __forceinline__ bool positive(bf16 h) {
+  return (__builtin_bit_cast(uint16_t, h) & 0x7FFF) != 0;
 }
 
-// acc += A[16 x 32] B[32 x 16]; A(r, k) = a[r*ars + k*aks],
-// B(k, c) = b[k*bks + c*bcs].  Lane l supplies row/column l % 16 and the
-// eight k of group l / 16; acc[i] is C(4 (l / 16) + i, l % 16).
-__device__ __forceinline__ floatx4 mma(const bf16* a, int ars, int aks,
-                                       const bf16* b, int bks, int bcs,
-                                       floatx4 acc) {
-  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-  bf16x8 av, bv;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    av[j] = a[r * ars + (8 * g + j) * aks];
-    bv[j] = b[(8 * g + j) * bks + r * bcs];
-  }
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc, 0, 0, 0);
+// C += A[16 x 32] B[32 x 16].  Lane l's fragment is row (of A) or column (of
+// B) l % 16, the eight k from 8 (l / 16) on; acc[i] is C(4 (l / 16) + i, l % 16).
+__device__ __forceinline__ floatx4 mma(bf16x8 a, bf16x8 b, floatx4 acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+}
+__device__ __forceinline__ bf16x8 frag(const bf16* p) {  // 16-byte aligned
+  return *(const bf16x8*)p;
+}
+// LDS traffic between the lanes of a wavefront, which is in order
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 __device__ __forceinline__ floatx4 splat(float v) { return floatx4{v, v, v, v}; }
 
-// per-matrix pass: diagonal, row sums, slot-rule check
-__global__ void spai_prepare_kernel(int64_t n, const int32_t* __restrict__ rp,
-                                    const int32_t* __restrict__ ci,
-                                    const double* __restrict__ v,
-                                    double* __restrict__ diag,
-                                    double* __restrict__ rsum, int* err) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int p0 = rp[i], p1 = rp[i + 1];
-  int dpos = -1;
-  double s = 0.0;
-  for (int p = p0; p < p1; ++p) {
-    if (ci[p] == i) dpos = p;
-    s += v[p];
-  }
-  const bool bad = dpos < 0 || !(v[dpos] > 0.0) || dpos - p0 > 4 ||
-                   p1 - dpos - 1 > 4;
-  if (bad) atomicOr(err, 1);
-  diag[i] = bad ? 1.0 : v[dpos];
-  rsum[i] = s;
-}
-
-struct TileArgs {
-  int64_t n;
+// Rows [first, last) of a matrix of n rows: row i's diagonal and row sum are
+// at dbase + i, its features and outputs at xbase + i - first.  xbase is a
+// multiple of kRowBlock.
+struct RowSpan {
   const int32_t* __restrict__ rp;
   const int32_t* __restrict__ ci;
   const double* __restrict__ v;
-  const double* __restrict__ diag;
-  const double* __restrict__ rsum;
+  int64_t n, first, last, dbase, xbase;
+};
+
+struct Group {
+  RowSpan mat[kGroupMats];
+  int count;
+  double* __restrict__ diag;
+  double* __restrict__ rsum;
+  bf16* __restrict__ x;            // [rows][kFp]
+  float* __restrict__ y;           // [rows][kO]: outputs, then dL/dy
+  // train: the matrices' entries by scratch row, see EntryRows
+  int32_t* __restrict__ ecol;
+  double* __restrict__ eval;
+  double* __restrict__ rowloss;    // [rows]
   const Packed* __restrict__ pk;
-  double* __restrict__ mvals;    // predict: M values on A's pattern
-  float* __restrict__ partials;  // train: [gridDim.x][kGradLen]
-  double* __restrict__ loss_part;  // train: [gridDim.x]
-  double scale;                  // train: 1 / rows of the batch
-  int accumulate;                // train: add to the existing partials
-  // train, symmetric objective: dL/dm per entry of A's pattern and each
-  // row's loss, computed beforehand (null: the row merge below)
+  double* __restrict__ mvals;      // predict: M values on A's pattern
+  double scale;                    // train: 1 / rows of the batch
+  // train, symmetric objective (one matrix): dL/dm per entry of A's pattern
+  // and each row's loss, computed beforehand
   const double* __restrict__ gm;
-  const double* __restrict__ rowloss;
+  const double* __restrict__ rl;
+};
+
+// the span that scratch row x (of a whole workgroup) lies in
+__device__ __forceinline__ int span_of(const Group& G, int64_t x) {
+  int k = 0;
+  while (k + 1 < G.count && x >= G.mat[k + 1].xbase) ++k;
+  return k;
+}
+
+// A row's entries, kEntries places 64 rows at a time: place k of scratch row x
+// at entry_at(x) + 64 k, the columns ascending and INT32_MAX behind them, so
+// that lanes on neighbouring rows read neighbouring words (from the CSR rows
+// the merge of the slot rows took three times as long: a lane's rows lie 36
+// and 72 bytes from the next lane's).
+constexpr int kEntries = kO + 1;
+__device__ __forceinline__ int64_t entry_at(int64_t x) {
+  return (x >> 6) * (64 * kEntries) + (x & 63);
+}
+
+// diagonal, row sums; with err the slot-rule check; the entries if G has
+// room for them
+__global__ void spai_prepare_kernel(Group G, int* err) {
+  const int64_t x = blockIdx.x * (int64_t)blockDim.x;
+  const RowSpan& A = G.mat[span_of(G, x)];
+  const int64_t i = x + threadIdx.x - A.xbase;
+  if (i >= A.n) return;
+  const int p0 = A.rp[i], p1 = A.rp[i + 1];
+  int dpos = -1;
+  double s = 0.0;
+  for (int p = p0; p < p1; ++p) {
+    if (A.ci[p] == i) dpos = p;
+    s += A.v[p];
+  }
+  const bool bad = dpos < 0 || !(A.v[dpos] > 0.0) || dpos - p0 > 4 ||
+                   p1 - dpos - 1 > 4;
+  if (bad && err) atomicOr(err, 1);
+  G.diag[A.dbase + i] = bad ? 1.0 : A.v[dpos];
+  G.rsum[A.dbase + i] = s;
+  if (!G.ecol) return;
+  const int64_t o = entry_at(A.xbase + i);
+  int c[kO];
+  double v[kO];
+#pragma unroll
+  for (int k = 0; k < kO; ++k) {
+    const bool in = p0 + k < p1;
+    c[k] = in ? A.ci[p0 + k] : INT32_MAX;
+    v[k] = in ? A.v[p0 + k] : 0.0;
+  }
+#pragma unroll
+  for (int k = 0; k < kO; ++k) {
+    G.ecol[o + 64 * k] = c[k];
+    G.eval[o + 64 * k] = v[k];
+  }
+  G.ecol[o + 64 * kO] = INT32_MAX;
+  G.eval[o + 64 * kO] = 0.0;
+}
+
+// Two forms of a matrix's rows.  slots(): the places of row i's slots (and
+// their columns, INT32_MAX for none), pos[4] its diagonal, pos[3..0] the entries left of it from the nearest outwards,
+// pos[5..8] those right of it (-1 unused).  cursor(j): where row j's first
+// entry is (col() and val() there, INT32_MAX behind the last; none(i): behind
+// the last), step() to the next.
+struct CsrRows {
+  const int32_t* __restrict__ rp;
+  const int32_t* __restrict__ ci;
+  const double* __restrict__ v;
+  struct Cursor {
+    int p, e;
+  };
+  __device__ __forceinline__ void slots(int64_t i, int* pos, int* j) const {
+    const int p0 = rp[i], p1 = rp[i + 1];
+    int d = p0;
+    while (ci[d] != (int32_t)i) ++d;  // present: checked by the prepare pass
+    pos[4] = d;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      pos[3 - k] = (d - 1 - k >= p0) ? d - 1 - k : -1;
+      pos[5 + k] = (d + 1 + k < p1) ? d + 1 + k : -1;
+    }
+#pragma unroll
+    for (int s = 0; s < kO; ++s) j[s] = pos[s] >= 0 ? ci[pos[s]] : INT32_MAX;
+  }
+  __device__ __forceinline__ double val_at(int64_t, int p) const { return v[p]; }
+  __device__ __forceinline__ Cursor cursor(int64_t j) const {
+    return Cursor{rp[j], rp[j + 1]};
+  }
+  __device__ __forceinline__ Cursor none(int64_t) const { return Cursor{0, 0}; }
+  __device__ __forceinline__ void step(Cursor& c) const { ++c.p; }
+  __device__ __forceinline__ int col(const Cursor& c) const {
+    return c.p < c.e ? ci[c.p] : INT32_MAX;
+  }
+  __device__ __forceinline__ double val(const Cursor& c) const {
+    return c.p < c.e ? v[c.p] : 0.0;
+  }
+};
+struct EntryRows {
+  const int32_t* __restrict__ c;
+  const double* __restrict__ v;
+  int64_t base;  // scratch row of row 0
+  using Cursor = int64_t;
+  __device__ __forceinline__ void slots(int64_t i, int* pos, int* j) const {
+    const int32_t* row = c + entry_at(base + i);
+    int d = 0, own[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) own[k] = row[64 * k];
+#pragma unroll
+    for (int k = 1; k < 5; ++k) d = own[k] == (int32_t)i ? k : d;
+#pragma unroll
+    for (int s = 0; s < kO; ++s) {
+      const int k = s - 4 + d;  // at most 8
+      j[s] = row[64 * (k < 0 ? kO : k)];
+      pos[s] = j[s] != INT32_MAX ? k : -1;
+    }
+  }
+  __device__ __forceinline__ double val_at(int64_t i, int p) const {
+    return v[entry_at(base + i) + 64 * p];
+  }
+  __device__ __forceinline__ Cursor cursor(int64_t j) const { return entry_at(base + j); }
+  __device__ __forceinline__ Cursor none(int64_t i) const {
+    return entry_at(base + i) + 64 * kO;  // the word behind row i
+  }
+  __device__ __forceinline__ void step(Cursor& q) const { q += 64; }
+  __device__ __forceinline__ int col(const Cursor& q) const { return c[q]; }
+  __device__ __forceinline__ double val(const Cursor& q) const { return v[q]; }
 };
 
 // Row i's residual e_i - sum_s m_s A_{j_s,:} by a merge of the slot rows
 // (their columns ascend): returns ||.||^2 and adds dL/dm_s to gs[s].
-__device__ __forceinline__ double row_residual(const int32_t* __restrict__ rp,
-                                               const int32_t* __restrict__ ci,
-                                               const double* __restrict__ v,
-                                               int64_t i, const int* pos,
+template <typename Rows>
+__device__ __forceinline__ double row_residual(const Rows& A, int64_t i, const int* j,
                                                const double* m, double* gs) {
 #pragma clang fp contract(off)
-  int hp[kO], he[kO], hc[kO];
+  typename Rows::Cursor hp[kO];
+  int hc[kO];
   double hv[kO];
 #pragma unroll
+  for (int s = 0; s < kO; ++s)
+    hp[s] = j[s] != INT32_MAX ? A.cursor(j[s]) : A.none(i);
+#pragma unroll
   for (int s = 0; s < kO; ++s) {
-    hp[s] = he[s] = 0;
-    if (pos[s] >= 0) {
-      const int j = ci[pos[s]];
-      hp[s] = rp[j];
-      he[s] = rp[j + 1];
-    }
-    hc[s] = hp[s] < he[s] ? ci[hp[s]] : INT32_MAX;
-    hv[s] = hp[s] < he[s] ? v[hp[s]] : 0.0;
+    hc[s] = A.col(hp[s]);
+    hv[s] = A.val(hp[s]);
   }
   double lrow = 0.0;
   for (;;) {
@@ -186,56 +311,234 @@ __device__ __forceinline__ double row_residual(const int32_t* __restrict__ rp,
     for (int s = 0; s < kO; ++s)
       if (hc[s] == c) {
         gs[s] += -2.0 * res * hv[s];
-        ++hp[s];
-        hc[s] = hp[s] < he[s] ? ci[hp[s]] : INT32_MAX;
-        hv[s] = hp[s] < he[s] ? v[hp[s]] : 0.0;
+        // hv is read before its load goes out: the load then writes its
+        // register, and the wait for it comes once, before the next column
+        __builtin_amdgcn_sched_barrier(0);
+        A.step(hp[s]);
+        hc[s] = A.col(hp[s]);
+        hv[s] = A.val(hp[s]);
       }
   }
   return lrow;
 }
 
-// Row i's slot positions: pos[4] its diagonal, pos[3..0] the entries left
-// of it from the nearest outwards, pos[5..8] those right of it (-1 unused).
-__device__ __forceinline__ void row_slots(const int32_t* __restrict__ rp,
-                                          const int32_t* __restrict__ ci, int64_t i,
-                                          int* pos) {
-  const int p0 = rp[i], p1 = rp[i + 1];
-  int d = p0;
-  while (ci[d] != (int32_t)i) ++d;  // present: checked by the prepare pass
-  pos[4] = d;
+// row i's features
+template <typename Rows>
+__device__ __forceinline__ void row_features(const Rows& A,
+                                             const double* __restrict__ diag,
+                                             const double* __restrict__ rsum,
+                                             int64_t i, float* x) {
+#pragma clang fp contract(off)
+  int pos[kO], js[kO];
+  A.slots(i, pos, js);
+  const double di = diag[i];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    pos[3 - k] = (d - 1 - k >= p0) ? d - 1 - k : -1;
-    pos[5 + k] = (d + 1 + k < p1) ? d + 1 + k : -1;
+  for (int k = 0; k < 8; ++k) {
+    const int p = pos[k < 4 ? k : k + 1], j = js[k < 4 ? k : k + 1];
+    x[k] = x[8 + k] = x[16 + k] = 0.f;
+    if (p >= 0) {
+      const double dj = diag[j];
+      x[k] = (float)(A.val_at(i, p) / di);
+      x[8 + k] = (float)((dj - di) / (dj + di));
+      x[16 + k] = (float)(rsum[j] / dj);
+    }
   }
 }
 
-template <bool TRAIN>
-__global__ __launch_bounds__(256) void spai_tile_kernel(TileArgs A) {
+// Features of every scratch row (zero past a span's end).
+__global__ __launch_bounds__(kRowBlock) void spai_features_kernel(Group G) {
+  const int64_t xb = blockIdx.x * (int64_t)kRowBlock;
+  const RowSpan& A = G.mat[span_of(G, xb)];
+  const int64_t xr = xb + threadIdx.x, i = xr - A.xbase + A.first;
+  float x[kFp];
+#pragma unroll
+  for (int f = 0; f < kFp; ++f) x[f] = 0.f;
+  const double* diag = G.diag + A.dbase;
+  const double* rsum = G.rsum + A.dbase;
+  if (i < A.last) {
+    if (G.ecol) row_features(EntryRows{G.ecol, G.eval, A.xbase}, diag, rsum, i, x);
+    else row_features(CsrRows{A.rp, A.ci, A.v}, diag, rsum, i, x);
+  }
+  bf16x8* out = (bf16x8*)(G.x + xr * kFp);
+#pragma unroll
+  for (int q = 0; q < kFp / 8; ++q) {
+    bf16x8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = to_bf16(x[8 * q + j]);
+    out[q] = o;
+  }
+}
+
+// Y of every scratch row, a tile per wavefront.
+__global__ __launch_bounds__(kWaves * 64) void spai_forward_kernel(Group G) {
 #pragma clang fp contract(off)
-  __shared__ Packed sw;
-  __shared__ __attribute__((aligned(16))) bf16 pool[kWaves * kPool];
-  __shared__ float b3tmp[kTile * kO];
+  __shared__ __attribute__((aligned(16))) bf16 pool[kWaves * kTile * kLd];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
-  {  // weights into LDS
-    const uint32_t* src = (const uint32_t*)A.pk;
-    uint32_t* dst = (uint32_t*)&sw;
-    for (int k = threadIdx.x; k < (int)(sizeof(Packed) / 4); k += blockDim.x)
-      dst[k] = src[k];
+  const Packed& w = *G.pk;
+  bf16* H = pool + wave * kTile * kLd;  // H1, then H2, by rows
+  const int64_t row = (blockIdx.x * (int64_t)kWaves + wave) * kTile;
+  bf16x8 xf[4], wf[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    xf[q] = frag(G.x + (row + q * 16 + r) * kFp + 8 * g);
+    wf[q] = frag(w.w1t + (q * 16 + r) * kFp + 8 * g);
   }
-  __syncthreads();
-  bf16* X = pool + wave * kPool + oX;
-  bf16* H1 = pool + wave * kPool + oH1;
-  bf16* H2 = pool + wave * kPool + oH2;
-  bf16* dY = pool + wave * kPool + oYD;
-  float* Y = (float*)dY;  // Y[64][16] fp32 shares the bytes of dY[64][32]
-  bf16* D = pool + wave * kPool + oD;
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+      const floatx4 acc = mma(xf[mt], wf[nt], splat(w.b1[nt * 16 + r]));
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        H[(mt * 16 + 4 * g + e) * kLd + nt * 16 + r] = to_bf16(fmaxf(acc[e], 0.f));
+    }
+  wave_sync();
+  bf16x8 hf[4][2], w2[4][2];
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      hf[q][kb] = frag(H + (q * 16 + r) * kLd + kb * 32 + 8 * g);
+      w2[q][kb] = frag(w.w2t + (q * 16 + r) * kH + kb * 32 + 8 * g);
+    }
+  wave_sync();
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+      floatx4 acc = splat(w.b2[nt * 16 + r]);
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) acc = mma(hf[mt][kb], w2[nt][kb], acc);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        H[(mt * 16 + 4 * g + e) * kLd + nt * 16 + r] = to_bf16(fmaxf(acc[e], 0.f));
+    }
+  wave_sync();
+  bf16x8 w3[2];
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb) w3[kb] = frag(w.w3t + r * kH + kb * 32 + 8 * g);
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+    floatx4 acc = splat(w.b3[r]);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+      acc = mma(frag(H + (mt * 16 + r) * kLd + kb * 32 + 8 * g), w3[kb], acc);
+    if (r < kO) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) G.y[(row + mt * 16 + 4 * g + e) * kO + r] = acc[e];
+    }
+  }
+}
 
-  floatx4 aW1[2][4], aW2[4][4], aW3[4];
-  float ab1[4], ab2[4], ab3[kO];
-  double lsum = 0.0;
-  if (TRAIN) {
+enum { kPredict, kMerge, kGiven };  // what the row pass does
+
+// Per row: M's values from Y (kPredict); or the row's loss and dL/dy, in Y's
+// place, from the merge of the slot rows (kMerge) or from G.gm and G.rl.
+template <int MODE>
+__global__ __launch_bounds__(kRowBlock) void spai_rows_kernel(Group G) {
+#pragma clang fp contract(off)
+  const int64_t xb = blockIdx.x * (int64_t)kRowBlock;
+  const RowSpan& A = G.mat[span_of(G, xb)];
+  const int64_t xr = xb + threadIdx.x, i = xr - A.xbase + A.first;
+  float* y = G.y + xr * kO;
+  if (i >= A.last) {
+    if (MODE != kPredict) {
+#pragma unroll
+      for (int s = 0; s < kO; ++s) y[s] = 0.f;
+      G.rowloss[xr] = 0.0;
+    }
+    return;
+  }
+  const CsrRows C{A.rp, A.ci, A.v};
+  const EntryRows E{G.ecol, G.eval, A.xbase};
+  int pos[kO], js[kO];
+  if (MODE == kMerge) E.slots(i, pos, js);
+  else C.slots(i, pos, js);
+  const double di = G.diag[A.dbase + i];
+  double m[kO], gs[kO];
+  float out[kO];
+#pragma unroll
+  for (int s = 0; s < kO; ++s) out[s] = MODE == kGiven ? 0.f : y[s];
+#pragma unroll
+  for (int s = 0; s < kO; ++s) {
+    gs[s] = 0.0;
+    m[s] = MODE == kGiven || pos[s] < 0
+               ? 0.0
+               : ((s == 4 ? 1.0 : 0.0) + (double)out[s]) / di;
+  }
+  if (MODE == kPredict) {
+#pragma unroll
+    for (int s = 0; s < kO; ++s)
+      if (pos[s] >= 0) G.mvals[pos[s]] = m[s];
+    return;
+  }
+  if (MODE == kGiven) {
+#pragma unroll
+    for (int s = 0; s < kO; ++s) gs[s] = pos[s] >= 0 ? G.gm[pos[s]] : 0.0;
+    G.rowloss[xr] = G.rl[i];
+  } else {
+    G.rowloss[xr] = row_residual(E, i, js, m, gs);
+  }
+#pragma unroll
+  for (int s = 0; s < kO; ++s)
+    y[s] = (float)(G.scale * gs[s] / di);  // 0 for a slot without an entry
+}
+
+// The backward pass's LDS, in bf16 elements per wavefront.  R1: H1, then dH2,
+// by rows; C1: H1, then dH1, by columns; C2: H2, then dH2, by columns.
+constexpr int oR1 = 0, oC1 = oR1 + kTile * kLd, oC2 = oC1 + kH * kLd,
+              oX = oC2 + kH * kLd, oYr = oX + kFp * kLd, oYc = oYr + kTile * kLdY,
+              kPool = oYc + kOn * kLd;
+// its use for the workgroup's sums: the matrices' gradients of each
+// wavefront, the bias gradients of each lane group, dL/dy and loss per lane
+constexpr int kMats = gB1;  // floats of the three matrices
+constexpr int fB = kWaves * kMats, fB3 = fB + kWaves * 4 * 2 * kH,
+              fLoss = fB3 + kWaves * kTile * kO;
+static_assert(fLoss % 2 == 0 && (size_t)fLoss * 4 + kWaves * kTile * 8 <=
+                                    (size_t)kWaves * kPool * sizeof(bf16),
+              "the sums fit the tiles' LDS");
+static_assert(gB2 == gB1 + kH && gB3 == gB2 + kH, "bias order");
+
+// Gradient and loss partials of a group, workgroup b's at index b; those of
+// workgroups below `started` are added to.
+__global__ __launch_bounds__(kWaves * 64, 1) void spai_backward_kernel(
+    Group G, float* __restrict__ partials, double* __restrict__ loss_part,
+    int started) {
+#pragma clang fp contract(off)
+  __shared__ __attribute__((aligned(16))) bf16 pool[kWaves * kPool];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  bf16* R1 = pool + wave * kPool + oR1;
+  bf16* C1 = pool + wave * kPool + oC1;
+  bf16* C2 = pool + wave * kPool + oC2;
+  bf16* Xc = pool + wave * kPool + oX;
+  bf16* Yr = pool + wave * kPool + oYr;
+  bf16* Yc = pool + wave * kPool + oYc;
+  const Packed& w = *G.pk;
+  bf16x8 w1t[4], w2t[4][2], w2[4][2], w3[4];
+  float b1[4], b2[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int c = q * 16 + r;
+    w1t[q] = frag(w.w1t + c * kFp + 8 * g);
+    w3[q] = frag(w.w3 + c * kOk + 8 * g);
+    b1[q] = w.b1[c];
+    b2[q] = w.b2[c];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      w2t[q][kb] = frag(w.w2t + c * kH + kb * 32 + 8 * g);
+      w2[q][kb] = frag(w.w2 + c * kH + kb * 32 + 8 * g);
+    }
+  }
+  bool add = (int)blockIdx.x < started;
+
+  for (int k = 0; k < G.count; ++k) {
+    const int64_t ntiles = (G.mat[k].n + kTile - 1) / kTile;
+    if ((int64_t)blockIdx.x * kWaves >= ntiles && add) continue;  // + 0
+    floatx4 aW1[2][4], aW2[4][4], aW3[4];
+    float ab1[4], ab2[4], ab3[kO];
+    double lsum = 0.0;
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       aW3[a] = splat(0.f);
@@ -249,255 +552,239 @@ __global__ __launch_bounds__(256) void spai_tile_kernel(TileArgs A) {
       for (int b = 0; b < 4; ++b) aW1[a][b] = splat(0.f);
 #pragma unroll
     for (int s = 0; s < kO; ++s) ab3[s] = 0.f;
-  }
 
-  const int64_t ntiles = (A.n + kTile - 1) / kTile;
-  for (int64_t t = (int64_t)blockIdx.x * kWaves + wave; t < ntiles;
-       t += (int64_t)gridDim.x * kWaves) {
-    // ---- per-row features (lane = row)
-    const int64_t i = t * kTile + lane;
-    const bool valid = i < A.n;
-    int pos[kO];
-    double di = 1.0;
+    for (int64_t t = (int64_t)blockIdx.x * kWaves + wave; t < ntiles;
+         t += (int64_t)gridDim.x * kWaves) {
+      const int64_t row = G.mat[k].xbase + t * kTile;
+      bf16x8 xf[4];
 #pragma unroll
-    for (int s = 0; s < kO; ++s) pos[s] = -1;
-    float x[kF];
+      for (int mt = 0; mt < 4; ++mt)
+        xf[mt] = frag(G.x + (row + mt * 16 + r) * kFp + 8 * g);
+      float dy[kO];
 #pragma unroll
-    for (int f = 0; f < kF; ++f) x[f] = 0.f;
-    if (valid) {
-      row_slots(A.rp, A.ci, i, pos);
-      di = A.diag[i];
+      for (int s = 0; s < kO; ++s) dy[s] = G.y[(row + lane) * kO + s];
+      lsum += G.rowloss[row + lane];
+      {  // dL/dy by rows and by columns, X by columns
+        bf16x8 lo, hi;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int p = pos[k < 4 ? k : k + 1];
-        if (p >= 0) {
-          const int j = A.ci[p];
-          const double dj = A.diag[j];
-          x[k] = (float)(A.v[p] / di);
-          x[8 + k] = (float)((dj - di) / (dj + di));
-          x[16 + k] = (float)(A.rsum[j] / dj);
+        for (int s = 0; s < kOn; ++s) {
+          const bf16 d = to_bf16(s < kO ? dy[s] : 0.f);
+          if (s < kO) ab3[s] += dy[s];
+          if (s < 8) lo[s] = d;
+          else hi[s - 8] = d;
+          Yc[s * kLd + lane] = d;
+        }
+        *(bf16x8*)(Yr + lane * kLdY) = lo;
+        *(bf16x8*)(Yr + lane * kLdY + 8) = hi;
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) Xc[(8 * g + j) * kLd + mt * 16 + r] = xf[mt][j];
+      }
+      // H1 and H2 again
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+          const floatx4 acc = mma(xf[mt], w1t[nt], splat(b1[nt]));
+          bf16x4 h;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            h[e] = to_bf16(fmaxf(acc[e], 0.f));
+            R1[(mt * 16 + 4 * g + e) * kLd + nt * 16 + r] = h[e];
+          }
+          *(bf16x4*)(C1 + (nt * 16 + r) * kLd + mt * 16 + 4 * g) = h;
+        }
+      wave_sync();
+      {
+        bf16x8 hf[4][2];
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int kb = 0; kb < 2; ++kb)
+            hf[mt][kb] = frag(R1 + (mt * 16 + r) * kLd + kb * 32 + 8 * g);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int nt = 0; nt < 4; ++nt) {
+            floatx4 acc = splat(b2[nt]);
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) acc = mma(hf[mt][kb], w2t[nt][kb], acc);
+            bf16x4 h;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = to_bf16(fmaxf(acc[e], 0.f));
+            *(bf16x4*)(C2 + (nt * 16 + r) * kLd + mt * 16 + 4 * g) = h;
+          }
+      }
+      wave_sync();
+      // dW3[64 hid][16 out] += H2^T dY
+      {
+        bf16x8 yf[2];
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) yf[kb] = frag(Yc + r * kLd + kb * 32 + 8 * g);
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int kb = 0; kb < 2; ++kb)
+            aW3[mt] = mma(frag(C2 + (mt * 16 + r) * kLd + kb * 32 + 8 * g), yf[kb],
+                          aW3[mt]);
+      }
+      wave_sync();
+      // dH2 = dY W3^T * [H2 > 0]; outputs from 16 on are zero
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        bf16x8 yf;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) yf[j] = (bf16)0.f;
+        if (g < 2) yf = frag(Yr + (mt * 16 + r) * kLdY + 8 * g);
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+          const floatx4 acc = mma(yf, w3[nt], splat(0.f));
+          bf16x4* own = (bf16x4*)(C2 + (nt * 16 + r) * kLd + mt * 16 + 4 * g);
+          const bf16x4 h = *own;
+          bf16x4 d;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float vv = positive(h[e]) ? acc[e] : 0.f;
+            ab2[nt] += vv;
+            d[e] = to_bf16(vv);
+            R1[(mt * 16 + 4 * g + e) * kLd + nt * 16 + r] = d[e];
+          }
+          *own = d;
         }
       }
-    }
+      wave_sync();
+      // dW2[64 in][64 out] += H1^T dH2
+      {
+        bf16x8 df[4][2];
 #pragma unroll
-    for (int f = 0; f < kFp; ++f) X[lane * kFp + f] = to_bf16(f < kF ? x[f] : 0.f);
-    __builtin_amdgcn_wave_barrier();
-
-    // ---- forward
+        for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+          for (int kb = 0; kb < 2; ++kb)
+            df[nt][kb] = frag(C2 + (nt * 16 + r) * kLd + kb * 32 + 8 * g);
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        floatx4 acc = splat(sw.b1[nt * 16 + r]);
-        acc = mma(X + mt * 16 * kFp, kFp, 1, sw.w1 + nt * 16, kH, 1, acc);
+        for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          H1[(mt * 16 + 4 * g + e) * kH + nt * 16 + r] = to_bf16(fmaxf(acc[e], 0.f));
+          for (int kb = 0; kb < 2; ++kb) {
+            const bf16x8 hf = frag(C1 + (mt * 16 + r) * kLd + kb * 32 + 8 * g);
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt)
+              aW2[mt][nt] = mma(hf, df[nt][kb], aW2[mt][nt]);
+          }
       }
-    __builtin_amdgcn_wave_barrier();
+      wave_sync();
+      // dH1 = dH2 W2^T * [H1 > 0]
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        floatx4 acc = splat(sw.b2[nt * 16 + r]);
+      for (int mt = 0; mt < 4; ++mt) {
+        bf16x8 df[2];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
-          acc = mma(H1 + mt * 16 * kH + kb * 32, kH, 1,
-                    sw.w2 + kb * 32 * kH + nt * 16, kH, 1, acc);
+          df[kb] = frag(R1 + (mt * 16 + r) * kLd + kb * 32 + 8 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          H2[(mt * 16 + 4 * g + e) * kH + nt * 16 + r] = to_bf16(fmaxf(acc[e], 0.f));
-      }
-    __builtin_amdgcn_wave_barrier();
+        for (int nt = 0; nt < 4; ++nt) {
+          floatx4 acc = splat(0.f);
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-      floatx4 acc = splat(sw.b3[r]);
+          for (int kb = 0; kb < 2; ++kb) acc = mma(df[kb], w2[nt][kb], acc);
+          bf16x4* own = (bf16x4*)(C1 + (nt * 16 + r) * kLd + mt * 16 + 4 * g);
+          const bf16x4 h = *own;
+          bf16x4 d;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-        acc = mma(H2 + mt * 16 * kH + kb * 32, kH, 1, sw.w3 + kb * 32 * kOk,
-                  kOk, 1, acc);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) Y[(mt * 16 + 4 * g + e) * kOn + r] = acc[e];
-    }
-    __builtin_amdgcn_wave_barrier();
-    float y[kO];
-#pragma unroll
-    for (int s = 0; s < kO; ++s) y[s] = Y[lane * kOn + s];
-    double m[kO];
-#pragma unroll
-    for (int s = 0; s < kO; ++s)
-      m[s] = pos[s] < 0 ? 0.0 : ((s == 4 ? 1.0 : 0.0) + (double)y[s]) / di;
-
-    if (!TRAIN) {
-      if (valid) {
-#pragma unroll
-        for (int s = 0; s < kO; ++s)
-          if (pos[s] >= 0) A.mvals[pos[s]] = m[s];
-      }
-      __builtin_amdgcn_wave_barrier();
-      continue;
-    }
-
-    // ---- (M A)_i by a merge of the slot rows; g_s = dL/dm_s (or both
-    // from the symmetric objective's passes)
-    double gs[kO];
-#pragma unroll
-    for (int s = 0; s < kO; ++s) gs[s] = 0.0;
-    double lrow = 0.0;
-    if (A.gm) {
-      if (valid) {
-#pragma unroll
-        for (int s = 0; s < kO; ++s) gs[s] = pos[s] >= 0 ? A.gm[pos[s]] : 0.0;
-        lrow = A.rowloss[i];
-      }
-    } else {
-      lrow = row_residual(A.rp, A.ci, A.v, i, pos, m, gs);
-    }
-    if (valid) lsum += lrow;
-    float dy[kO];
-#pragma unroll
-    for (int s = 0; s < kO; ++s) {
-      dy[s] = (valid && pos[s] >= 0) ? (float)(A.scale * gs[s] / di) : 0.f;
-      ab3[s] += dy[s];
-    }
-    // lane's Y row is read; its dY row occupies the same bytes
-#pragma unroll
-    for (int s = 0; s < kOk; ++s) dY[lane * kOk + s] = to_bf16(s < kO ? dy[s] : 0.f);
-    __builtin_amdgcn_wave_barrier();
-
-    // ---- backward
-    // dW3[64 hid][16 out] += H2^T dY
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
-        aW3[mt] = mma(H2 + mt * 16 + kb * 32 * kH, 1, kH, dY + kb * 32 * kOk,
-                      kOk, 1, aW3[mt]);
-    // dH2 = dY W3^T * [H2 > 0] -> D
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        floatx4 acc = mma(dY + mt * 16 * kOk, kOk, 1, sw.w3 + nt * 16 * kOk, 1,
-                          kOk, splat(0.f));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int idx = (mt * 16 + 4 * g + e) * kH + nt * 16 + r;
-          const float vv = from_bf16(H2[idx]) > 0.f ? acc[e] : 0.f;
-          ab2[nt] += vv;
-          D[idx] = to_bf16(vv);
+          for (int e = 0; e < 4; ++e) {
+            const float vv = positive(h[e]) ? acc[e] : 0.f;
+            ab1[nt] += vv;
+            d[e] = to_bf16(vv);
+          }
+          *own = d;
         }
       }
-    __builtin_amdgcn_wave_barrier();
-    // dW2[64 in][64 out] += H1^T dH2
+      wave_sync();
+      // dW1[32 feat][64 hid] += X^T dH1
+      {
+        bf16x8 df[4][2];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+        for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
+          for (int kb = 0; kb < 2; ++kb)
+            df[nt][kb] = frag(C1 + (nt * 16 + r) * kLd + kb * 32 + 8 * g);
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-          aW2[mt][nt] = mma(H1 + mt * 16 + kb * 32 * kH, 1, kH,
-                            D + kb * 32 * kH + nt * 16, kH, 1, aW2[mt][nt]);
-    // dH1 = dH2 W2^T * [H1 > 0] -> H2's region (H2 is no longer read)
+        for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+          for (int kb = 0; kb < 2; ++kb) {
+            const bf16x8 xt = frag(Xc + (mt * 16 + r) * kLd + kb * 32 + 8 * g);
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        floatx4 acc = splat(0.f);
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-          acc = mma(D + mt * 16 * kH + kb * 32, kH, 1, sw.w2 + nt * 16 * kH + kb * 32,
-                    1, kH, acc);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int idx = (mt * 16 + 4 * g + e) * kH + nt * 16 + r;
-          const float vv = from_bf16(H1[idx]) > 0.f ? acc[e] : 0.f;
-          ab1[nt] += vv;
-          H2[idx] = to_bf16(vv);
-        }
+            for (int nt = 0; nt < 4; ++nt)
+              aW1[mt][nt] = mma(xt, df[nt][kb], aW1[mt][nt]);
+          }
       }
-    __builtin_amdgcn_wave_barrier();
-    // dW1[32 feat][64 hid] += X^T dH1
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-          aW1[mt][nt] = mma(X + mt * 16 + kb * 32 * kFp, 1, kFp,
-                            H2 + kb * 32 * kH + nt * 16, kH, 1, aW1[mt][nt]);
-    __builtin_amdgcn_wave_barrier();
-  }
-  if (!TRAIN) return;
+      wave_sync();
+    }
 
-  // ---- workgroup sum of the wavefronts' gradients, in a fixed order:
-  // wavefront by wavefront, and for values several lanes of one wavefront
-  // hold, lane group by lane group (every step behind a workgroup barrier)
-  __syncthreads();
-  float* red = (float*)pool;                        // kGradLen floats
-  double* lt = (double*)(pool + 2 * kGradLen + 8);  // kWaves * 64 doubles
-  for (int w = 0; w < kWaves; ++w) {
-    if (wave == w) {
-      const bool first = w == 0;
+    // ---- workgroup sum of the wavefronts' gradients, in a fixed order:
+    // wavefront by wavefront, and for values several lanes of one wavefront
+    // hold, lane group by lane group (dL/dy and loss: lane by lane)
+    __syncthreads();
+    float* red = (float*)pool;
+    double* lt = (double*)(red + fLoss);
+    float* mine = red + wave * kMats;
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int idx = gW1 + (mt * 16 + 4 * g + e) * kH + nt * 16 + r;
-            red[idx] = (first ? 0.f : red[idx]) + aW1[mt][nt][e];
-          }
+        for (int e = 0; e < 4; ++e)
+          mine[gW1 + (mt * 16 + 4 * g + e) * kH + nt * 16 + r] = aW1[mt][nt][e];
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
+        for (int e = 0; e < 4; ++e)
+          mine[gW2 + (mt * 16 + 4 * g + e) * kH + nt * 16 + r] = aW2[mt][nt][e];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int idx = gW2 + (mt * 16 + 4 * g + e) * kH + nt * 16 + r;
-            red[idx] = (first ? 0.f : red[idx]) + aW2[mt][nt][e];
-          }
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int idx = gW3 + (mt * 16 + 4 * g + e) * kOn + r;
-          red[idx] = (first ? 0.f : red[idx]) + aW3[mt][e];
-        }
-#pragma unroll
-      for (int s = 0; s < kO; ++s) b3tmp[lane * kO + s] = ab3[s];
-      lt[threadIdx.x] = lsum;
+      for (int e = 0; e < 4; ++e)
+        mine[gW3 + (nt * 16 + 4 * g + e) * kOn + r] = aW3[nt][e];
+      red[fB + ((wave * 4 + g) * 2 + 0) * kH + nt * 16 + r] = ab1[nt];
+      red[fB + ((wave * 4 + g) * 2 + 1) * kH + nt * 16 + r] = ab2[nt];
     }
-    for (int gg = 0; gg < 4; ++gg) {
-      __syncthreads();
-      if (wave == w && g == gg) {
-        const bool z = w == 0 && gg == 0;
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-          const int i1 = gB1 + nt * 16 + r, i2 = gB2 + nt * 16 + r;
-          red[i1] = (z ? 0.f : red[i1]) + ab1[nt];
-          red[i2] = (z ? 0.f : red[i2]) + ab2[nt];
-        }
+    for (int s = 0; s < kO; ++s) red[fB3 + threadIdx.x * kO + s] = ab3[s];
+    lt[threadIdx.x] = lsum;
+    __syncthreads();
+    float* dst = partials + (size_t)blockIdx.x * kGradLen;
+    constexpr int kQuads = kMats / 4 / (kWaves * 64);
+    static_assert(kQuads * 4 * kWaves * 64 == kMats && kGradLen % 4 == 0, "quads");
+    floatx4 old[kQuads];
+#pragma unroll
+    for (int q = 0; q < kQuads; ++q)
+      old[q] = add ? ((floatx4*)dst)[q * kWaves * 64 + threadIdx.x] : splat(0.f);
+#pragma unroll
+    for (int q = 0; q < kQuads; ++q) {
+      const int at = q * kWaves * 64 + threadIdx.x;
+      floatx4 v = ((floatx4*)red)[at];
+#pragma unroll
+      for (int u = 1; u < kWaves; ++u) v += ((floatx4*)(red + u * kMats))[at];
+      ((floatx4*)dst)[at] = old[q] + v;
+    }
+    if (threadIdx.x < 2 * kH) {
+      float v = 0.f;
+#pragma unroll
+      for (int u = 0; u < 4 * kWaves; ++u) v += red[fB + u * 2 * kH + threadIdx.x];
+      dst[gB1 + threadIdx.x] = (add ? dst[gB1 + threadIdx.x] : 0.f) + v;
+    } else if (threadIdx.x < 2 * kH + kOn) {
+      const int s = threadIdx.x - 2 * kH;
+      float v = 0.f;
+      if (s < kO) {
+#pragma unroll 16
+        for (int u = 0; u < kWaves * kTile; ++u) v += red[fB3 + u * kO + s];
       }
+      dst[gB3 + s] = (add ? dst[gB3 + s] : 0.f) + v;
+    } else if (threadIdx.x == 3 * kTile) {
+      double l = 0.0;
+#pragma unroll 16
+      for (int u = 0; u < kWaves * kTile; ++u) l += lt[u];
+      loss_part[blockIdx.x] = (add ? loss_part[blockIdx.x] : 0.0) + G.scale * l;
     }
-    __syncthreads();
-    if (threadIdx.x < kOn) {
-      float acc = w == 0 ? 0.f : red[gB3 + threadIdx.x];
-      if (threadIdx.x < kO)
-        for (int l = 0; l < kTile; ++l) acc += b3tmp[l * kO + threadIdx.x];
-      red[gB3 + threadIdx.x] = acc;
-    }
+    add = true;
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    double l = 0.0;
-    for (int k = 0; k < kWaves * 64; ++k) l += lt[k];
-    A.loss_part[blockIdx.x] =
-        (A.accumulate ? A.loss_part[blockIdx.x] : 0.0) + A.scale * l;
-  }
-  float* dst = A.partials + (size_t)blockIdx.x * kGradLen;
-  for (int k = threadIdx.x; k < kGradLen; k += blockDim.x)
-    dst[k] = (A.accumulate ? dst[k] : 0.f) + red[k];
 }
 
 // ---- the symmetric objective (1/n) ||I - S A||_F^2, S = (M + M^T) / 2:
@@ -538,7 +825,7 @@ __global__ void spai_mirror_mean_kernel(int64_t nnz, const double* __restrict__ 
 }
 
 // each row's residual under S's values: the row's loss and g_p = dL/dS_p
-__global__ void spai_row_loss_kernel(int64_t n, const int32_t* __restrict__ rp,
+__global__ __launch_bounds__(kRowBlock) void spai_row_loss_kernel(int64_t n, const int32_t* __restrict__ rp,
                                      const int32_t* __restrict__ ci,
                                      const double* __restrict__ v,
                                      const double* __restrict__ svals,
@@ -546,15 +833,16 @@ __global__ void spai_row_loss_kernel(int64_t n, const int32_t* __restrict__ rp,
                                      double* __restrict__ rowloss) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= n) return;
-  int pos[kO];
-  row_slots(rp, ci, i, pos);
+  const CsrRows A{rp, ci, v};
+  int pos[kO], js[kO];
+  A.slots(i, pos, js);
   double m[kO], gs[kO];
 #pragma unroll
   for (int s = 0; s < kO; ++s) {
     m[s] = pos[s] >= 0 ? svals[pos[s]] : 0.0;
     gs[s] = 0.0;
   }
-  rowloss[i] = row_residual(rp, ci, v, i, pos, m, gs);
+  rowloss[i] = row_residual(A, i, js, m, gs);
 #pragma unroll
   for (int s = 0; s < kO; ++s)
     if (pos[s] >= 0) g[pos[s]] = gs[s];
@@ -571,12 +859,24 @@ __device__ __forceinline__ int partial_index(int k) {
 }
 
 __device__ __forceinline__ void store_packed(Packed* pk, int k, float w) {
-  if (k < kB1) pk->w1[k] = to_bf16(w);
-  else if (k < kW2) pk->b1[k - kB1] = w;
-  else if (k < kB2) pk->w2[k - kW2] = to_bf16(w);
-  else if (k < kW3) pk->b2[k - kB2] = w;
-  else if (k < kB3) pk->w3[((k - kW3) / kO) * kOk + (k - kW3) % kO] = to_bf16(w);
-  else pk->b3[k - kB3] = w;
+  const bf16 b = to_bf16(w);
+  if (k < kB1) {
+    pk->w1t[(k % kH) * kFp + k / kH] = b;
+  } else if (k < kW2) {
+    pk->b1[k - kB1] = w;
+  } else if (k < kB2) {
+    const int q = k - kW2;
+    pk->w2[q] = b;
+    pk->w2t[(q % kH) * kH + q / kH] = b;
+  } else if (k < kW3) {
+    pk->b2[k - kB2] = w;
+  } else if (k < kB3) {
+    const int q = k - kW3;
+    pk->w3[(q / kO) * kOk + q % kO] = b;
+    pk->w3t[(q % kO) * kH + q / kO] = b;
+  } else {
+    pk->b3[k - kB3] = w;
+  }
 }
 
 struct AdamStep {
@@ -584,8 +884,11 @@ struct AdamStep {
 };
 
 // sum the workgroup partials (in workgroup order); either write the
-// gradient (grad != null) or take an Adam step on the master weights
-__global__ void spai_update_kernel(int nparts, const float* __restrict__ partials,
+// gradient (grad != null) or take an Adam step on the master weights.  A
+// chain of nparts additions: the loads of 64 go out together (one at a time
+// it took 74 us at 256 partials).
+constexpr int kUpdateBlock = 64;
+__global__ __launch_bounds__(kUpdateBlock) void spai_update_kernel(int nparts, const float* __restrict__ partials,
                                    const double* __restrict__ loss_part,
                                    float* __restrict__ master, float* __restrict__ m1,
                                    float* __restrict__ m2, Packed* __restrict__ pk,
@@ -593,14 +896,18 @@ __global__ void spai_update_kernel(int nparts, const float* __restrict__ partial
                                    float* __restrict__ grad, AdamStep st) {
 #pragma clang fp contract(off)
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k == 0) {
+  if (blockIdx.x == gridDim.x - 1) {  // a workgroup for the loss
+    if (threadIdx.x > 0) return;
     double l = 0.0;
+#pragma unroll 64
     for (int b = 0; b < nparts; ++b) l += loss_part[b];
     *loss_out = l;
+    return;
   }
   if (k >= kNP) return;
   const int pi = partial_index(k);
   float gsum = 0.f;
+#pragma unroll 64
   for (int b = 0; b < nparts; ++b) gsum += partials[(size_t)b * kGradLen + pi];
   if (grad) {
     grad[k] = gsum;
@@ -632,7 +939,11 @@ struct spk_spai_model_s {
   DevBuf<float> partials;
   DevBuf<double> loss_part, loss_hist;
   DevBuf<float> grad;
-  DevBuf<double> diag, rsum;
+  DevBuf<double> diag, rsum;  // per row of what is prepared
+  DevBuf<bf16> x;             // the passes' scratch, see Group
+  DevBuf<float> y;
+  DevBuf<double> rowloss, eval;
+  DevBuf<int32_t> ecol;
   DevBuf<int> err;
   int64_t step = 0;
   int nparts = 0;
@@ -659,56 +970,112 @@ struct spk_spai_model_s {
     reset_optimizer();
     SPK_HIP_TRY(hipStreamSynchronize(s));
   }
-  // diagonal / row sums of A into the model's scratch; throws on a matrix
-  // the slot rules reject
-  void prepare(spk_csr_s& A, bool check) {
-    SPK_REQUIRE(A.nrows == A.ncols, SPK_INVALID_ARGUMENT,
-                "learned SPAI needs a square matrix");
-    const size_t n = (size_t)A.nrows;
-    if (diag.n < n) {
-      diag.alloc(n);
-      rsum.alloc(n);
+  static int64_t padded(int64_t rows) {
+    return (rows + kRowBlock - 1) / kRowBlock * kRowBlock;
+  }
+  Group group() {
+    Group G{};
+    G.diag = diag.p;
+    G.rsum = rsum.p;
+    G.x = x.p;
+    G.y = y.p;
+    G.rowloss = rowloss.p;
+    G.pk = pk.p;
+    return G;
+  }
+  static RowSpan span(const spk_csr_s& A, int64_t first, int64_t last, int64_t dbase,
+                      int64_t xbase) {
+    return RowSpan{A.rp.p, A.ci.p, A.v64.p, A.nrows, first, last, dbase, xbase};
+  }
+  void need_rows(int64_t rows) {
+    if (diag.n < (size_t)rows) {
+      diag.alloc((size_t)rows);
+      rsum.alloc((size_t)rows);
     }
-    hipStream_t s = stream();
-    if (check) SPK_HIP_TRY(hipMemsetAsync(err.p, 0, sizeof(int), s));
-    hipLaunchKernelGGL(spai_prepare_kernel, dim3(ceil_div(A.nrows, 256)), dim3(256),
-                       0, s, A.nrows, (const int32_t*)A.rp.p,
-                       (const int32_t*)A.ci.p, (const double*)A.v64.p, diag.p,
-                       rsum.p, err.p);
+  }
+  void need_scratch(int64_t rows, bool train) {
+    if (x.n < (size_t)rows * kFp) x.alloc((size_t)rows * kFp);
+    if (y.n < (size_t)rows * kO) y.alloc((size_t)rows * kO);
+    if (train && rowloss.n < (size_t)rows) rowloss.alloc((size_t)rows);
+  }
+  void need_entries(int64_t rows) {
+    if (ecol.n < (size_t)rows * kEntries) ecol.alloc((size_t)rows * kEntries);
+    if (eval.n < (size_t)rows * kEntries) eval.alloc((size_t)rows * kEntries);
+  }
+  void launch_prepare(const Group& G, int64_t rows, int* e) {
+    hipLaunchKernelGGL(spai_prepare_kernel, dim3(ceil_div(rows, kRowBlock)),
+                       dim3(kRowBlock), 0, stream(), G, e);
     SPK_HIP_TRY(hipGetLastError());
-    if (check) {
-      int h = 0;
-      SPK_HIP_TRY(hipMemcpyAsync(&h, err.p, sizeof(int), hipMemcpyDeviceToHost, s));
-      SPK_HIP_TRY(hipStreamSynchronize(s));
-      SPK_REQUIRE(!h, SPK_INVALID_ARGUMENT,
+  }
+  // diagonal / row sums of A into the model's scratch; *e is set for a
+  // matrix the slot rules reject
+  void prepare(spk_csr_s& A, int* e) {
+    need_rows(padded(A.nrows));
+    Group G = group();
+    G.count = 1;
+    G.mat[0] = span(A, 0, A.nrows, 0, 0);
+    launch_prepare(G, A.nrows, e);
+  }
+  // Prepares matrix by matrix, with mirrors for the symmetric objective;
+  // throws what the first rejected one is rejected for.
+  void check(const spk_csr* mats, int64_t count) {
+    const bool sym = objective == SPK_SPAI_LOSS_SYMMETRIC;
+    if (err.n < (size_t)(2 * count)) err.alloc((size_t)(2 * count));
+    hipStream_t s = stream();
+    SPK_HIP_TRY(hipMemsetAsync(err.p, 0, (size_t)(2 * count) * sizeof(int), s));
+    int64_t k = 0;
+    for (; k < count; ++k) {
+      if (!mats[k] || mats[k]->nrows != mats[k]->ncols) break;
+      prepare(*mats[k], err.p + 2 * k);
+      if (sym) mirrors(*mats[k], err.p + 2 * k + 1);
+    }
+    std::vector<int> h((size_t)(2 * count), 0);
+    SPK_HIP_TRY(hipMemcpyAsync(h.data(), err.p, h.size() * sizeof(int),
+                               hipMemcpyDeviceToHost, s));
+    SPK_HIP_TRY(hipStreamSynchronize(s));
+    for (int64_t q = 0; q < k; ++q) {
+      SPK_REQUIRE(!h[(size_t)(2 * q)], SPK_INVALID_ARGUMENT,
                   "learned SPAI needs a positive diagonal and at most 4 "
                   "entries on each side of it in every row");
+      SPK_REQUIRE(!h[(size_t)(2 * q + 1)], SPK_INVALID_ARGUMENT,
+                  "the symmetric objective needs a structurally symmetric pattern");
     }
+    if (k == count) return;
+    SPK_REQUIRE(mats[k], SPK_INVALID_ARGUMENT, "null matrix");
+    SPK_REQUIRE(false, SPK_INVALID_ARGUMENT, "learned SPAI needs a square matrix");
   }
-  TileArgs args(spk_csr_s& A) {
-    TileArgs t{};
-    t.n = A.nrows;
-    t.rp = A.rp.p;
-    t.ci = A.ci.p;
-    t.v = A.v64.p;
-    t.diag = diag.p;
-    t.rsum = rsum.p;
-    t.pk = pk.p;
-    return t;
-  }
-  // grid of a predicting launch over A's row tiles
-  int predict_grid(const spk_csr_s& A) const {
-    const int64_t ntiles = (A.nrows + kTile - 1) / kTile;
-    const int64_t want = (ntiles + kWaves - 1) / kWaves;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(want, nparts));
-  }
-  // M's values on A's pattern (every entry is a slot: prepare checked)
-  void predict_into(spk_csr_s& A, double* mvals) {
-    TileArgs t = args(A);
-    t.mvals = mvals;
-    hipLaunchKernelGGL(spai_tile_kernel<false>, dim3(predict_grid(A)),
-                       dim3(kWaves * 64), 0, stream(), t);
+  void launch_features(const Group& G, int64_t rows) {
+    hipLaunchKernelGGL(spai_features_kernel, dim3((int)(rows / kRowBlock)),
+                       dim3(kRowBlock), 0, stream(), G);
     SPK_HIP_TRY(hipGetLastError());
+  }
+  void launch_forward(const Group& G, int64_t rows) {
+    static_assert(kRowBlock % (kWaves * kTile) == 0, "whole workgroups");
+    hipLaunchKernelGGL(spai_forward_kernel, dim3((int)(rows / (kWaves * kTile))),
+                       dim3(kWaves * 64), 0, stream(), G);
+    SPK_HIP_TRY(hipGetLastError());
+  }
+  template <int MODE>
+  void launch_rows(const Group& G, int64_t rows) {
+    hipLaunchKernelGGL(spai_rows_kernel<MODE>, dim3((int)(rows / kRowBlock)),
+                       dim3(kRowBlock), 0, stream(), G);
+    SPK_HIP_TRY(hipGetLastError());
+  }
+  // M's values on the prepared A's pattern (every entry is a slot: prepare
+  // checked), kGroupRows rows at a time
+  void predict_into(spk_csr_s& A, double* mvals) {
+    need_scratch(padded(std::min(A.nrows, kGroupRows)), false);
+    for (int64_t first = 0; first < A.nrows; first += kGroupRows) {
+      const int64_t last = std::min(A.nrows, first + kGroupRows);
+      Group G = group();
+      G.count = 1;
+      G.mat[0] = span(A, first, last, 0, 0);
+      G.mvals = mvals;
+      const int64_t rows = padded(last - first);
+      launch_features(G, rows);
+      launch_forward(G, rows);
+      launch_rows<kPredict>(G, rows);
+    }
   }
   // The symmetric objective's passes before the backward one: M, the
   // mirrors, S, each row's loss and dL/dS, then dL/dm (into gmv / rowl).
@@ -724,28 +1091,20 @@ struct spk_spai_model_s {
     }
     if (rowl.n < n) rowl.alloc(n);
   }
-  // the mirror positions of A's entries; check: SPK_INVALID_ARGUMENT for a
-  // pattern that is not structurally symmetric
-  void mirrors(const spk_csr_s& A, bool check) {
+  // the mirror positions of A's entries; *e is set for a pattern that is not
+  // structurally symmetric
+  void mirrors(const spk_csr_s& A, int* e) {
     symmetric_scratch(A);
     hipStream_t s = stream();
-    if (check) SPK_HIP_TRY(hipMemsetAsync(err.p, 0, sizeof(int), s));
     hipLaunchKernelGGL(spai_mirror_kernel, dim3((int)ceil_div(A.nrows, 256)),
                        dim3(256), 0, s, A.nrows, (const int32_t*)A.rp.p,
-                       (const int32_t*)A.ci.p, mirror.p, err.p);
+                       (const int32_t*)A.ci.p, mirror.p, e);
     SPK_HIP_TRY(hipGetLastError());
-    if (check) {
-      int h = 0;
-      SPK_HIP_TRY(hipMemcpyAsync(&h, err.p, sizeof(int), hipMemcpyDeviceToHost, s));
-      SPK_HIP_TRY(hipStreamSynchronize(s));
-      SPK_REQUIRE(!h, SPK_INVALID_ARGUMENT,
-                  "the symmetric objective needs a structurally symmetric pattern");
-    }
   }
   void symmetric_grad(spk_csr_s& A) {
     hipStream_t s = stream();
     predict_into(A, mv.p);
-    mirrors(A, false);
+    mirrors(A, err.p);  // checked before
     const int gr = (int)ceil_div(A.nrows, 256);
     const int ge = (int)std::min<int64_t>(ceil_div(A.nnz > 0 ? A.nnz : 1, 256), 65536);
     hipLaunchKernelGGL(spai_mirror_mean_kernel, dim3(ge), dim3(256), 0, s, A.nnz,
@@ -757,19 +1116,63 @@ struct spk_spai_model_s {
                        (const double*)gsv.p, (const int32_t*)mirror.p, gmv.p);
     SPK_HIP_TRY(hipGetLastError());
   }
-  void train_tiles(spk_csr_s& A, double scale, bool accumulate) {
-    TileArgs t = args(A);
-    if (objective == SPK_SPAI_LOSS_SYMMETRIC) {
-      symmetric_grad(A);
-      t.gm = gmv.p;
-      t.rowloss = rowl.p;
+  // The gradient and loss partials of a batch (its matrices checked);
+  // returns the number of workgroups that have one.
+  int train_batch(const std::vector<spk_csr_s*>& batch, double scale) {
+    const bool sym = objective == SPK_SPAI_LOSS_SYMMETRIC;
+    int started = 0;
+    for (size_t k = 0; k < batch.size();) {
+      size_t e = k;
+      int64_t rows = 0;
+      while (e < batch.size() &&
+             (e == k || (!sym && e - k < (size_t)kGroupMats &&
+                         rows + padded(batch[e]->nrows) <= kGroupRows)))
+        rows += padded(batch[e++]->nrows);
+      need_rows(rows);
+      need_scratch(rows, true);
+      if (!sym) need_entries(rows);
+      Group G = group();
+      if (!sym) {
+        G.ecol = ecol.p;
+        G.eval = eval.p;
+      }
+      G.scale = scale;
+      int64_t most = 0, base = 0;
+      for (size_t q = k; q < e; ++q) {
+        const spk_csr_s& A = *batch[q];
+        G.mat[G.count++] = span(A, 0, A.nrows, base, base);
+        base += padded(A.nrows);
+        most = std::max<int64_t>(most, ceil_div(A.nrows, kTile * kWaves));
+      }
+      launch_prepare(G, rows, nullptr);
+      if (sym) {
+        symmetric_grad(*batch[k]);
+        G.gm = gmv.p;
+        G.rl = rowl.p;
+      }
+      launch_features(G, rows);
+      if (sym) {
+        launch_rows<kGiven>(G, rows);
+      } else {
+        launch_forward(G, rows);
+        launch_rows<kMerge>(G, rows);
+      }
+      const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>(most, nparts));
+      hipLaunchKernelGGL(spai_backward_kernel, dim3(blocks), dim3(kWaves * 64), 0,
+                         stream(), G, partials.p, loss_part.p, started);
+      SPK_HIP_TRY(hipGetLastError());
+      started = std::max(started, blocks);
+      k = e;
     }
-    t.partials = partials.p;
-    t.loss_part = loss_part.p;
-    t.scale = scale;
-    t.accumulate = accumulate ? 1 : 0;
-    hipLaunchKernelGGL(spai_tile_kernel<true>, dim3(nparts), dim3(kWaves * 64), 0,
-                       stream(), t);
+    return started;
+  }
+  // sums the batch's partials into loss_hist[at], and into grad or the
+  // weights
+  void update(int parts, int64_t at, float* gradient, const AdamStep& st) {
+    hipLaunchKernelGGL(spai_update_kernel, dim3((kNP + kUpdateBlock - 1) / kUpdateBlock + 1),
+                       dim3(kUpdateBlock), 0, stream(), parts,
+                       (const float*)partials.p, (const double*)loss_part.p, master.p,
+                       m1.p, m2.p, pk.p, loss_hist.p + at, gradient, st);
     SPK_HIP_TRY(hipGetLastError());
   }
 };
@@ -975,44 +1378,20 @@ spk_status spk_spai_model_get_objective(spk_spai_model m, int* objective) {
 spk_status spk_spai_features(spk_csr A, float* d_features) {
   return guarded([&] {
     SPK_REQUIRE(A && d_features, SPK_INVALID_ARGUMENT, "null argument");
-    // computed by the same per-row code as the tile kernel, through a model
-    // whose forward pass is skipped: a dedicated small kernel
+    // computed by the same per-row code as the features pass, through a
+    // model that holds only its scratch
     spk_spai_model_s tmp;
     tmp.err.alloc(1);
-    tmp.prepare(*A, true);
-    const int32_t* rp = A->rp.p;
-    const int32_t* ci = A->ci.p;
-    const double* v = A->v64.p;
+    tmp.check(&A, 1);
+    const CsrRows R{A->rp.p, A->ci.p, A->v64.p};
     const double* diag = tmp.diag.p;
     const double* rsum = tmp.rsum.p;
     float* X = d_features;
     launch_map(A->nrows, [=] __device__(int64_t i) {
-      const int p0 = rp[i], p1 = rp[i + 1];
-      int d = p0;
-      while (ci[d] != (int32_t)i) ++d;
-      int pos[kO];
-      pos[4] = d;
+      float x[kF];
+      row_features(R, diag, rsum, i, x);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        pos[3 - k] = (d - 1 - k >= p0) ? d - 1 - k : -1;
-        pos[5 + k] = (d + 1 + k < p1) ? d + 1 + k : -1;
-      }
-      const double di = diag[i];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int p = pos[k < 4 ? k : k + 1];
-        float a = 0.f, b = 0.f, c = 0.f;
-        if (p >= 0) {
-          const int j = ci[p];
-          const double dj = diag[j];
-          a = (float)(v[p] / di);
-          b = (float)((dj - di) / (dj + di));
-          c = (float)(rsum[j] / dj);
-        }
-        X[i * kF + k] = a;
-        X[i * kF + 8 + k] = b;
-        X[i * kF + 16 + k] = c;
-      }
+      for (int f = 0; f < kF; ++f) X[i * kF + f] = x[f];
     });
     SPK_HIP_TRY(hipStreamSynchronize(stream()));
   });
@@ -1022,15 +1401,10 @@ spk_status spk_spai_loss_grad(spk_spai_model m, spk_csr A, double* loss,
                               float* grad) {
   return guarded([&] {
     SPK_REQUIRE(m && A && loss, SPK_INVALID_ARGUMENT, "null argument");
-    m->prepare(*A, true);
-    if (m->objective == SPK_SPAI_LOSS_SYMMETRIC) m->mirrors(*A, true);
-    m->train_tiles(*A, 1.0 / (double)A->nrows, false);
+    m->check(&A, 1);
+    const int parts = m->train_batch({A}, 1.0 / (double)A->nrows);
     hipStream_t s = stream();
-    hipLaunchKernelGGL(spai_update_kernel, dim3((kNP + 255) / 256), dim3(256), 0,
-                       s, m->nparts, (const float*)m->partials.p,
-                       (const double*)m->loss_part.p, m->master.p, m->m1.p,
-                       m->m2.p, m->pk.p, m->loss_hist.p, m->grad.p, AdamStep{});
-    SPK_HIP_TRY(hipGetLastError());
+    m->update(parts, 0, m->grad.p, AdamStep{});
     SPK_HIP_TRY(hipMemcpyAsync(loss, m->loss_hist.p, 8, hipMemcpyDeviceToHost, s));
     if (grad)
       SPK_HIP_TRY(hipMemcpyAsync(grad, m->grad.p, kNP * 4, hipMemcpyDeviceToHost, s));
@@ -1048,11 +1422,7 @@ spk_status spk_spai_train(spk_spai_model m, const spk_csr* mats, int64_t count,
     SPK_REQUIRE(cfg->epochs >= 0 && cfg->batch_matrices > 0 &&
                     cfg->learning_rate > 0.0,
                 SPK_INVALID_ARGUMENT, "bad training configuration");
-    for (int64_t k = 0; k < count; ++k) {
-      SPK_REQUIRE(mats[k], SPK_INVALID_ARGUMENT, "null matrix");
-      m->prepare(*mats[k], true);
-      if (m->objective == SPK_SPAI_LOSS_SYMMETRIC) m->mirrors(*mats[k], true);
-    }
+    m->check(mats, count);
     const int64_t per_epoch = (count + cfg->batch_matrices - 1) / cfg->batch_matrices;
     const int64_t total = cfg->epochs * per_epoch;
     if (m->loss_hist.n < (size_t)(total > 0 ? total : 1))
@@ -1070,12 +1440,12 @@ spk_status spk_spai_train(spk_spai_model m, const spk_csr* mats, int64_t count,
       for (int64_t b0 = 0; b0 < count; b0 += cfg->batch_matrices) {
         const int64_t b1e = std::min(count, b0 + cfg->batch_matrices);
         int64_t rows = 0;
-        for (int64_t k = b0; k < b1e; ++k) rows += mats[order[(size_t)k]]->nrows;
+        std::vector<spk_csr_s*> batch;
         for (int64_t k = b0; k < b1e; ++k) {
-          spk_csr_s& A = *mats[order[(size_t)k]];
-          m->prepare(A, false);
-          m->train_tiles(A, 1.0 / (double)rows, k > b0);
+          batch.push_back(mats[order[(size_t)k]]);
+          rows += batch.back()->nrows;
         }
+        const int parts = m->train_batch(batch, 1.0 / (double)rows);
         m->step += 1;
         AdamStep st;
         st.lr = (float)cfg->learning_rate;
@@ -1084,12 +1454,7 @@ spk_status spk_spai_train(spk_spai_model m, const spk_csr* mats, int64_t count,
         st.eps = 1e-8f;
         st.bc1 = (float)(1.0 - std::pow((double)b1, (double)m->step));
         st.bc2 = (float)(1.0 - std::pow((double)b2, (double)m->step));
-        hipLaunchKernelGGL(spai_update_kernel, dim3((kNP + 255) / 256), dim3(256),
-                           0, s, m->nparts, (const float*)m->partials.p,
-                           (const double*)m->loss_part.p, m->master.p, m->m1.p,
-                           m->m2.p, m->pk.p, m->loss_hist.p + h, (float*)nullptr,
-                           st);
-        SPK_HIP_TRY(hipGetLastError());
+        m->update(parts, h, nullptr, st);
         ++h;
       }
     }
@@ -1104,7 +1469,7 @@ spk_status spk_spai_predict(spk_spai_model m, spk_csr A, spk_csr* M_out) {
   return guarded([&] {
     TraceRange trace_("spk_spai_predict");
     SPK_REQUIRE(m && A && M_out, SPK_INVALID_ARGUMENT, "null argument");
-    m->prepare(*A, true);
+    m->check(&A, 1);
     spk_csr_s* M = clone_pattern(*A);
     try {
       m->predict_into(*A, M->v64.p);
