@@ -151,6 +151,11 @@ __global__ __launch_bounds__(256) void pat_insert_kernel(int64_t n,
         }
       }
       if (k == h) break;
+      // a store of rows that do not repeat fills the table at once: its
+      // threads leave (probing on to the end took 1.6 ms at 1.1 million rows)
+      if ((probe & 3) == 3 &&
+          __hip_atomic_load(&t->fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        return;
     }
   }
 }
