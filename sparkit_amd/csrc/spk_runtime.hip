@@ -84,6 +84,7 @@ class Pool {
     std::lock_guard<std::mutex> lk(m_);
     if (!open()) return hipMalloc(p, bytes);
     Size& c = sizes_[size];
+    c.used = ++uses_;
     if (c.ready.empty() && c.idle.size() >= idle_limit(size)) {
       if (hipDeviceSynchronize() == hipSuccess) {
         for (auto& s : sizes_) {
@@ -120,13 +121,16 @@ class Pool {
     const size_t size = it->second;
     owned_.erase(it);
     if (!open()) return false;
-    if (size > kLargest || kept_ + size > kMost || blocks_ >= kMostBlocks) {
+    if (size > kLargest) {
       (void)hipFree(p);
       return true;
     }
-    sizes_[size].idle.push_back(p);
+    Size& c = sizes_[size];
+    c.idle.push_back(p);
+    c.used = ++uses_;
     kept_ += size;
     ++blocks_;
+    while (kept_ > kMost || blocks_ > kMostBlocks) evict();
     return true;
   }
   void drain() {
@@ -137,6 +141,7 @@ class Pool {
  private:
   struct Size {
     std::vector<void*> ready, idle;
+    unsigned long long used = 0;  // when it was last asked for or freed into
   };
   static constexpr size_t kMost = size_t(2) << 30;      // bytes kept, at most
   static constexpr size_t kLargest = size_t(256) << 20;  // a kept block's size
@@ -172,6 +177,19 @@ class Pool {
     } catch (const std::bad_alloc&) {  // then it goes back by hipFree
     }
   }
+  // a block of the size that has lain longest goes back
+  void evict() {
+    auto old = sizes_.end();
+    for (auto it = sizes_.begin(); it != sizes_.end(); ++it)
+      if ((!it->second.ready.empty() || !it->second.idle.empty()) &&
+          (old == sizes_.end() || it->second.used < old->second.used))
+        old = it;
+    std::vector<void*>& v = old->second.ready.empty() ? old->second.idle : old->second.ready;
+    (void)hipFree(v.back());
+    v.pop_back();
+    kept_ -= old->first;
+    --blocks_;
+  }
   void give_back() {  // hipFree waits for the device itself
     for (auto& s : sizes_) {
       for (void* p : s.second.ready) (void)hipFree(p);
@@ -184,6 +202,7 @@ class Pool {
   std::map<size_t, Size> sizes_;
   std::unordered_map<void*, size_t> owned_;
   size_t kept_ = 0, blocks_ = 0;
+  unsigned long long uses_ = 0;
 };
 Pool& pool() {
   static Pool* p = new Pool();  // outlives the objects that free into it

@@ -29,6 +29,21 @@ def test_sizes(spk, n):
         del a, b
 
 
+def test_more_than_the_pool_keeps(spk):
+    """3 GB of freed vectors of one size, then many small ones: the pool
+    returns the oldest, and every vector still holds its own values."""
+    big = [spk.DeviceVector.zeros(1 << 24) for _ in range(24)]
+    del big
+    small = [spk.DeviceVector.from_numpy(np.full(100 + k, float(k))) for k in range(700)]
+    small2 = small[::2]
+    del small
+    again = [spk.DeviceVector.from_numpy(np.full(100 + k, -1.0)) for k in range(700)]
+    for k, v in enumerate(small2):
+        assert np.array_equal(v.numpy(), np.full(100 + 2 * k, 2.0 * k))
+    for k, v in enumerate(again):
+        assert np.array_equal(v.numpy(), np.full(100 + k, -1.0))
+
+
 def test_freed_while_in_use(spk):
     """multiply's result is dropped and made again while the products are
     queued: each kept one holds its own product."""
