@@ -1077,6 +1077,9 @@ def main():
              "spmv_dot_us": round(dus, 2), "spmv_dot_GBs": round(dgbs, 1),
              "spmv_dot_frac_hbm_peak": round(dgbs / HBM_PEAK_GBS, 4),
              "spmv_bytes": bs, "spmv_layout": inp.layout}
+        if gbs > HBM_PEAK_GBS:
+            r["spmv_rate_note"] = ("the CSR form's bytes over the time; a store "
+                                   "whose rows repeat reads one byte a row")
         panels = inp.A.panels
         if panels > 1:
             # rows scatter over all columns: every product is a random
