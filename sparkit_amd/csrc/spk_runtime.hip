@@ -113,25 +113,30 @@ class Pool {
     if (e == hipSuccess) own(*p, size);
     return e;
   }
-  // false: not a block of this pool
-  bool put(void* p) {
+  enum Put { kTaken, kForeign, kFreed };  // kFreed: it has been freed before
+  Put put(void* p) {
     std::lock_guard<std::mutex> lk(m_);
     auto it = owned_.find(p);
-    if (it == owned_.end()) return false;
-    const size_t size = it->second;
-    owned_.erase(it);
-    if (!open()) return false;
+    if (it == owned_.end()) return kForeign;
+    if (it->second.kept) return kFreed;
+    const size_t size = it->second.size;
+    if (!open()) {
+      owned_.erase(it);
+      return kForeign;
+    }
     if (size > kLargest) {
+      owned_.erase(it);
       (void)hipFree(p);
-      return true;
+      return kTaken;
     }
     Size& c = sizes_[size];
     c.idle.push_back(p);
     c.used = ++uses_;
+    it->second.kept = true;
     kept_ += size;
     ++blocks_;
     while (kept_ > kMost || blocks_ > kMostBlocks) evict();
-    return true;
+    return kTaken;
   }
   void drain() {
     std::lock_guard<std::mutex> lk(m_);
@@ -139,6 +144,10 @@ class Pool {
   }
 
  private:
+  struct Block {
+    size_t size;
+    bool kept;
+  };
   struct Size {
     std::vector<void*> ready, idle;
     unsigned long long used = 0;  // when it was last asked for or freed into
@@ -171,9 +180,13 @@ class Pool {
     }
     return dev == g_ctx.device && st == hipStreamCaptureStatusNone;
   }
+  void drop(void* p) {
+    owned_.erase(p);
+    (void)hipFree(p);
+  }
   void own(void* p, size_t size) {
     try {
-      owned_[p] = size;
+      owned_[p] = Block{size, false};
     } catch (const std::bad_alloc&) {  // then it goes back by hipFree
     }
   }
@@ -185,22 +198,22 @@ class Pool {
           (old == sizes_.end() || it->second.used < old->second.used))
         old = it;
     std::vector<void*>& v = old->second.ready.empty() ? old->second.idle : old->second.ready;
-    (void)hipFree(v.back());
+    drop(v.back());
     v.pop_back();
     kept_ -= old->first;
     --blocks_;
   }
   void give_back() {  // hipFree waits for the device itself
     for (auto& s : sizes_) {
-      for (void* p : s.second.ready) (void)hipFree(p);
-      for (void* p : s.second.idle) (void)hipFree(p);
+      for (void* p : s.second.ready) drop(p);
+      for (void* p : s.second.idle) drop(p);
     }
     sizes_.clear();
     kept_ = blocks_ = 0;
   }
   std::mutex m_;
   std::map<size_t, Size> sizes_;
-  std::unordered_map<void*, size_t> owned_;
+  std::unordered_map<void*, Block> owned_;  // handed out or kept
   size_t kept_ = 0, blocks_ = 0;
   unsigned long long uses_ = 0;
 };
@@ -238,12 +251,12 @@ void set_error(const std::string& msg) { g_last_error = msg; }
 
 hipError_t pool_malloc(void** p, size_t bytes) { return pool().get(p, bytes); }
 void pool_free(void* p) {
-  bool kept = false;
+  Pool::Put r = Pool::kForeign;
   try {
-    kept = pool().put(p);
+    r = pool().put(p);
   } catch (const std::bad_alloc&) {  // called by destructors
   }
-  if (!kept) (void)hipFree(p);
+  if (r == Pool::kForeign) (void)hipFree(p);
 }
 
 Context& ctx() {
@@ -422,7 +435,10 @@ spk_status spk_malloc(void** dptr, size_t bytes) {
 spk_status spk_free(void* dptr) {
   return guarded([&] {
     ctx();
-    if (!dptr || pool().put(dptr)) return;
+    if (!dptr) return;
+    const Pool::Put r = pool().put(dptr);
+    if (r == Pool::kTaken) return;
+    if (r == Pool::kFreed) SPK_HIP_TRY(hipErrorInvalidValue);  // as hipFree says
     SPK_HIP_TRY(hipStreamSynchronize(stream()));
     SPK_HIP_TRY(hipFree(dptr));
   });

@@ -111,3 +111,18 @@ print("ok")
 """
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
     assert r.stdout.strip().endswith("ok"), r.stderr
+
+
+def test_a_second_free_is_refused(spk):
+    """The pool keeps the block, and the next owners get distinct ones."""
+    import ctypes as C
+
+    from sparkit_amd import _lib
+    for nbytes in (64, 4096, 1 << 20):
+        p = C.c_void_p()
+        _lib.call("spk_malloc", C.byref(p), nbytes)
+        _lib.call("spk_free", p)
+        with pytest.raises(spk.SpkError):
+            _lib.call("spk_free", p)
+        vs = [spk.DeviceVector(nbytes // 8) for _ in range(40)]
+        assert len({v.ptr.value for v in vs}) == 40
