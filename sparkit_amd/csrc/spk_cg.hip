@@ -590,8 +590,7 @@ extern "C" spk_status spk_cg_solve_noalloc(spk_csr A, spk_precond M_left,
     const size_t vb = arena_round((size_t)(n > 0 ? n : 1) * (fp32 ? 4 : 8));
     const size_t partials =
         std::max(blocks, (size_t)2 * (size_t)vec_grid(n > 0 ? n : 1));
-    size_t need = 5 * vb + arena_round(kLinkWords * sizeof(unsigned long long)) +
-                  arena_round(sizeof(double) * partials) +
+    size_t need = 5 * vb + arena_round(sizeof(double) * partials) +
                   3 * arena_round(sizeof(double) * 2 * (size_t)kProMaxPartials) +
                   arena_round(1024);
     if (cfg->collect_residuals)

@@ -34,8 +34,7 @@ struct GridLink {
 constexpr size_t kLinkSlotWords = (size_t)2 * kLinkWidth * kLinkBlocks * 2;
 constexpr size_t kLinkWords = kLinkSlotWords + 2;
 
-// The link's device memory (zeroed when made; under a no-allocation scope a
-// piece of its scratch, cleared by a kernel).
+// The library's link; its device memory is made and cleared with the library.
 GridLink grid_link();
 // Throws SPK_HIP_ERROR when an exchange's bounded wait has expired
 // (synchronises); the flag is cleared.

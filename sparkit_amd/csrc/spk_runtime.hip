@@ -28,7 +28,6 @@ struct Arena {
   size_t slot_bytes[kArenaSlots] = {};
   double* partials = nullptr;
   size_t partials_count = 0;
-  GridLink link{};
 };
 Arena* g_arena = nullptr;
 
@@ -58,13 +57,11 @@ __global__ void link_clear_kernel(unsigned long long* w, int n) {
   if (k < n) w[k] = 0;
 }
 
-// a link over kLinkWords words at w, cleared
-GridLink make_link(unsigned long long* w) {
+// the link's words: slots, tag and flag
+void clear_link(unsigned long long* w, hipStream_t s) {
   const int n = (int)kLinkWords;
-  hipLaunchKernelGGL(link_clear_kernel, dim3((n + 255) / 256), dim3(256), 0, stream(),
-                     w, n);
+  hipLaunchKernelGGL(link_clear_kernel, dim3((n + 255) / 256), dim3(256), 0, s, w, n);
   SPK_HIP_TRY(hipGetLastError());
-  return GridLink{w, (unsigned*)(w + kLinkSlotWords), (int*)(w + kLinkSlotWords + 1)};
 }
 
 // ---- the device memory pool
@@ -244,6 +241,10 @@ void init_device(int device) {
   SPK_HIP_TRY(hipEventCreate(&g_ev1));
   g_partials = new DevBuf<double>(1 << 16);
   g_ws.reset(new Workspace());
+  // made here, so that a solve which may not allocate has it too
+  g_link = new DevBuf<unsigned long long>(kLinkWords);
+  clear_link(g_link->p, g_ctx.stream);
+  SPK_HIP_TRY(hipStreamSynchronize(g_ctx.stream));
 }
 }  // namespace
 
@@ -332,19 +333,8 @@ double* reduce_partials(size_t count) {
 
 GridLink grid_link() {
   ctx();
-  if (g_arena) {
-    Arena& a = *g_arena;
-    if (!a.link.slots)
-      a.link = make_link((unsigned long long*)arena_carve(
-          a, kLinkWords * sizeof(unsigned long long)));
-    return a.link;
-  }
-  static GridLink link;  // of g_link's memory
-  if (!g_link) {
-    g_link = new DevBuf<unsigned long long>(kLinkWords);
-    link = make_link(g_link->p);
-  }
-  return link;
+  unsigned long long* w = g_link->p;
+  return GridLink{w, (unsigned*)(w + kLinkSlotWords), (int*)(w + kLinkSlotWords + 1)};
 }
 
 void check_link(const GridLink& l) {
@@ -352,7 +342,7 @@ void check_link(const GridLink& l) {
   SPK_HIP_TRY(hipMemcpyAsync(&h, l.expired, sizeof(int), hipMemcpyDeviceToHost, stream()));
   SPK_HIP_TRY(hipStreamSynchronize(stream()));
   if (!h) return;
-  (void)make_link(l.slots);  // flag and slots cleared
+  clear_link(l.slots, stream());
   SPK_HIP_TRY(hipStreamSynchronize(stream()));
   SPK_REQUIRE(false, SPK_HIP_ERROR,
               "grid exchange: a bounded wait expired (results invalid)");

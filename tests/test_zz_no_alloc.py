@@ -126,3 +126,22 @@ def test_noalloc_cg_rejects_what_it_cannot_hold(spk):
     with pytest.raises(spk.InvalidArgument, match="FP32 copy"):
         spk.conjugate_gradient_noalloc(
             b32, x32, spk.CGConfig(1e-6, 100, 100, False, spk.F32), fresh)
+
+
+@pytest.mark.parametrize("over", [0, 1])
+def test_noalloc_cg_residual_history_that_just_fits(spk, over):
+    """A residual history that fills the 64 MiB beside what a solve of 64
+    rows needs (five vectors of 512 bytes, 256 bytes of reduction partials,
+    three hand-off arrays of 65,536, 1,024 for the state, each a multiple of
+    256) is taken; an iteration more is refused."""
+    room = (64 << 20) - (5 * 512 + 256 + 3 * 65536 + 1024)
+    A = spk.poisson_2d(8, 8, 0.25)
+    b, x = spk.uniform_pm1(3, A.nrows), spk.DeviceVector.zeros(A.nrows)
+    cfg = spk.CGConfig(1e-10, 1000, room // 8 + over, True, spk.F64)
+    if over:
+        with pytest.raises(spk.InvalidArgument, match="scratch"):
+            spk.conjugate_gradient_noalloc(b, x, cfg, A, spk.jacobi(A))
+        return
+    s = spk.conjugate_gradient_noalloc(b, x, cfg, A, spk.jacobi(A))
+    assert s.converged and len(s.iteration_residuals) == s.computed_iterations
+    assert spk.true_relres(A, b, x) < 1e-9
