@@ -60,6 +60,15 @@ void* spk_get_stream(void);
 spk_status spk_synchronize(void);
 spk_status spk_device_info(int* num_cus, char* name, size_t name_len);
 
+/* Some kernels of (F)GMRES and CG exchange sums between blocks that all have
+ * to be running.  While other work on the GPU keeps some of them from
+ * starting, the others wait, about 0.1 s at most; the solve, or its restart
+ * cycle, is then taken back and done by kernels that wait for nobody, with
+ * the same result up to rounding.  On a stream with a CU mask those are used
+ * from the start.  For tests: the polls after which such a wait gives up
+ * (0: the default). */
+spk_status spk_set_exchange_polls(uint32_t polls);
+
 /* Device memory from a pool of at most 2 GiB of freed blocks, given back by
  * spk_finalize and when an allocation would fail.  Freed memory is handed out
  * again only after all work on the device queued before the spk_free has

@@ -49,7 +49,7 @@ struct CgState {
   double bnorm, rz, alpha, beta, resnorm, tol;
   int64_t iters;
   int32_t done, converged, collect;
-  int32_t expired;  // a grid exchange's bounded wait ended without its value
+  int32_t expired;  // an exchange between blocks did not go through
   double* history;
   // one-kernel hand-off path: rz by step parity (a kernel reads one and
   // writes the other), the step whose residual update ran
@@ -67,14 +67,13 @@ struct CgCtl {
   __device__ void record(int step, double rr) const {
     if (st->collect) st->history[st->iters + step] = sqrt(rr);
   }
-  __device__ void finish(int steps, double rr, double, double rz, bool ended,
-                         bool ok) const {
+  __device__ void finish(int steps, double rr, double, double rz, bool ended) const {
     st->iters += steps;
     st->resnorm = sqrt(rr);
     st->rz = rz;
-    if (ended && ok) st->converged = 1;
-    if (ended) st->done = 1;
+    if (ended) st->converged = st->done = 1;
   }
+  __device__ void expire() const { st->expired = 1; }
 };
 constexpr int kCgSteps = 4096;  // steps of one launch, at most
 constexpr int kCgQueue = 8;     // launches between two looks at the state,
@@ -242,24 +241,19 @@ void cg_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
   const int* done = &S->done;
   // the one-kernel hand-off needs few partials: every block of the next
   // kernel reads all of them
-  const bool steps_fit = right_id && (jac || is_identity(ML)) && cg_steps_fit<T>(*A);
-  const bool handoff = !steps_fit && right_id && (jac || spmv_left) &&
+  const GridLink link = grid_link();
+  const bool steps_fit = right_id && (jac || is_identity(ML)) && cg_steps_fit<T>(*A, link);
+  const bool handoff = right_id && (jac || spmv_left) &&
                        spmv_partials_count<T>(*A) <= kProMaxPartials &&
                        (!spmv_left || spmv_partials_count<T>(*ML->M) <= kProMaxPartials) &&
                        pro_grid(n) <= kProMaxPartials;
   // Jacobi-PCG whose SpMV has too many row blocks for a prologue: the SpMV
   // keeps its finisher (alpha), the r update hands its partials to the
   // x / p pass
-  const bool mixed = !steps_fit && !handoff && right_id && jac && pro_grid(n) <= kProMaxPartials;
+  const bool mixed = !handoff && right_id && jac && pro_grid(n) <= kProMaxPartials;
   double* part1 = nullptr;
   double* part2 = nullptr;
   double* part3 = nullptr;
-  if (handoff || mixed) {
-    const size_t pb = sizeof(double) * 2 * (size_t)kProMaxPartials;
-    part1 = (double*)ws.get(kWsCg + 7, pb);
-    part2 = (double*)ws.get(kWsCg + 8, pb);
-    part3 = (double*)ws.get(kWsCg + 9, pb);
-  }
 
   auto restart = [&](int64_t k) {  // reorthogonalize(), :216-230
     if (jac) {
@@ -453,8 +447,9 @@ void cg_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
   };
   auto is_done = [&]() { return st.download().done != 0; };
   if (steps_fit) {
-    const GridLink link = grid_link();
-    const int* expired = link.expired;
+    // x0, for a solve that has to be taken back (this path has no use for q)
+    const CgState start = h;
+    if (!cg_one_block<T>(*A)) launch_map(n, [=] __device__(int64_t i) { q[i] = x[i]; });
     for (int64_t k = 0; k < cfg->max_iterations;) {
       // short restart intervals: several launches between two looks
       int64_t queued = 0;
@@ -466,15 +461,26 @@ void cg_solve(spk_csr_s* A, spk_precond_s* ML, spk_precond_s* MR,
         k += m;
         queued += m;
       }
-      launch_map(1, [=] __device__(int64_t) { S->expired = *expired; });
-      if (is_done()) break;
+      h = st.download();
+      if (h.done || h.expired) break;
     }
-  } else {
+    if (h.expired) {  // (several blocks) again from x0, by the kernels per step
+      renew_link(link);
+      launch_map(n, [=] __device__(int64_t i) { x[i] = q[i]; });
+      st.upload(start);
+    }
+  }
+  if (!steps_fit || h.expired) {
+    if (handoff || mixed) {
+      const size_t pb = sizeof(double) * 2 * (size_t)kProMaxPartials;
+      part1 = (double*)ws.get(kWsCg + 7, pb);
+      part2 = (double*)ws.get(kWsCg + 8, pb);
+      part3 = (double*)ws.get(kWsCg + 9, pb);
+    }
     chunked_loop(cfg->max_iterations, issue, is_done);
   }
 
   h = st.download();
-  if (h.expired) check_link(grid_link());
   out->residual_norm = h.resnorm;
   out->computed_iterations = h.iters;
   out->converged = h.converged;

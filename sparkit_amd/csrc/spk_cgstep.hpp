@@ -41,12 +41,11 @@ __device__ __forceinline__ float fma_t(float a, float b, float c) {
 template <typename T>
 constexpr int cg_entry_regs = 2 * (int)(sizeof(T) / 4) + 1;
 
-// Rows per thread: the fewest that leave at most 256 blocks; 0: the rows'
+// Rows per thread: the fewest that leave at most `blocks` blocks; 0: the rows'
 // entries do not fit (four rows of nine FP64 entries would need 180 registers
 // for the entries alone).  K: entries a row holds (padded).
 template <typename T>
-inline int cg_rows_per_thread(int64_t n, int K) {
-  const int blocks = std::min(kLinkBlocks, ctx().num_cus);
+inline int cg_rows_per_thread(int64_t n, int K, int blocks) {
   const int64_t r = (n + (int64_t)blocks * kCgBlock - 1) / ((int64_t)blocks * kCgBlock);
   const int limit = K * cg_entry_regs<T> * 4 <= 160 ? 4 : 3;
   return r <= limit ? (int)r : 0;
@@ -54,20 +53,28 @@ inline int cg_rows_per_thread(int64_t n, int K) {
 inline int cg_row_entries(const spk_csr_s& A) {
   return A.max_len <= 5 ? 5 : A.max_len <= 7 ? 7 : A.max_len <= 9 ? 9 : 0;
 }
+// One block, whose exchanges stay in LDS, holds the rows.
+template <typename T>
+bool cg_one_block(const spk_csr_s& A) {
+  const int limit = cg_row_entries(A) * cg_entry_regs<T> * 4 <= 160 ? 4 : 3;
+  return A.nrows <= (int64_t)kCgBlock * limit;
+}
 // the plain layout with short rows, few enough of them
 template <typename T>
-bool cg_steps_fit(const spk_csr_s& A) {
+bool cg_steps_fit(const spk_csr_s& A, const GridLink& link) {
   const int K = cg_row_entries(A);
   return K > 0 && A.nrows == A.ncols && A.panels.empty() && A.xt_groups == 0 &&
          !(std::is_same<T, float>::value && A.half32) &&
-         cg_rows_per_thread<T>(A.nrows, K) > 0;
+         cg_rows_per_thread<T>(A.nrows, K, link.blocks) > 0;
 }
 
 // Ctl::skip(): the launch is a no-op.  Ctl::rz(): <r, z> at the start.
 // Ctl::ends(rr): whether the step with |r|^2 = rr is the last of the solve
 // (p is then left as it is).  Ctl::record(step, rr) after every step and
-// Ctl::finish(steps, rr, rz before the last step, rz after it, ended, ok) run
-// in one thread of block 0 and touch only what no block reads again.
+// Ctl::finish(steps, rr, rz before the last step, rz after it, ended) run in
+// one thread of block 0 and touch only what no block reads again.
+// Ctl::expire(): an exchange did not go through; x, r and p are then parts of
+// several steps' and the launch, with those queued after it, is to be undone.
 template <typename T, int K, int R, typename Ctl>
 __global__ __launch_bounds__(kCgBlock + 64) void cg_steps_kernel(
     unsigned n, const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
@@ -76,6 +83,7 @@ __global__ __launch_bounds__(kCgBlock + 64) void cg_steps_kernel(
     GridLink link) {
   __shared__ double red[link_lds(kCgBlock)];
   if (ctl.skip()) return;  // set only after every block has been here
+  const int stale = link_open<kCgBlock>(link);
   unsigned tag = *link.tag;
   double rz = ctl.rz();
   const unsigned i0 =
@@ -110,7 +118,7 @@ __global__ __launch_bounds__(kCgBlock + 64) void cg_steps_kernel(
     }
   }
   double rr = 0.0, rz0 = rz;
-  bool ok = true, ended = false;
+  bool ended = false;
   int done = 0;
   while (done < steps && !ended) {
     T q[R];
@@ -124,7 +132,7 @@ __global__ __launch_bounds__(kCgBlock + 64) void cg_steps_kernel(
       q[u] = s;
       s1[0] += (double)pv[u] * (double)s;
     }
-    ok = ok && link_sum<1, kCgBlock>(link, ++tag, s1, red);
+    if (!link_sum<1, kCgBlock>(link, stale, ++tag, s1, red)) break;
     const T a = (T)(rz / s1[0]);
     double s2[2] = {0.0, 0.0};
     T zv[R];
@@ -141,10 +149,10 @@ __global__ __launch_bounds__(kCgBlock + 64) void cg_steps_kernel(
     }
     // z has reached memory before this block's sums say so
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    ok = ok && link_sum<2, kCgBlock>(link, ++tag, s2, red);
+    if (!link_sum<2, kCgBlock>(link, stale, ++tag, s2, red)) break;
     rr = s2[0];
     rz0 = rz;
-    ended = !ok || ctl.ends(rr);
+    ended = ctl.ends(rr);
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl.record(done, rr);
     ++done;
     if (!ended) {
@@ -165,6 +173,10 @@ __global__ __launch_bounds__(kCgBlock + 64) void cg_steps_kernel(
       }
     }
   }
+  if (done < steps && !ended) {  // an exchange did not go through
+    if (threadIdx.x == 0) ctl.expire();
+    return;
+  }
 #pragma unroll
   for (int u = 0; u < R; ++u) {
     const unsigned i = i0 + u * kCgBlock;
@@ -175,8 +187,8 @@ __global__ __launch_bounds__(kCgBlock + 64) void cg_steps_kernel(
     }
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    if (gridDim.x > 1) *link.tag = tag;
-    ctl.finish(done, rr, rz0, rz, ended, ok);
+    link_close(link, tag);
+    ctl.finish(done, rr, rz0, rz, ended);
   }
 }
 
@@ -185,10 +197,8 @@ template <typename T, typename Ctl>
 void launch_cg_steps(spk_csr_s& A, const T* invd, T* x, T* r, T* p, T* z, int steps,
                      const Ctl& ctl, const GridLink& link) {
   const int K = cg_row_entries(A);
-  // one block, whose exchanges stay in LDS, while its threads hold the rows
-  const int64_t solo = (int64_t)kCgBlock * (K * cg_entry_regs<T> * 4 <= 160 ? 4 : 3);
-  const int rows = A.nrows <= solo ? (int)((A.nrows + kCgBlock - 1) / kCgBlock)
-                                   : cg_rows_per_thread<T>(A.nrows, K);
+  const int rows = cg_one_block<T>(A) ? (int)((A.nrows + kCgBlock - 1) / kCgBlock)
+                                      : cg_rows_per_thread<T>(A.nrows, K, link.blocks);
   const CsrView<T> m = A.view<T>();
   auto run = [&](auto kk, auto rr) {
     constexpr int KK = decltype(kk)::value, RR = decltype(rr)::value;

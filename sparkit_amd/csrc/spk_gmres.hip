@@ -37,7 +37,7 @@ struct GmState {
   int32_t collect;
   int32_t j_final;
   int32_t flexible;
-  int32_t expired;    // a grid exchange's bounded wait ended without its value
+  int32_t expired;    // an exchange between blocks did not go through
   double* history;
   double* H;  // (m+1) x m, column-major, leading dimension m+1
   double* cs;
@@ -126,9 +126,8 @@ constexpr int kMgsSolo = 16 * kMgsBlock;
 // 262,144 (more blocks: more slots for every block to read).
 constexpr int kMgsGrain = 4 * kMgsBlock;
 
-inline int mgs_blocks() { return std::min(kLinkBlocks, ctx().num_cus); }
-inline bool mgs_fits(int64_t n, int64_t m) {
-  return m <= kMgsMaxCols && n <= (int64_t)mgs_blocks() * kMgsBlock * kMgsMaxElems;
+inline bool mgs_fits(int64_t n, int64_t m, const GridLink& link) {
+  return m <= kMgsMaxCols && n <= (int64_t)link.blocks * kMgsBlock * kMgsMaxElems;
 }
 
 // One modified Gram-Schmidt step in one launch (gmres.hpp:258-280): w =
@@ -154,6 +153,7 @@ __global__ __launch_bounds__(kMgsBlock + 64) void mgs_step_kernel(
   __shared__ double red[link_lds(kMgsBlock)];
   __shared__ double hc[kMgsMaxCols + 1], cs[kMgsMaxCols], sn[kMgsMaxCols];
   if (st->stop) return;  // written only after every block has been here
+  const int stale = link_open<kMgsBlock>(link);
   unsigned tag = *link.tag;
   // the link's wavefront holds no elements
   const unsigned i0 =
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kMgsBlock + 64) void mgs_step_kernel(
       if (e < n) x[u] = dl[e] * x[u];
     }
   }
-  bool ok = true;
+  bool lost = false;
   for (int i = 0; i <= j; ++i) {
     if (i < j) {
       const T* vn = V + (size_t)(i + 1) * ldv;
@@ -190,7 +190,8 @@ __global__ __launch_bounds__(kMgsBlock + 64) void mgs_step_kernel(
     double s[1] = {0.0};
 #pragma unroll
     for (int u = 0; u < E; ++u) s[0] += (double)v[u] * (double)x[u];
-    ok = ok && link_sum<1, kMgsBlock>(link, ++tag, s, red);
+    lost = !link_sum<1, kMgsBlock>(link, stale, ++tag, s, red);
+    if (lost) break;
 #pragma unroll
     for (int u = 0; u < E; ++u) x[u] = (T)((double)x[u] - s[0] * (double)v[u]);
     if (threadIdx.x == 0) hc[i] = s[0];
@@ -200,7 +201,10 @@ __global__ __launch_bounds__(kMgsBlock + 64) void mgs_step_kernel(
   double s[1] = {0.0};
 #pragma unroll
   for (int u = 0; u < E; ++u) s[0] += (double)x[u] * (double)x[u];
-  ok = ok && link_sum<1, kMgsBlock>(link, ++tag, s, red);
+  if (lost || !link_sum<1, kMgsBlock>(link, stale, ++tag, s, red)) {
+    if (threadIdx.x == 0) st->expired = 1;
+    return;
+  }
   const double hn = sqrt(s[0]);
   // normalise V_{j+1} if h > 0 (gmres.hpp:276-280 divides, fgmres.hpp:283
   // multiplies by the reciprocal)
@@ -222,9 +226,8 @@ __global__ __launch_bounds__(kMgsBlock + 64) void mgs_step_kernel(
     }
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    if (gridDim.x > 1) *link.tag = tag;
-    if (ok) arnoldi_finish(st, j, hn, hc, cs, sn);
-    else st->stop = 1;  // the host reports it
+    link_close(link, tag);
+    arnoldi_finish(st, j, hn, hc, cs, sn);
   }
 }
 
@@ -235,7 +238,9 @@ template <typename T>
 void launch_mgs_step(int64_t n, const T* V, size_t ldv, const T* w0, const T* dl, T* w,
                      const T* dr, T* z, int j, GmState* st, const GridLink& link) {
   const int64_t share =
-      n <= kMgsSolo ? n : std::max<int64_t>(kMgsGrain, (n + mgs_blocks() - 1) / mgs_blocks());
+      n <= kMgsSolo ? n
+                    : std::max<int64_t>(link.blocks > 1 ? kMgsGrain : n,
+                                        (n + link.blocks - 1) / link.blocks);
   const int64_t e = (share + kMgsBlock - 1) / kMgsBlock;
   auto run = [&](auto size) {
     constexpr int E = decltype(size)::value;
@@ -398,9 +403,8 @@ void gmres_solve(bool flexible, spk_csr_s* A, spk_precond_s* ML,
                                              (size_t)vec_grid(n)));
   }
   // modified Gram-Schmidt with V_{j+1} in registers, one launch a step
-  const bool mgs_one = !cgs2 && mgs_fits(n, m);
-  GridLink link{};
-  if (mgs_one) link = grid_link();
+  const GridLink link = grid_link();
+  bool mgs_one = !cgs2 && mgs_fits(n, m, link);
   DevState<GmState> st(kWsGmres + 5);
   GmState h{};
   h.tol = cfg->tolerance;
@@ -435,6 +439,7 @@ void gmres_solve(bool flexible, spk_csr_s* A, spk_precond_s* ML,
   int64_t iters = 0;
   while (iters < cfg->max_iterations && !h.converged && !h.done) {
     TraceRange cycle_("gmres restart cycle");
+    const GmState before = h;
     // compute_initial_residual (gmres.hpp:211-241 / fgmres.hpp:206-224)
     if (is_identity(left)) {
       launch_spmv(*A, (const T*)x, EpiResidual<T>{b, V}, s);
@@ -569,19 +574,24 @@ void gmres_solve(bool flexible, spk_csr_s* A, spk_precond_s* ML,
     hipLaunchKernelGGL(back_substitute_kernel, dim3(1), dim3(256), 0, s, S);
     const T* Zc = Z;
     launch_map(n, [=] __device__(int64_t e) {
+      if (S->expired) return;
       const int nj = S->j_final + 1;
       double sum = 0.0;
       for (int k = 0; k < nj; ++k) sum += (double)Zc[(size_t)k * nn + e] * S->y[k];
       x[e] = (T)((double)x[e] + sum);
     }, done);
     // close the cycle: a converged cycle finishes the solve
-    const int* expired = link.expired;
     launch_map(1, [=] __device__(int64_t) {
       if (S->converged) S->done = 1;
-      if (expired) S->expired = *expired;
-    });
+    }, done);
     h = st.download();
-    if (h.expired) check_link(link);
+    if (h.expired) {  // the cycle again, by the kernels per vector
+      renew_link(link);
+      mgs_one = false;
+      h = before;
+      st.upload(h);
+      continue;
+    }
     iters = h.iters;
     if (monitor && !h.converged && !h.done && !(*monitor)(iters, h.resnorm))
       break;

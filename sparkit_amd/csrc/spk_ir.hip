@@ -53,7 +53,7 @@ struct RcgState {
   double bnorm, rnorm, rupd, rz, alpha, beta, tol, delta;
   int64_t iters, updates;
   int32_t hold, converged, pad;
-  int32_t expired;  // a grid exchange's bounded wait ended without its value
+  int32_t expired;  // an exchange between blocks did not go through
   // one-kernel hand-off: rz by step parity, and the step whose second
   // kernel ran (gates the third)
   double rzb[2];
@@ -70,12 +70,12 @@ struct RcgCtl {
     return rn <= st->delta * st->rupd || rn / st->bnorm < st->tol;
   }
   __device__ void record(int, double) const {}
-  __device__ void finish(int steps, double, double rz0, double rz, bool ended,
-                         bool) const {
+  __device__ void finish(int steps, double, double rz0, double rz, bool ended) const {
     st->iters += steps;
     st->rz = ended ? rz0 : rz;  // the update's beta divides by the last step's
     if (ended) st->hold = 1;
   }
+  __device__ void expire() const { st->expired = 1; }
 };
 constexpr int kRcgSteps = 4096;  // steps of one launch, at most
 
@@ -173,9 +173,9 @@ void cg_reliable(spk_csr_s* A, spk_precond_s* M, const spk_ir_config* cfg,
   const float* invd = jac ? M->inv_diag<float>() : nullptr;
   // the one-kernel hand-off (every block of the next kernel sums the
   // previous partials) when the partials are few
-  const bool steps_fit = (jac || ident) && cg_steps_fit<float>(*A);
-  const GridLink link = steps_fit ? grid_link() : GridLink{};
-  const bool handoff = !steps_fit && (jac || ident || spai) &&
+  const GridLink link = grid_link();
+  bool steps_fit = (jac || ident) && cg_steps_fit<float>(*A, link);
+  const bool handoff = (jac || ident || spai) &&
                        spmv_partials_count<float>(*A) <= kProMaxPartials &&
                        pro_grid(n) <= kProMaxPartials &&
                        (!spai || spmv_partials_count<float>(*M->M) <= kProMaxPartials);
@@ -364,6 +364,7 @@ void cg_reliable(spk_csr_s* A, spk_precond_s* M, const spk_ir_config* cfg,
   };
 
   restart(true);
+  RcgState updated = h;  // as of the last update
   int64_t k = 0;
   if (history) history[0] = rnorm / bnorm;
   // `issued` numbers the queued steps (parity and step stamps); the budget
@@ -380,10 +381,18 @@ void cg_reliable(spk_csr_s* A, spk_precond_s* M, const spk_ir_config* cfg,
           launch_cg_steps(*A, invd, xi, r32, p, z,
                           (int)std::min<int64_t>(cfg->max_inner - ran, kRcgSteps),
                           RcgCtl{S}, link);
-          const int* expired = link.expired;
-          launch_map(1, [=] __device__(int64_t) { S->expired = *expired; });
           h = st.download();
-          if (h.expired) check_link(link);
+          if (h.expired) {
+            // the steps since the update go: on from x, which it left, by the
+            // kernels per step
+            renew_link(link);
+            steps_fit = false;
+            h = updated;
+            h.rz = 1.0;
+            st.upload(h);
+            restart(true);
+            continue;
+          }
           ran = h.iters;
           if (h.hold) break;
           continue;
@@ -410,6 +419,7 @@ void cg_reliable(spk_csr_s* A, spk_precond_s* M, const spk_ir_config* cfg,
     ++k;
     if (history) history[k] = h.rnorm / h.bnorm;
     if (h.converged || k >= cfg->max_outer || h.iters >= cfg->max_inner) break;
+    updated = h;
     restart(false);
   }
   out->relres = h.rnorm / h.bnorm;

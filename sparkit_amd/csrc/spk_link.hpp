@@ -1,7 +1,7 @@
 // spk_link.hpp -- sums over a whole grid inside one kernel.
 //
-// A persistent kernel of at most kLinkBlocks blocks (one per CU, so all of
-// them are resident) adds numbers over its blocks without ending: every
+// A persistent kernel of at most GridLink::blocks blocks (one per CU, so that
+// all of them are resident) adds numbers over its blocks without ending: every
 // block publishes its sum in a slot of its own and reads everybody's.  A
 // kernel boundary plus a one-block finisher costs about 4.5 us on this
 // chip; one exchange costs about 2 us and leaves each block's data in its
@@ -17,6 +17,13 @@
 // block 0 at the end of a kernel), so the words of an earlier launch never
 // match.  All blocks add the slots in the same order: the totals are
 // bit-identical everywhere.
+//
+// Other work on the GPU can keep a block from starting for as long as it
+// likes.  A wait therefore gives up after GridLink::polls polls: its block
+// leaves the kernel with nothing written, the link is marked for renewal, and
+// so are the state of the solve and of every later kernel that finds the link
+// so.  The host then renews the link, goes back to the state before those
+// launches and takes the kernels that need no exchange.
 #pragma once
 
 #include "spk_internal.hpp"
@@ -29,20 +36,42 @@ constexpr int kLinkWidth = 2;  // sums per exchange, at most
 struct GridLink {
   unsigned long long* slots;  // [2][kLinkWidth][kLinkBlocks][2]
   unsigned* tag;              // the last tag used by an earlier launch
-  int* expired;               // set when a wait ended without its value
+  int* expired;               // set: to be renewed before its next use
+  int blocks;                 // of a launch, at most
+  unsigned polls;             // of a wait, at most
 };
 constexpr size_t kLinkSlotWords = (size_t)2 * kLinkWidth * kLinkBlocks * 2;
 constexpr size_t kLinkWords = kLinkSlotWords + 2;
 
-// The library's link; its device memory is made and cleared with the library.
+// The library's link (its device memory is made and cleared with the library)
+// for launches on the library stream.  On a stream that is masked to some of
+// the CUs it allows one block, which waits for nobody.
 GridLink grid_link();
-// Throws SPK_HIP_ERROR when an exchange's bounded wait has expired
-// (synchronises); the flag is cleared.
-void check_link(const GridLink& l);
+// Clears the slots, the tag and the flag, in stream order.
+void renew_link(const GridLink& l);
 
-// Ticks of the 100 MHz clock after which a wait gives up: other work on the
-// GPU may keep some of the blocks from starting for a while, not for ever.
-constexpr unsigned long long kLinkTimeout = 1000000000ull;  // 10 s
+// A poll is a round trip through memory, 0.5 us and more: 0.1 s or so, during
+// which a process that is swapped out polls nothing.  An exchange takes a few
+// polls, and giving up costs no more than that and the steps since.
+constexpr unsigned kLinkPolls = 1u << 17;
+// Beyond this tag the link is renewed, so that tags never come round to those
+// that unused slots still hold; a launch uses fewer than are left.
+constexpr unsigned kLinkLastTag = 0xF0000000u;
+
+// What link_sum has to know of the link's state at the start of the kernel; the
+// load is under way beside the data's (DATA threads hold data).
+template <int DATA>
+__device__ __forceinline__ int link_open(const GridLink& l) {
+  int e = 0;
+  if (threadIdx.x >= DATA && gridDim.x > 1) e = *l.expired;
+  return __builtin_amdgcn_readfirstlane(e);
+}
+// the end of a kernel whose exchanges all went through; one thread of block 0
+__device__ __forceinline__ void link_close(const GridLink& l, unsigned tag) {
+  if (gridDim.x == 1) return;
+  *l.tag = tag;
+  if (tag >= kLinkLastTag) *l.expired = 1;
+}
 
 __device__ __forceinline__ unsigned long long link_word(unsigned tag, unsigned half) {
   return ((unsigned long long)tag << 32) | half;
@@ -54,15 +83,16 @@ __device__ __forceinline__ unsigned long long link_word(unsigned tag, unsigned h
 // loads in flight would wait for all of them before it saw a slot.  The
 // link's wavefront adds nothing (its v is ignored).  red: link_lds(DATA)
 // doubles of LDS.  tag: the exchange's number, the same in every block and
-// one more than the last.  false: the wait expired (every later exchange of
-// the kernel is to be skipped).
+// one more than the last.  stale: link_open's answer.  false, in every thread:
+// the link is to be renewed or the wait expired, v holds nothing and the block
+// has to leave.
 constexpr int link_lds(int data) {
   return 2 * kLinkWidth * (data / 64) + kLinkWidth + 1;
 }
 
 template <int W, int DATA>
-__device__ __forceinline__ bool link_sum(const GridLink& l, unsigned tag, double (&v)[W],
-                                         double* red) {
+__device__ __forceinline__ bool link_sum(const GridLink& l, int stale, unsigned tag,
+                                         double (&v)[W], double* red) {
   constexpr int NW = DATA / 64, NS = kLinkBlocks / 64;
   static_assert(W <= kLinkWidth && NW <= 64, "slots");
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, G = gridDim.x;
@@ -94,15 +124,14 @@ __device__ __forceinline__ bool link_sum(const GridLink& l, unsigned tag, double
       const double t = wave_sum_dpp(lane < NW ? part[k * NW + lane] : 0.0);
       // lane 0 stores the low word, lane 1 the high one
       const unsigned half = (unsigned)(lane == 0 ? __double2loint(t) : __double2hiint(t));
-      if (lane < 2)
+      if (lane < 2 && !stale)
         __hip_atomic_store(set + ((size_t)k * kLinkBlocks + blockIdx.x) * 2 + lane,
                            link_word(tag, half), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
     }
     unsigned long long lo[W][NS], hi[W][NS];
     bool ok = true;
-    unsigned spins = 0;
-    unsigned long long began = 0;
+    unsigned polls = stale ? l.polls : 0;
     for (;;) {
       bool all = true;
 #pragma unroll
@@ -122,14 +151,10 @@ __device__ __forceinline__ bool link_sum(const GridLink& l, unsigned tag, double
 #pragma unroll
         for (int q = 0; q < NS; ++q)
           all = all && (unsigned)(lo[k][q] >> 32) == tag && (unsigned)(hi[k][q] >> 32) == tag;
-      if (__all(all)) break;
-      if ((++spins & 1023u) == 0) {
-        const unsigned long long now = wall_clock64();
-        if (began == 0) began = now;
-        else if (now - began > kLinkTimeout) {
-          ok = false;
-          break;
-        }
+      if (__all(all) && !stale) break;
+      if (++polls >= l.polls) {
+        ok = false;
+        break;
       }
     }
 #pragma unroll
@@ -150,7 +175,8 @@ __device__ __forceinline__ bool link_sum(const GridLink& l, unsigned tag, double
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < W; ++k) v[k] = tot[k];
-  return tot[kLinkWidth] == 0.0;
+  // one answer for the wavefront: its branches are scalar
+  return __builtin_amdgcn_readfirstlane(__double2hiint(tot[kLinkWidth])) == 0;
 }
 
 }  // namespace spk

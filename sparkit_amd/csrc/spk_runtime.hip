@@ -2,6 +2,7 @@
 // timers, the workspace pool and the reduction scratch.
 #include "spk_link.hpp"
 
+#include <algorithm>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -55,6 +56,22 @@ DevBuf<unsigned long long>* g_link = nullptr;
 __global__ void link_clear_kernel(unsigned long long* w, int n) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k < n) w[k] = 0;
+}
+
+unsigned g_link_polls = kLinkPolls;
+
+bool g_own_all_cus = true;  // of g_ctx.stream, which does not change
+
+// Whether a stream may use every CU: one made with a CU mask may not.
+bool stream_has_all_cus(hipStream_t s) {
+  uint32_t mask[64] = {};
+  if (hipExtStreamGetCUMask(s, 64, mask) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  int cus = 0;
+  for (uint32_t w : mask) cus += __builtin_popcount(w);
+  return cus >= g_ctx.num_cus;
 }
 
 // the link's words: slots, tag and flag
@@ -241,6 +258,7 @@ void init_device(int device) {
   SPK_HIP_TRY(hipEventCreate(&g_ev1));
   g_partials = new DevBuf<double>(1 << 16);
   g_ws.reset(new Workspace());
+  g_own_all_cus = stream_has_all_cus(g_ctx.stream);
   // made here, so that a solve which may not allocate has it too
   g_link = new DevBuf<unsigned long long>(kLinkWords);
   clear_link(g_link->p, g_ctx.stream);
@@ -332,21 +350,15 @@ double* reduce_partials(size_t count) {
 }
 
 GridLink grid_link() {
-  ctx();
-  unsigned long long* w = g_link->p;
-  return GridLink{w, (unsigned*)(w + kLinkSlotWords), (int*)(w + kLinkSlotWords + 1)};
+  unsigned long long* w = (ctx(), g_link->p);
+  return GridLink{w, (unsigned*)(w + kLinkSlotWords), (int*)(w + kLinkSlotWords + 1),
+                  (g_user_stream ? stream_has_all_cus(g_user_stream) : g_own_all_cus)
+                      ? std::min(kLinkBlocks, g_ctx.num_cus)
+                      : 1,
+                  g_link_polls};
 }
 
-void check_link(const GridLink& l) {
-  int h = 0;
-  SPK_HIP_TRY(hipMemcpyAsync(&h, l.expired, sizeof(int), hipMemcpyDeviceToHost, stream()));
-  SPK_HIP_TRY(hipStreamSynchronize(stream()));
-  if (!h) return;
-  clear_link(l.slots, stream());
-  SPK_HIP_TRY(hipStreamSynchronize(stream()));
-  SPK_REQUIRE(false, SPK_HIP_ERROR,
-              "grid exchange: a bounded wait expired (results invalid)");
-}
+void renew_link(const GridLink& l) { clear_link(l.slots, stream()); }
 
 }  // namespace spk
 
@@ -409,6 +421,10 @@ spk_status spk_device_info(int* num_cus, char* name, size_t name_len) {
       std::snprintf(name, name_len, "%s (%s)", prop.name, prop.gcnArchName);
     }
   });
+}
+
+spk_status spk_set_exchange_polls(uint32_t polls) {
+  return guarded([&] { g_link_polls = polls ? polls : kLinkPolls; });
 }
 
 spk_status spk_malloc(void** dptr, size_t bytes) {
