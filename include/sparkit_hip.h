@@ -69,6 +69,13 @@ spk_status spk_device_info(int* num_cus, char* name, size_t name_len);
  * (0: the default). */
 spk_status spk_set_exchange_polls(uint32_t polls);
 
+/* The ILU(0) construction and triangular sweeps that run in one launch wait
+ * for each other's rows.  A wait is given up when nothing of its launch has
+ * got on for this long, in ticks of 10 ns (0: the default, 10 s; 1: after 512
+ * polls, whatever has got on): a sweep then fails with SPK_HIP_ERROR, the
+ * construction goes on without waits.  For tests. */
+spk_status spk_set_sweep_wait(uint64_t ticks);
+
 /* Device memory from a pool of at most 2 GiB of freed blocks, given back by
  * spk_finalize and when an allocation would fail.  Freed memory is handed out
  * again only after all work on the device queued before the spk_free has

@@ -133,6 +133,7 @@ _SIGS = {
     "spk_synchronize": ([], None),
     "spk_device_info": ([C.POINTER(C.c_int), C.c_char_p, C.c_size_t], None),
     "spk_set_exchange_polls": ([C.c_uint32], None),
+    "spk_set_sweep_wait": ([C.c_uint64], None),
     "spk_malloc": ([C.POINTER(vp), C.c_size_t], None),
     "spk_free": ([vp], None),
     "spk_memcpy_htod": ([vp, vp, C.c_size_t], None),

@@ -252,19 +252,21 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
   w.alloc((size_t)nnz);
   dpos.alloc((size_t)n);
   sweep_error.alloc(kErrorWords);
-  ticket.alloc(10);  // two sweeps' tickets; counters of the construction
+  constexpr int kCount = 2 * kTriTicketWords;  // counters of the construction
+  ticket.alloc(kCount + 6);
   SPK_HIP_TRY(hipMemcpyAsync(rp.p, A.rp.p, (n + 1) * 4, hipMemcpyDeviceToDevice, s));
   if (nnz) SPK_HIP_TRY(hipMemcpyAsync(ci.p, A.ci.p, nnz * 4, hipMemcpyDeviceToDevice, s));
   DevBuf<double> ordered;  // the values, where the rows had to be sorted
   hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, s, sweep_error.p, kErrorWords);
   int h[5];
   for (bool sorted = false;;) {
-    hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, s, ticket.p, 10);
+    hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, s, ticket.p,
+                       kCount + 6);
     hipLaunchKernelGGL(ilu_rows_kernel, dim3(std::min(blocks_for(n), 1024u)), dim3(256), 0, s, n,
-                       (const int32_t*)rp.p, (const int32_t*)ci.p, dpos.p, ticket.p + 4,
-                       (unsigned long long*)(ticket.p + 6));
+                       (const int32_t*)rp.p, (const int32_t*)ci.p, dpos.p,
+                       ticket.p + kCount, (unsigned long long*)(ticket.p + kCount + 2));
     SPK_HIP_TRY(hipGetLastError());
-    SPK_HIP_TRY(hipMemcpyAsync(h, ticket.p + 4, sizeof(h), hipMemcpyDeviceToHost, s));
+    SPK_HIP_TRY(hipMemcpyAsync(h, ticket.p + kCount, sizeof(h), hipMemcpyDeviceToHost, s));
     SPK_HIP_TRY(hipStreamSynchronize(s));
     SPK_REQUIRE((h[0] & 1) == 0, SPK_INVALID_ARGUMENT, "ilu0: missing diagonal entry");
     SPK_REQUIRE((h[0] & 4) == 0, SPK_INVALID_ARGUMENT, "ilu0: repeated diagonal entry");
@@ -280,7 +282,7 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
   {
     DevBuf<int32_t> lvl;
     int count[2];
-    tri_levels(P, lvl, count);
+    find_levels(lvl, count);
     levels_l = lower.levels = count[0];
     levels_u = upper.levels = count[1];
     tri_layout(P, true, lvl.p, lower);
@@ -289,24 +291,54 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
   level_launch = wide_levels();
   per_level = n >= kMaxTileSweepRows;
   const double* in = ordered.p ? ordered.p : A.v64.p;
-  if (h[1] <= kTriFactorLen && (h[0] & 8) == 0) {
-    tri_factor(P, lower, in, w, modified, h[1], h[4], ticket.p, sweep_error.p);
-  } else {
-    // long rows, or a column twice: one launch per dependency level, a
-    // thread per row
-    SPK_HIP_TRY(hipMemcpyAsync(w.p, in, nnz * 8, hipMemcpyDeviceToDevice, s));
-    build_levels();
-    for (size_t l = 0; l + 1 < lvl_ptr_l.size(); ++l) {
-      const int cnt = lvl_ptr_l[l + 1] - lvl_ptr_l[l];
-      hipLaunchKernelGGL(ilu_factor_level_kernel, dim3(blocks_for(cnt)), dim3(256), 0, s,
-                         lvl_rows_l.p + lvl_ptr_l[l], cnt, rp.p, ci.p, dpos.p, w.p,
-                         modified ? 1 : 0);
-    }
-    SPK_HIP_TRY(hipGetLastError());
+  bool tiled = h[1] <= kTriFactorLen && (h[0] & 8) == 0;
+  for (;;) {
+    if (tiled)
+      tri_factor(P, lower, in, w, modified, h[1], h[4], ticket.p, sweep_error.p);
+    else  // long rows, or a column twice
+      factor_by_levels(in, modified);
+    tri_values(P, true, w.p, lower);
+    tri_values(P, false, w.p, upper);
+    if (!sweep_errors() || !tiled) break;
+    tiled = false;  // a wait expired: again, without waits
   }
-  tri_values(P, true, w.p, lower);
-  tri_values(P, false, w.p, upper);
-  check_sweeps();
+}
+
+// One launch per dependency level, a thread per row.
+void spk_precond_s::factor_by_levels(const double* in, bool modified) {
+  hipStream_t s = stream();
+  SPK_HIP_TRY(hipMemcpyAsync(w.p, in, nnz * 8, hipMemcpyDeviceToDevice, s));
+  build_levels();
+  for (size_t l = 0; l + 1 < lvl_ptr_l.size(); ++l) {
+    const int cnt = lvl_ptr_l[l + 1] - lvl_ptr_l[l];
+    hipLaunchKernelGGL(ilu_factor_level_kernel, dim3(blocks_for(cnt)), dim3(256), 0, s,
+                       lvl_rows_l.p + lvl_ptr_l[l], cnt, rp.p, ci.p, dpos.p, w.p,
+                       modified ? 1 : 0);
+  }
+  SPK_HIP_TRY(hipGetLastError());
+}
+
+// tri_levels, on the host where a wait of it expired
+void spk_precond_s::find_levels(DevBuf<int32_t>& lvl, int count[2]) {
+  if (tri_levels(pattern(), lvl, count)) return;
+  hipStream_t s = stream();
+  std::vector<int32_t> hrp((size_t)n + 1), hd((size_t)n), hc((size_t)nnz), l((size_t)(2 * n));
+  SPK_HIP_TRY(hipMemcpyAsync(hrp.data(), rp.p, (n + 1) * 4, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipMemcpyAsync(hd.data(), dpos.p, n * 4, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipMemcpyAsync(hc.data(), ci.p, nnz * 4, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipStreamSynchronize(s));
+  count[0] = count[1] = 0;
+  auto row = [&](int64_t i, int64_t p, int64_t pe, int32_t* out, int* most) {
+    int32_t v = 0;
+    for (; p < pe; ++p) v = std::max(v, out[hc[(size_t)p]] + 1);
+    out[i] = v;
+    *most = std::max(*most, v + 1);
+  };
+  for (int64_t i = 0; i < n; ++i) row(i, hrp[i], hd[i], l.data(), count);
+  for (int64_t i = n - 1; i >= 0; --i)
+    row(i, hd[i] + 1, hrp[i + 1], l.data() + n, count + 1);
+  SPK_HIP_TRY(hipMemcpyAsync(lvl.p, l.data(), 8 * n, hipMemcpyHostToDevice, s));
+  SPK_HIP_TRY(hipStreamSynchronize(s));
 }
 
 void spk_precond_s::sort_rows(const spk_csr_s& A, DevBuf<double>& values) {
@@ -364,8 +396,7 @@ void spk_precond_s::reset_sentinels() {
   SPK_HIP_TRY(hipGetLastError());
 }
 
-void spk_precond_s::check_sweeps() {
-  if (kind != kIlu) return;
+int spk_precond_s::sweep_errors() {
   // word 0: 1 = a forward, 2 = a backward sweep's bounded wait expired, 4 =
   // the factorization's;
   // words 1..kErrorWords-1 must stay zero (a guard against stray writes)
@@ -375,17 +406,21 @@ void spk_precond_s::check_sweeps() {
   SPK_HIP_TRY(hipStreamSynchronize(stream()));
   bool guard_ok = true;
   for (int k = 1; k < kErrorWords; ++k) guard_ok = guard_ok && h[k] == 0;
-  if (h[0] == 0 && guard_ok) return;
+  if (h[0] == 0 && guard_ok) return 0;
   SPK_HIP_TRY(hipMemsetAsync(sweep_error.p, 0, sizeof(h), stream()));
   SPK_HIP_TRY(hipStreamSynchronize(stream()));
   SPK_REQUIRE(guard_ok, SPK_HIP_ERROR,
               "ILU sweep status words overwritten (a stray device write)");
-  SPK_REQUIRE((h[0] & 4) == 0, SPK_HIP_ERROR,
-              "ilu0: bounded wait expired in the factorization");
-  SPK_REQUIRE(false, SPK_HIP_ERROR,
+  return h[0];
+}
+
+void spk_precond_s::check_sweeps() {
+  if (kind != kIlu) return;
+  const int e = sweep_errors();
+  SPK_REQUIRE(e == 0, SPK_HIP_ERROR,
               std::string("ILU triangular sweep: bounded wait expired in the ") +
-                  (h[0] & 1 ? "forward" : "") + (h[0] == 3 ? " and " : "") +
-                  (h[0] & 2 ? "backward" : "") + " sweep (results invalid)");
+                  (e & 1 ? "forward" : "") + (e == 3 ? " and " : "") +
+                  (e & 2 ? "backward" : "") + " sweep (results invalid)");
 }
 
 template <typename T, bool LOWER>
@@ -425,7 +460,7 @@ void spk_precond_s::backward(const T* b, T* x) {
   hipStream_t s = stream();
   hipLaunchKernelGGL((fill_sentinel_kernel<T>), dim3(blocks_for(n)), dim3(256), 0, s, x, n);
   SPK_HIP_TRY(hipGetLastError());
-  tri_sweep<T, false>(upper, (T*)b, x, false, (T*)nullptr, ticket.p + 2, sweep_error.p, s);
+  tri_sweep<T, false>(upper, (T*)b, x, false, (T*)nullptr, ticket.p + kTriTicketWords, sweep_error.p, s);
 }
 
 void spk_precond_s::build_factors() {
@@ -459,7 +494,7 @@ void spk_precond_s::build_levels() {
   hipStream_t s = stream();
   DevBuf<int32_t> lvl;
   int count[2];
-  tri_levels(pattern(), lvl, count);
+  find_levels(lvl, count);
   std::vector<int32_t> h((size_t)(2 * n));
   SPK_HIP_TRY(hipMemcpyAsync(h.data(), lvl.p, 8 * n, hipMemcpyDeviceToHost, s));
   SPK_HIP_TRY(hipStreamSynchronize(s));
@@ -660,7 +695,7 @@ void spk_precond_s::apply(const T* in, T* out) {
         break;
       }
       tri_sweep<T, true>(lower, (T*)in, y, false, out, ticket.p, sweep_error.p, stream());
-      tri_sweep<T, false>(upper, y, out, true, (T*)nullptr, ticket.p + 2, sweep_error.p,
+      tri_sweep<T, false>(upper, y, out, true, (T*)nullptr, ticket.p + kTriTicketWords, sweep_error.p,
                           stream());
       break;
     }

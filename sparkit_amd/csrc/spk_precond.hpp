@@ -50,6 +50,8 @@ struct spk_precond_s {
   spk::TriPattern pattern() const { return {n, rp.p, ci.p, dpos.p}; }
   bool wide_levels() const;
   void factor(const spk_csr_s& A, bool modified);
+  void factor_by_levels(const double* in, bool modified);
+  void find_levels(spk::DevBuf<int32_t>& lvl, int count[2]);
   void sort_rows(const spk_csr_s& A, spk::DevBuf<double>& values);
   // the L and U stores, the level lists
   void build_factors();
@@ -102,6 +104,8 @@ struct spk_precond_s {
   T* tmp();
   template <typename T, bool LOWER>
   void level_sweep(const T* b, T* x);
+  // the sweeps' and the factorization's status word, cleared (synchronises)
+  int sweep_errors();
   // throws if a triangular sweep reported an expired wait (synchronises)
   void check_sweeps();
   // refill the scratch vectors with the ready sentinel

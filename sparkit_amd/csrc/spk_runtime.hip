@@ -1,6 +1,7 @@
 // spk_runtime.hip -- device selection, the library stream, device memory,
 // timers, the workspace pool and the reduction scratch.
 #include "spk_link.hpp"
+#include "spk_tri.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -425,6 +426,10 @@ spk_status spk_device_info(int* num_cus, char* name, size_t name_len) {
 
 spk_status spk_set_exchange_polls(uint32_t polls) {
   return guarded([&] { g_link_polls = polls ? polls : kLinkPolls; });
+}
+
+spk_status spk_set_sweep_wait(uint64_t ticks) {
+  return guarded([&] { set_tri_wait(ticks); });
 }
 
 spk_status spk_malloc(void** dptr, size_t bytes) {

@@ -8,23 +8,41 @@
 namespace spk {
 namespace {
 
-constexpr unsigned long long kWaitTicks = 1000000000ull;  // 10 s of the 100 MHz clock
+// The block's ticket (ticket[0] counts those taken, ticket[1] the tiles done:
+// the last returns both to zero for the next launch) and the launch's beat
+// (ticket[2]), a number that changes while any tile gets on: a healthy chain
+// of dependencies may take longer than any limit on a single wait.
+static_assert(kTriTicketWords > 2, "ticket");
+__device__ __forceinline__ void beat(int* ticket) {
+  if ((threadIdx.x & 63) == 0)
+    (void)__hip_atomic_fetch_add(ticket + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
-// A bounded wait: false once it has lasted kWaitTicks (the clock is read
-// every 1024 polls).
+// A bounded wait, for a whole wavefront: false once the beat has stood still
+// for `ticks` of the 100 MHz clock (looked at every 256 polls).  A wait that
+// lasts sleeps between its polls, up to 3 us: polls by every waiting wavefront
+// keep the memory from those that work.
 struct Wait {
-  unsigned spins = 0;
-  unsigned long long began = 0;
-  __device__ bool again() {
-    if ((++spins & 1023u) != 0) return true;
+  unsigned polls = 0;
+  int seen = 0;
+  unsigned long long since = 0;
+  __device__ bool again(const int* ticket, unsigned long long ticks) {
+    ++polls;
+    for (unsigned k = polls >> 6 < 16u ? polls >> 6 : 16u; k > 0; --k)
+      __builtin_amdgcn_s_sleep(8);
+    if ((polls & 255u) != 0) return true;
+    const int b =
+        __hip_atomic_load(ticket + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned long long now = wall_clock64();
-    if (began == 0) began = now;
-    return now - began < kWaitTicks;
+    if (since == 0 || (b != seen && ticks > 1)) {
+      since = now;
+      seen = b;
+    }
+    return now - since < ticks;
   }
 };
-
-// The block's ticket (ticket[0] counts those taken, ticket[1] the tiles done:
-// the last returns both to zero for the next launch).
+constexpr unsigned long long kWaitTicks = 1000000000ull;  // 10 s
+unsigned long long g_wait_ticks = kWaitTicks;
 __device__ __forceinline__ int take_tile(int* ticket) {
   int t = 0;
   if ((threadIdx.x & 63) == 0)
@@ -32,6 +50,7 @@ __device__ __forceinline__ int take_tile(int* ticket) {
   return __builtin_amdgcn_readfirstlane(t);
 }
 __device__ __forceinline__ void tile_done(int* ticket, int tiles) {
+  beat(ticket);
   if ((threadIdx.x & 63) != 0) return;
   if (__hip_atomic_fetch_add(ticket + 1, 1, __ATOMIC_RELAXED,
                              __HIP_MEMORY_SCOPE_AGENT) == tiles - 1) {
@@ -58,11 +77,12 @@ constexpr int kLevelSleep = 16;
 constexpr int kLevelBlock = 256;
 constexpr int kLevelRows = kTileRows / kLevelBlock;
 __global__ __launch_bounds__(kLevelBlock) void tri_level_kernel(
-    TriPattern P, int tiles, int32_t* lvl, int* ticket, int* maxlvl, int* error) {
+    TriPattern P, int tiles, int32_t* lvl, int* ticket, int* maxlvl, int* error,
+    unsigned long long ticks) {
   __shared__ int32_t mine[kTileRows];
   __shared__ int shared_tile;
   const bool lower = blockIdx.x < (unsigned)tiles;
-  int* tk = ticket + (lower ? 0 : 2);
+  int* tk = ticket + (lower ? 0 : kTriTicketWords);
   int32_t* out = lvl + (lower ? 0 : P.n);
   if (threadIdx.x < 64) {
     const int t = take_tile(tk);
@@ -92,6 +112,7 @@ __global__ __launch_bounds__(kLevelBlock) void tri_level_kernel(
   for (int u = 0; u < kLevelRows; ++u)
     if (p[u] < pe[u]) c[u] = P.ci[p[u]];
   Wait w;
+  unsigned moves = 0;
   while (__any(left > 0)) {
     int l[kLevelRows];
 #pragma unroll
@@ -126,8 +147,13 @@ __global__ __launch_bounds__(kLevelBlock) void tri_level_kernel(
     bool moved = false;
 #pragma unroll
     for (int u = 0; u < kLevelRows; ++u) moved = moved || l[u] >= 0;
-    if (!__any(moved)) __builtin_amdgcn_s_sleep(kLevelSleep);
-    if (!w.again()) {
+    if (__any(moved)) {
+      w = Wait{};
+      if ((++moves & 255u) == 0) beat(tk);
+      continue;
+    }
+    __builtin_amdgcn_s_sleep(kLevelSleep);
+    if (!w.again(tk, ticks)) {
       if ((threadIdx.x & 63) == 0) atomicOr(error, 4);
       break;
     }
@@ -453,7 +479,7 @@ enum { kPlain = 0, kMark = 1, kReset = 2 };
 // tiles of 1,024 rows 0.47 and 1.29.
 template <typename T, bool LOWER, int MODE>
 __global__ __launch_bounds__(64 * kGroupTiles) void tri_sweep_kernel(
-    TriView<T> A, T* b, T* x, T* mark, int* ticket, int* error) {
+    TriView<T> A, T* b, T* x, T* mark, int* ticket, int* error, unsigned long long ticks) {
 #pragma clang fp contract(off)
   __shared__ T val[kGroupRows + 1];
   __shared__ int taken;
@@ -489,6 +515,7 @@ __global__ __launch_bounds__(64 * kGroupTiles) void tri_sweep_kernel(
     if (nth == 0 && f > 0) {
       hnow = hnext;
       hnext = headers(f + 64);
+      beat(ticket);
     }
     const int pos = __builtin_amdgcn_readlane(hnow.x, nth);
     g.rows = __builtin_amdgcn_readlane(hnow.y, nth);
@@ -531,7 +558,7 @@ __global__ __launch_bounds__(64 * kGroupTiles) void tri_sweep_kernel(
           if (!is_ready(xv[k])) xv[k] = q[k] < 0 ? raw_load(at(x, ~q[k])) : lds_load(val + q[k]);
           all = all && is_ready(xv[k]);
         }
-        if (!w.again()) {
+        if (!w.again(ticket, ticks)) {
           dead = true;
           if (lane == 0) atomicOr(error, LOWER ? 1 : 2);
         }
@@ -547,6 +574,7 @@ __global__ __launch_bounds__(64 * kGroupTiles) void tri_sweep_kernel(
     T s = solve(g.c, g.v, g.u, g.b);
     const int batches = g.batches < 0 ? -g.batches : g.batches;
     for (int j = 1; j < batches; ++j) {  // wider rows
+      if ((j & 255) == 0) beat(ticket);
       const int l = lane < g.rows ? lane : g.rows - 1;
       const unsigned e = g.group + (unsigned)(j * g.rows + l);
       const int4 c = A.cols[e];
@@ -608,7 +636,8 @@ __global__ __launch_bounds__(64 * kGroupTiles) void tri_sweep_kernel(
 __global__ __launch_bounds__(64) void tri_factor_kernel(TriPattern P, TriView<double> A,
                                                         double* w, double* pivot,
                                                         int max_len, int modified,
-                                                        int* ticket, int* error) {
+                                                        int* ticket, int* error,
+                                                        unsigned long long ticks) {
 #pragma clang fp contract(off)
   extern __shared__ double buf[];
   int* cbuf = (int*)(buf + max_len * 64);
@@ -616,6 +645,7 @@ __global__ __launch_bounds__(64) void tri_factor_kernel(TriPattern P, TriView<do
   const int s0 = A.first[tile], s1 = A.first[tile + 1];
   bool dead = false;
   for (int q = s0; q < s1; ++q) {
+    if ((q & 15) == 0) beat(ticket);
     const int4 h = A.steps[q];
     const bool in = lane < h.y;
     int i = 0, p0 = 0, len = 0, nl = 0;
@@ -640,7 +670,7 @@ __global__ __launch_bounds__(64) void tri_factor_kernel(TriPattern P, TriView<do
       for (;;) {
         if (!ok) ok = load_ready(pivot + k, &d);
         if (__all(ok)) break;
-        if (dead || !wt.again()) {
+        if (dead || !wt.again(ticket, ticks)) {
           if (!dead && lane == 0) atomicOr(error, 4);
           dead = true;
           break;
@@ -733,7 +763,7 @@ struct ProgramStage {
 __global__ __launch_bounds__(64) void tri_factor_short_kernel(
     int tiles, const int32_t* __restrict__ first, const int4* __restrict__ steps,
     const RowProgram* __restrict__ prog, const double* __restrict__ in, double* f,
-    int modified, int* ticket, int* error) {
+    int modified, int* ticket, int* error, unsigned long long ticks) {
 #pragma clang fp contract(off)
   // the row's entries; kShort: what updates of no entry write to
   __shared__ double buf[(kShort + 1) * 64];
@@ -753,6 +783,7 @@ __global__ __launch_bounds__(64) void tri_factor_short_kernel(
     if (nth == 0 && q > 0) {
       hnow = hnext;
       hnext = headers(q + 64);
+      beat(ticket);
     }
     const int pos = __builtin_amdgcn_readlane(hnow.x, nth);
     const int rows = __builtin_amdgcn_readlane(hnow.y, nth);
@@ -794,7 +825,7 @@ __global__ __launch_bounds__(64) void tri_factor_short_kernel(
         all = all && (u >= nl || ok);
       }
       if (__all(all)) break;
-      if (dead || !wt.again()) {
+      if (dead || !wt.again(ticket, ticks)) {
         if (!dead && lane == 0) atomicOr(error, 4);
         dead = true;
         break;
@@ -887,24 +918,27 @@ TriView<float> TriTiles::view<float>() {
   return {n, tiles, rows.p, first.p, steps.p, cols.p, v32.p, d32.p};
 }
 
-void tri_levels(const TriPattern& P, DevBuf<int32_t>& lvl, int levels[2]) {
+void set_tri_wait(unsigned long long ticks) { g_wait_ticks = ticks ? ticks : kWaitTicks; }
+
+bool tri_levels(const TriPattern& P, DevBuf<int32_t>& lvl, int levels[2]) {
   levels[0] = levels[1] = 0;
   lvl.alloc((size_t)(2 * P.n + (P.n ? 0 : 1)));
-  if (P.n == 0) return;
+  if (P.n == 0) return true;
   hipStream_t s = stream();
-  DevBuf<int> st(8);  // two tickets, two maxima, the error word
+  constexpr int kMax = 2 * kTriTicketWords;
+  DevBuf<int> st(kMax + 4);  // two tickets, two maxima, the error word
   fill_words(st, 0, s);
   fill_words(lvl, ~0ull, s);
   const int tiles = tile_count(P.n);
   hipLaunchKernelGGL(tri_level_kernel, dim3(2 * tiles), dim3(kLevelBlock), 0, s, P, tiles,
-                     lvl.p, st.p, st.p + 4, st.p + 6);
+                     lvl.p, st.p, st.p + kMax, st.p + kMax + 2, g_wait_ticks);
   SPK_HIP_TRY(hipGetLastError());
-  int h[8];
-  SPK_HIP_TRY(hipMemcpyAsync(h, st.p, sizeof(h), hipMemcpyDeviceToHost, s));
+  int h[3];
+  SPK_HIP_TRY(hipMemcpyAsync(h, st.p + kMax, sizeof(h), hipMemcpyDeviceToHost, s));
   SPK_HIP_TRY(hipStreamSynchronize(s));
-  SPK_REQUIRE(h[6] == 0, SPK_HIP_ERROR, "ilu0: dependency levels: bounded wait expired");
-  levels[0] = h[4];
-  levels[1] = h[5];
+  levels[0] = h[0];
+  levels[1] = h[1];
+  return h[2] == 0;
 }
 
 void tri_layout(const TriPattern& P, bool lower, const int32_t* lvl, TriTiles& T) {
@@ -957,7 +991,8 @@ void tri_factor(const TriPattern& P, const TriTiles& lower, const double* in, De
                        s, P, (const int32_t*)lower.rows.p, prog.p);
     hipLaunchKernelGGL(tri_factor_short_kernel, dim3(lower.tiles), dim3(64), 0, s,
                        lower.tiles, (const int32_t*)lower.first.p, (const int4*)lower.steps.p,
-                       (const RowProgram*)prog.p, in, f.p, modified ? 1 : 0, ticket, error);
+                       (const RowProgram*)prog.p, in, f.p, modified ? 1 : 0, ticket, error,
+                       g_wait_ticks);
     SPK_HIP_TRY(hipGetLastError());
     SPK_HIP_TRY(hipStreamSynchronize(s));  // the programs end here
     return;
@@ -969,7 +1004,7 @@ void tri_factor(const TriPattern& P, const TriTiles& lower, const double* in, De
                     nullptr, nullptr, nullptr};
   hipLaunchKernelGGL(tri_factor_kernel, dim3(lower.tiles), dim3(64),
                      (size_t)max_len * 64 * (sizeof(double) + sizeof(int)), s, P, v, f.p,
-                     pivot.p, max_len, modified ? 1 : 0, ticket, error);
+                     pivot.p, max_len, modified ? 1 : 0, ticket, error, g_wait_ticks);
   SPK_HIP_TRY(hipGetLastError());
   SPK_HIP_TRY(hipStreamSynchronize(s));  // the pivots end here
 }
@@ -981,13 +1016,13 @@ void tri_sweep(TriTiles& A, T* b, T* x, bool reset_b, T* mark, int* ticket, int*
   const dim3 grid((A.tiles + kGroupTiles - 1) / kGroupTiles), block(64 * kGroupTiles);
   if (reset_b)
     hipLaunchKernelGGL((tri_sweep_kernel<T, LOWER, kReset>), grid, block, 0, s,
-                       A.view<T>(), b, x, mark, ticket, error);
+                       A.view<T>(), b, x, mark, ticket, error, g_wait_ticks);
   else if (mark)
     hipLaunchKernelGGL((tri_sweep_kernel<T, LOWER, kMark>), grid, block, 0, s, A.view<T>(),
-                       b, x, mark, ticket, error);
+                       b, x, mark, ticket, error, g_wait_ticks);
   else
     hipLaunchKernelGGL((tri_sweep_kernel<T, LOWER, kPlain>), grid, block, 0, s,
-                       A.view<T>(), b, x, mark, ticket, error);
+                       A.view<T>(), b, x, mark, ticket, error, g_wait_ticks);
   SPK_HIP_TRY(hipGetLastError());
 }
 template void tri_sweep<double, true>(TriTiles&, double*, double*, bool, double*, int*, int*, hipStream_t);

@@ -14,7 +14,8 @@
 // (ascending rows below the diagonal, descending above it), so every
 // dependency lies in a block that is running or has ended; within a tile the
 // steps ascend by level, and a row waits only for rows of lower levels.  The
-// wait of an unfinished row of the lowest level therefore always ends.
+// wait of an unfinished row of the lowest level therefore always ends.  Waits
+// are bounded all the same, by the time in which no tile gets on.
 #pragma once
 
 #include "spk_csr.hpp"
@@ -68,9 +69,16 @@ struct TriPattern {
   const int32_t* dpos;
 };
 
+// How long a wait may see no tile of its launch get on, in ticks of the 100
+// MHz clock (0: the default, 10 s; 1: every wait that lasts is given up, tiles
+// that get on or not); for tests.
+void set_tri_wait(unsigned long long ticks);
+// Words of what is `ticket` below, zero before the first launch.
+constexpr int kTriTicketWords = 4;
 // Dependency levels of the rows of both triangles (lvl[0..n-1] below the
-// diagonal, lvl[n..2n-1] above), and the number of levels of each.
-void tri_levels(const TriPattern& P, DevBuf<int32_t>& lvl, int levels[2]);
+// diagonal, lvl[n..2n-1] above), and the number of levels of each; false if a
+// bounded wait expired.
+bool tri_levels(const TriPattern& P, DevBuf<int32_t>& lvl, int levels[2]);
 // Order and steps of one triangle from its levels (T.levels is set).
 void tri_layout(const TriPattern& P, bool lower, const int32_t* lvl, TriTiles& T);
 // Fills the values from w (one per entry of the pattern).
@@ -78,7 +86,8 @@ void tri_values(const TriPattern& P, bool lower, const double* w, TriTiles& T);
 // The IKJ factorization (ilu.hpp:72-115) of the values `in` into f (one per
 // entry of the pattern), rows in the lower triangle's tile order.  max_len:
 // the longest row, at most kTriFactorLen; max_side: the most entries a row
-// has on one side of its diagonal.  No column is repeated in a row.
+// has on one side of its diagonal.  No column is repeated in a row.  A wait
+// that expired leaves 4 in *error, and f without meaning.
 constexpr int kTriFactorLen = 32;
 void tri_factor(const TriPattern& P, const TriTiles& lower, const double* in,
                 DevBuf<double>& f, bool modified, int max_len, int max_side, int* ticket,

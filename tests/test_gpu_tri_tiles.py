@@ -133,3 +133,49 @@ def test_rows_in_another_order(O, spk):
     for a, b in zip(F.factors(), G.factors()):
         for p, q in zip(a, b):
             assert np.array_equal(p, q)
+
+
+@pytest.fixture
+def sweep_wait(spk):
+    from sparkit_amd import _lib
+
+    def limit(ticks):
+        _lib.call("spk_set_sweep_wait", ticks)
+    yield limit
+    limit(0)
+
+
+@pytest.mark.parametrize("offsets,n,ms", [((-1, 1), 20480, 2),
+                                          (tuple(range(-12, 0)) + tuple(range(1, 13)), 6200, 40)])
+def test_a_long_chain_is_no_stall(O, spk, sweep_wait, offsets, n, ms):
+    """Waits of the last tiles last several times the limit (a tile of 2,048
+    dependent rows takes 5 ms to factor, 135 ms with 25 entries a row, 0.6 to
+    sweep), in which the tiles before them get on."""
+    print("chain", n, "limit", ms, "ms", flush=True)
+    A = _banded(O, n, offsets)
+    sweep_wait(ms * 100000)
+    _check(O, spk, A)
+
+
+@pytest.mark.parametrize("modified", [False, True])
+def test_waits_that_are_given_up(O, spk, sweep_wait, modified):
+    """The construction is done again without waits; a sweep says so, and the
+    next one is right."""
+    print("given up", modified, flush=True)
+    A = _banded(O, 20480, (-1, 1))
+    Lr, Ur = O.ilu0(A, modified)
+    r = O.uniform_pm1(5, A.nrows)
+    rd, z = spk.DeviceVector.from_numpy(r), spk.DeviceVector.zeros(A.nrows)
+    Ad = spk.CsrMatrix.from_oracle(A)
+    sweep_wait(1)
+    F = (spk.milu0 if modified else spk.ilu0)(Ad)
+    with pytest.raises(spk.SpkError, match="bounded wait"):
+        F.apply(rd, z)
+    sweep_wait(0)
+    assert F.levels() == (A.nrows, A.nrows)
+    (lrp, lci, lv), (urp, uci, uv) = F.factors()
+    assert np.array_equal(lv, Lr.vals) and np.array_equal(uv, Ur.vals)
+    z_ref = O.backward_solve(Ur, O.forward_solve(Lr, r))
+    for _ in range(2):
+        F.apply(rd, z)
+        assert np.array_equal(z.numpy(), z_ref)
