@@ -290,12 +290,12 @@ spk_status spk_precond_create_jacobi(spk_csr A, spk_precond* out);
  * non-square matrix or a missing diagonal. */
 spk_status spk_precond_create_ilu0(spk_csr A, int modified, spk_precond* out);
 /* Schedule of the ILU(0) triangular sweeps (no reference counterpart; the
- * arithmetic, and so the result, is the same for all): SPK_ILU_AUTO (0, the
- * default) and SPK_ILU_SYNC_FREE (2) run one launch per sweep, in which rows
- * wait for their dependencies' published values; SPK_ILU_LEVELS (1) runs one
- * launch per dependency level.  Under AUTO get_schedule names the factors'
- * shape, not the launches: LEVELS for at least 65536 rows and at most 4096
- * levels, else SYNC_FREE. */
+ * arithmetic, and so the result, is the same for all): SPK_ILU_LEVELS (1) runs
+ * one launch per dependency level, SPK_ILU_SYNC_FREE (2) one launch per sweep,
+ * in which rows wait for their dependencies' published values; SPK_ILU_AUTO
+ * (0, the default) takes LEVELS where 65,536 and more rows have few levels,
+ * as a multicolour ordering does, else SYNC_FREE.  get_schedule says which of
+ * the two runs. */
 #define SPK_ILU_AUTO 0
 #define SPK_ILU_LEVELS 1
 #define SPK_ILU_SYNC_FREE 2

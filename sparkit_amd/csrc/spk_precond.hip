@@ -150,9 +150,80 @@ __global__ void clear_words_kernel(int* p, int n) {
 }
 
 constexpr int kErrorWords = 64;  // sweep status word + guard words
-// the reported schedule's thresholds (see spk_precond_s::level_launch)
+// Few levels: from 65,536 rows on one launch per level, below a window.
 constexpr int64_t kLevelLaunchRows = 65536;
 constexpr int64_t kLevelLaunchMaxLevels = 4096;
+
+// A triangular sweep of few, wide levels in one launch: one thread per row in
+// padded level order (a wavefront holds rows of one level, which do not wait
+// for each other).  A small persistent grid walks the order, W threads at a
+// time, so only a window of a few levels waits; a row's dependencies are polled
+// kSweepBatch at a time and consumed in storage order, multiply-adds not
+// contracted: bit-identical to the sequential reference
+// (triangular_solve.hpp:42-53, 82-96).  Workgroups are dispatched in order, so
+// the earliest unfinished wavefront always has its dependencies resident or
+// finished.  reset_b returns b[i] to the sentinel after reading it; mark[i] is
+// filled with it (the next sweep's output).
+constexpr unsigned kSpinLimit = 1u << 22;
+constexpr int kSweepBatch = 4;
+template <typename T, bool LOWER>
+__global__ __launch_bounds__(256) void window_sweep_kernel(
+    const int32_t* __restrict__ rows, int n, const int32_t* __restrict__ rp,
+    const int32_t* __restrict__ ci, const T* __restrict__ v, T* b, T* x, bool reset_b,
+    T* mark, int* error) {
+#pragma clang fp contract(off)
+  const int W = gridDim.x * blockDim.x;
+  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += W) {
+    const int i = rows[t];
+    if (i < 0) continue;  // level padding
+    const int p0 = rp[i], p1 = rp[i + 1];
+    const int q1 = LOWER ? p1 - 1 : p1;
+    const int pd = LOWER ? p1 - 1 : p0;
+    T s = b[i];
+    if (reset_b) b[i] = sentinel_value<T>();
+    if (mark) mark[i] = sentinel_value<T>();
+    int p = LOWER ? p0 : p0 + 1;
+    unsigned spins = 0;
+    while (p < q1) {
+      const int cnt = q1 - p < kSweepBatch ? q1 - p : kSweepBatch;
+      int c[kSweepBatch];
+      T xv[kSweepBatch];
+      bool ok[kSweepBatch];
+#pragma unroll
+      for (int k = 0; k < kSweepBatch; ++k) {
+        ok[k] = k >= cnt;
+        c[k] = k < cnt ? ci[p + k] : 0;
+      }
+      bool all = false;
+      while (!all) {
+        all = true;
+#pragma unroll
+        for (int k = 0; k < kSweepBatch; ++k) {
+          if (!ok[k]) ok[k] = load_ready(x + c[k], &xv[k]);
+          all = all && ok[k];
+        }
+        if (!all) {
+          if (++spins > kSpinLimit) {
+            atomicOr(error, LOWER ? 1 : 2);
+            break;
+          }
+          __builtin_amdgcn_s_sleep(2);  // back off: fewer polls in flight
+        }
+      }
+      if (!all) {  // expired wait: publish what there is (reported)
+        p = q1;
+        break;
+      }
+#pragma unroll
+      for (int k = 0; k < kSweepBatch; ++k)
+        if (k < cnt) s = s - v[p + k] * xv[k];
+      p += cnt;
+    }
+    store_ready(x + i, s / v[pd]);
+    // keep this row's publication ahead of the next row's waits
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  }
+}
 
 // One dependency level of a triangular sweep: every row of the level reads
 // only rows of earlier levels (final, previous launches), so plain loads
@@ -191,6 +262,18 @@ std::vector<int32_t> group_levels(const std::vector<int32_t>& lvl,
   rows_out.resize(lvl.size());
   for (size_t i = 0; i < lvl.size(); ++i) rows_out[fill[lvl[i]]++] = (int32_t)i;
   return ptr;
+}
+
+// rows grouped by level, each level padded with -1 to a multiple of 64
+std::vector<int32_t> pad_levels(const std::vector<int32_t>& rows,
+                                const std::vector<int32_t>& ptr) {
+  std::vector<int32_t> out;
+  out.reserve(rows.size() + 64 * (ptr.size() - 1));
+  for (size_t l = 0; l + 1 < ptr.size(); ++l) {
+    out.insert(out.end(), rows.begin() + ptr[l], rows.begin() + ptr[l + 1]);
+    out.resize((out.size() + 63) / 64 * 64, -1);
+  }
+  return out;
 }
 
 // an n x n store with the given row offsets, columns and values not set
@@ -236,8 +319,31 @@ const float* spk_precond_s::inv_diag32() {
   return inv_d32.p;
 }
 
-bool spk_precond_s::wide_levels() const {
-  return n >= kLevelLaunchRows && std::max(levels_l, levels_u) <= kLevelLaunchMaxLevels;
+// Where a tile's chain of steps (2,048 rows: 32 and more) is longer than the
+// levels: up to 4 levels anywhere; beyond, from three tiles to 2^20 rows, up
+// to 24 levels, 64 where they are launched one by one.  One application (both
+// triangles, FP64) in tiles / as below: two colours of a 5-point stencil 100^2
+// 0.077 / 0.030 ms, 1000^2 0.093 / 0.058; four of a 9-point one 100^2 0.146 /
+// 0.042, 700^2 0.239 / 0.078; stencils in random order 3,600 rows (12 levels)
+// 0.065 / 0.072, 62,500 0.217 / 0.088, 512,000 (20) 0.399 / 0.322, 4.1M (22)
+// 1.03 / 1.44; 27 points 8,000 (49) 0.45 / 0.92, 216,000 (54) 1.94 / 1.77.
+bool spk_precond_s::few_levels() const {
+  const int levels = std::max(levels_l, levels_u);
+  return levels <= 4 || (n > 2 * kTileRows && n <= (1 << 20) &&
+                         levels <= (n < kLevelLaunchRows ? 24 : 64));
+}
+
+void spk_precond_s::set_schedule(int schedule) {
+  const bool launch =
+      n >= kLevelLaunchRows && std::max(levels_l, levels_u) <= kLevelLaunchMaxLevels;
+  sweep = schedule == SPK_ILU_LEVELS ? kLevels
+          : !few_levels() && n < kMaxTileSweepRows ? kTiles
+          : schedule == SPK_ILU_SYNC_FREE || !launch ? kWindow
+                                                     : kLevels;
+  if (sweep == kTiles) return;
+  build_factors();
+  build_levels();
+  if (sweep == kWindow) build_windows();
 }
 
 // ilu0_impl (ilu.hpp:35-141): the pattern, both triangles' layouts and the
@@ -288,8 +394,6 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
     tri_layout(P, true, lvl.p, lower);
     tri_layout(P, false, lvl.p + n, upper);
   }
-  level_launch = wide_levels();
-  per_level = n >= kMaxTileSweepRows;
   const double* in = ordered.p ? ordered.p : A.v64.p;
   bool tiled = h[1] <= kTriFactorLen && (h[0] & 8) == 0;
   for (;;) {
@@ -302,6 +406,7 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
     if (!sweep_errors() || !tiled) break;
     tiled = false;  // a wait expired: again, without waits
   }
+  set_schedule(SPK_ILU_AUTO);
 }
 
 // One launch per dependency level, a thread per row.
@@ -426,8 +531,6 @@ void spk_precond_s::check_sweeps() {
 template <typename T, bool LOWER>
 void spk_precond_s::level_sweep(const T* b, T* x) {
   hipStream_t s = stream();
-  build_factors();
-  build_levels();
   CsrView<T> v = (LOWER ? L : U)->view<T>();
   const std::vector<int32_t>& ptr = LOWER ? lvl_ptr_l : lvl_ptr_u;
   const int32_t* rows = LOWER ? lvl_rows_l.p : lvl_rows_u.p;
@@ -439,28 +542,45 @@ void spk_precond_s::level_sweep(const T* b, T* x) {
   SPK_HIP_TRY(hipGetLastError());
 }
 
+template <typename T, bool LOWER>
+void spk_precond_s::one_launch(T* b, T* x, bool reset_b, T* mark) {
+  hipStream_t s = stream();
+  if (sweep == kTiles) {
+    tri_sweep<T, LOWER>(LOWER ? lower : upper, b, x, reset_b, mark,
+                        ticket.p + (LOWER ? 0 : kTriTicketWords), sweep_error.p, s);
+    return;
+  }
+  const CsrView<T> v = (LOWER ? L : U)->view<T>();
+  hipLaunchKernelGGL((window_sweep_kernel<T, LOWER>),
+                     dim3(LOWER ? sweep_grid_l : sweep_grid_u), dim3(256), 0, s,
+                     (const int32_t*)(LOWER ? sweep_rows_l : sweep_rows_u).p,
+                     (int)(LOWER ? sweep_len_l : sweep_len_u), v.rp, v.ci, v.v, b, x, reset_b,
+                     mark, sweep_error.p);
+  SPK_HIP_TRY(hipGetLastError());
+}
+
 template <typename T>
 void spk_precond_s::forward(const T* b, T* x) {
-  if (per_level) {
+  if (sweep == kLevels) {
     level_sweep<T, true>(b, x);
     return;
   }
-  hipStream_t s = stream();
-  hipLaunchKernelGGL((fill_sentinel_kernel<T>), dim3(blocks_for(n)), dim3(256), 0, s, x, n);
+  hipLaunchKernelGGL((fill_sentinel_kernel<T>), dim3(blocks_for(n)), dim3(256), 0, stream(),
+                     x, n);
   SPK_HIP_TRY(hipGetLastError());
-  tri_sweep<T, true>(lower, (T*)b, x, false, (T*)nullptr, ticket.p, sweep_error.p, s);
+  one_launch<T, true>((T*)b, x, false, nullptr);
 }
 
 template <typename T>
 void spk_precond_s::backward(const T* b, T* x) {
-  if (per_level) {
+  if (sweep == kLevels) {
     level_sweep<T, false>(b, x);
     return;
   }
-  hipStream_t s = stream();
-  hipLaunchKernelGGL((fill_sentinel_kernel<T>), dim3(blocks_for(n)), dim3(256), 0, s, x, n);
+  hipLaunchKernelGGL((fill_sentinel_kernel<T>), dim3(blocks_for(n)), dim3(256), 0, stream(),
+                     x, n);
   SPK_HIP_TRY(hipGetLastError());
-  tri_sweep<T, false>(upper, (T*)b, x, false, (T*)nullptr, ticket.p + kTriTicketWords, sweep_error.p, s);
+  one_launch<T, false>((T*)b, x, false, nullptr);
 }
 
 void spk_precond_s::build_factors() {
@@ -507,6 +627,34 @@ void spk_precond_s::build_levels() {
   SPK_HIP_TRY(hipStreamSynchronize(s));
   lvl_rows_l = std::move(l);
   lvl_rows_u = std::move(u);
+}
+
+// the padded orders, and grids of about four levels of threads
+void spk_precond_s::build_windows() {
+  if (sweep_rows_l.p) return;
+  hipStream_t s = stream();
+  auto pad = [&](const DevBuf<int32_t>& rows, const std::vector<int32_t>& ptr,
+                 DevBuf<int32_t>& out, int64_t* len, unsigned* grid) {
+    std::vector<int32_t> h((size_t)n);
+    SPK_HIP_TRY(hipMemcpyAsync(h.data(), rows.p, n * 4, hipMemcpyDeviceToHost, s));
+    SPK_HIP_TRY(hipStreamSynchronize(s));
+    const std::vector<int32_t> padded = pad_levels(h, ptr);
+    SPK_REQUIRE(padded.size() < (size_t)INT32_MAX, SPK_INVALID_ARGUMENT,
+                "too many rows for the sweep order");
+    DevBuf<int32_t> d(padded.size());
+    SPK_HIP_TRY(hipMemcpyAsync(d.p, padded.data(), padded.size() * 4, hipMemcpyHostToDevice,
+                               s));
+    SPK_HIP_TRY(hipStreamSynchronize(s));
+    *len = (int64_t)padded.size();
+    const int64_t levels = (int64_t)ptr.size() - 1;
+    const int64_t w = levels > 0 ? *len / levels : 64;
+    const int64_t cap = std::max<int64_t>(4, 4 * ctx().num_cus);
+    const int64_t g = std::max<int64_t>(4, std::min((4 * w + 255) / 256, cap));
+    *grid = (unsigned)std::min<int64_t>(g, blocks_for(std::max<int64_t>(*len, 1)));
+    out = std::move(d);
+  };
+  pad(lvl_rows_u, lvl_ptr_u, sweep_rows_u, &sweep_len_u, &sweep_grid_u);
+  pad(lvl_rows_l, lvl_ptr_l, sweep_rows_l, &sweep_len_l, &sweep_grid_l);
 }
 
 // strict part of one factor row: L drops its last entry (the unit
@@ -689,14 +837,13 @@ void spk_precond_s::apply(const T* in, T* out) {
         break;
       }
       T* y = tmp<T>();
-      if (per_level) {  // one launch per level, no waiting
+      if (sweep == kLevels) {  // no waiting
         level_sweep<T, true>(in, y);
         level_sweep<T, false>((const T*)y, out);
         break;
       }
-      tri_sweep<T, true>(lower, (T*)in, y, false, out, ticket.p, sweep_error.p, stream());
-      tri_sweep<T, false>(upper, y, out, true, (T*)nullptr, ticket.p + kTriTicketWords, sweep_error.p,
-                          stream());
+      one_launch<T, true>((T*)in, y, false, out);
+      one_launch<T, false>(y, out, true, nullptr);
       break;
     }
     case kSpmv:
@@ -851,11 +998,10 @@ spk_status spk_ilu0_set_schedule(spk_precond M, int schedule) {
     SPK_REQUIRE(schedule >= 0 && schedule <= 2, SPK_INVALID_ARGUMENT,
                 "bad schedule");
     SPK_HIP_TRY(hipStreamSynchronize(stream()));
-    M->per_level = schedule == 1 || M->n >= kMaxTileSweepRows;
-    M->level_launch = schedule == 0 ? M->wide_levels() : schedule == 1;
+    M->set_schedule(schedule);
     // the per-level schedule leaves ordinary values in the scratch vector;
-    // the sweeps in tiles need it filled with the ready sentinel
-    if (!M->per_level) M->reset_sentinels();
+    // the others need it filled with the ready sentinel
+    if (M->sweep != spk_precond_s::kLevels) M->reset_sentinels();
   });
 }
 
@@ -905,7 +1051,7 @@ spk_status spk_ilu0_get_schedule(spk_precond M, int* schedule) {
   return guarded([&] {
     SPK_REQUIRE(M && schedule && M->kind == spk_precond_s::kIlu,
                 SPK_INVALID_ARGUMENT, "not an ILU(0) preconditioner");
-    *schedule = M->level_launch ? 1 : 2;
+    *schedule = M->sweep == spk_precond_s::kLevels ? SPK_ILU_LEVELS : SPK_ILU_SYNC_FREE;
   });
 }
 

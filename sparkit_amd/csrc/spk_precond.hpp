@@ -5,13 +5,16 @@
 //   rp, ci, dpos, w: A's pattern (columns ascending), each row's diagonal
 //            position and the factored values (L below the diagonal, U from
 //            it on);
-//   lower, upper: the two triangles in the sweeps' tile layout (spk_tri.hpp).
-// Made when something asks for them:
+//   lower, upper: the two triangles in the sweeps' tile layout (spk_tri.hpp),
+//            unless the levels are few.
+// Made when something asks for them, or the sweeps need them:
 //   L store: strictly-lower entries + unit diagonal LAST in each row; U
 //            store: diagonal FIRST + upper entries (the reference's layout,
 //            ilu.hpp:123-141), int32 indices;
 //   lvl_rows_l / lvl_ptr_l, lvl_rows_u / lvl_ptr_u: the rows grouped by
-//            dependency level, for the per-level schedule.
+//            dependency level;
+//   sweep_rows_l, sweep_rows_u: the same orders with every level padded by -1
+//            entries to a multiple of the wavefront size.
 // The numeric factorization runs the reference's IKJ loop (ilu.hpp:72-115),
 // a row per lane, with contraction of multiply-adds disabled, so the factors
 // are bit-identical to the sequential reference.
@@ -41,14 +44,17 @@ struct spk_precond_s {
   spk::DevBuf<double> tmp64;  // between the sweeps; kept filled with the
   spk::DevBuf<float> tmp32;   // ready sentinel between applications
   spk::DevBuf<int> sweep_error;  // set if a sweep's bounded wait expired
-  // The schedule asked for: per-level launches only when the caller chose
-  // them; level_launch is the reported schedule, which under AUTO names the
-  // factors' shape (at least kLevelLaunchRows rows, at most
-  // kLevelLaunchMaxLevels levels) whatever runs.
-  bool per_level = false;
-  bool level_launch = false;
+  // How the sweeps run: in tiles; or, where the levels are few, a row per
+  // thread over a window of levels in one launch, or one launch per level.
+  enum Sweep { kTiles, kWindow, kLevels } sweep = kTiles;
+  spk::DevBuf<int32_t> sweep_rows_l, sweep_rows_u;
+  int64_t sweep_len_l = 0, sweep_len_u = 0;
+  unsigned sweep_grid_l = 1, sweep_grid_u = 1;  // persistent window grids
   spk::TriPattern pattern() const { return {n, rp.p, ci.p, dpos.p}; }
-  bool wide_levels() const;
+  bool few_levels() const;
+  // chooses for SPK_ILU_AUTO (0), _LEVELS (1) or _SYNC_FREE (2) and makes what
+  // the sweeps need
+  void set_schedule(int schedule);
   void factor(const spk_csr_s& A, bool modified);
   void factor_by_levels(const double* in, bool modified);
   void find_levels(spk::DevBuf<int32_t>& lvl, int count[2]);
@@ -56,6 +62,7 @@ struct spk_precond_s {
   // the L and U stores, the level lists
   void build_factors();
   void build_levels();
+  void build_windows();
   // Approximate apply (jac_sweeps > 0): each triangular solve is replaced
   // by jac_sweeps Jacobi iterations from the diagonal-scaled right-hand
   // side, y <- r - L_s y and z <- (y - U_s z) / d_U, with L_s, U_s the
@@ -104,6 +111,9 @@ struct spk_precond_s {
   T* tmp();
   template <typename T, bool LOWER>
   void level_sweep(const T* b, T* x);
+  // x = L^-1 b or U^-1 b in one launch; reset_b and mark as tri_sweep's
+  template <typename T, bool LOWER>
+  void one_launch(T* b, T* x, bool reset_b, T* mark);
   // the sweeps' and the factorization's status word, cleared (synchronises)
   int sweep_errors();
   // throws if a triangular sweep reported an expired wait (synchronises)

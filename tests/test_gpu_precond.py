@@ -151,9 +151,33 @@ def test_ilu0_schedules_bit_exact(O, spk, schedule):
 
 
 def test_ilu0_auto_schedule_picks_levels_for_wide_levels(O, spk):
-    A = spk.convdiff_3d(48, 48, 48, 1.0, 0.1, 0.05, 0.02)
-    F = spk.ilu0(A)
-    assert F.schedule == "levels"          # 110592 rows, 142 levels
+    """A launch per level where 65,536 rows and more have few levels (two
+    colours: 2); one launch, in tiles, for a natural ordering's 142."""
+    n = 270 * 250
+    i = np.arange(n).reshape(270, 250)
+    colour = np.argsort(np.indices(i.shape).sum(0).ravel() % 2, kind="stable")
+    at = np.empty(n, np.int64)
+    at[colour] = np.arange(n)
+    r, c = [at], [at]
+    for p, q in ((i[1:], i[:-1]), (i[:, 1:], i[:, :-1])):
+        r += [at[p.ravel()], at[q.ravel()]]
+        c += [at[q.ravel()], at[p.ravel()]]
+    r, c = np.concatenate(r), np.concatenate(c)
+    two = O.make_matrix(n, n, r, c, np.where(r == c, 5.0, -0.5 - (r + c) % 7 / 14.0))
+    for A, schedule, levels in ((two, "levels", 2),
+                                (O.convdiff_3d(48, 48, 48, 1.0, 0.1, 0.05, 0.02),
+                                 "sync-free", 142)):
+        F = spk.ilu0(spk.CsrMatrix.from_oracle(A))
+        assert F.levels() == (levels, levels) and F.schedule == schedule
+        L, U = O.ilu0(A)
+        x = O.uniform_pm1(1, A.nrows)
+        z = spk.DeviceVector.zeros(A.nrows)
+        F.apply(dv(spk, x), z)
+        assert np.array_equal(z.numpy(), O.backward_solve(U, O.forward_solve(L, x)))
+        F.schedule = schedule  # what it says, set by name, is what ran
+        F.apply(dv(spk, x), z)
+        assert F.schedule == schedule
+        assert np.array_equal(z.numpy(), O.backward_solve(U, O.forward_solve(L, x)))
     S = spk.ilu0(spk.CsrMatrix.from_oracle(O.tridiagonal_matrix(300, -1., 4., -1.)))
     assert S.schedule == "sync-free"
 

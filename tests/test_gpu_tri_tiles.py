@@ -179,3 +179,45 @@ def test_waits_that_are_given_up(O, spk, sweep_wait, modified):
     for _ in range(2):
         F.apply(rd, z)
         assert np.array_equal(z.numpy(), z_ref)
+
+
+def _grid(O, nx, ny, order, points):
+    """A 5- or 9-point stencil, its rows in the given order."""
+    i = np.arange(nx * ny).reshape(nx, ny)
+    x, y = np.indices(i.shape)
+    key = {"two colours": (x + y) % 2, "four colours": x % 2 * 2 + y % 2,
+           "random": np.random.default_rng(nx).permutation(i.size).reshape(i.shape)}[order]
+    at = np.empty(i.size, np.int64)
+    at[np.argsort(key.ravel(), kind="stable")] = np.arange(i.size)
+    r, c = [at], [at]
+    pairs = [(i[1:], i[:-1]), (i[:, 1:], i[:, :-1])]
+    if points == 9:
+        pairs += [(i[1:, 1:], i[:-1, :-1]), (i[1:, :-1], i[:-1, 1:])]
+    for p, q in pairs:
+        r += [at[p.ravel()], at[q.ravel()]]
+        c += [at[q.ravel()], at[p.ravel()]]
+    r, c = np.concatenate(r), np.concatenate(c)
+    return O.make_matrix(i.size, i.size, r, c,
+                         np.where(r == c, points + 0.0, -0.5 - (r + c) % 7 / 14.0))
+
+
+@pytest.mark.parametrize("order,points", [("two colours", 5), ("four colours", 9),
+                                          ("random", 5), ("random", 9)])
+@pytest.mark.parametrize("nx,ny", [(9, 7), (64, 64), (64, 65), (255, 257), (256, 256),
+                                   (300, 230)])
+def test_few_levels(O, spk, order, points, nx, ny):
+    """Around three tiles (4,096 rows) and 65,536 rows, where the sweeps
+    change from tiles to a window of levels to a launch per level."""
+    print("few levels", order, points, nx, ny, flush=True)
+    A = _grid(O, nx, ny, order, points)
+    _check(O, spk, A, modified=points == 9)
+    F = spk.ilu0(spk.CsrMatrix.from_oracle(A))
+    L, U = O.ilu0(A)
+    r = O.uniform_pm1(3, A.nrows)
+    rd, z = spk.DeviceVector.from_numpy(r), spk.DeviceVector.zeros(A.nrows)
+    z_ref = O.backward_solve(U, O.forward_solve(L, r))
+    for schedule in ("sync-free", "levels", "auto", "levels", "sync-free"):
+        F.schedule = schedule
+        for _ in range(2):
+            F.apply(rd, z)
+            assert np.array_equal(z.numpy(), z_ref)
