@@ -97,13 +97,14 @@ __global__ void ilu_split_kernel(TriPattern P, const double* __restrict__ w,
 // Each row's diagonal position (ilu.hpp:54-66); out[0] |= 1 a missing
 // diagonal, 2 columns that do not ascend, 4 a repeated diagonal, 8 another
 // repeated column; out[1] the longest row; out[4] the most entries on one
-// side of the diagonal; *lower: the strictly lower entries.
+// side of the diagonal; out[5] how far the farthest column is from its row;
+// *lower: the strictly lower entries.
 __global__ void ilu_rows_kernel(int64_t n, const int32_t* __restrict__ rp,
                                 const int32_t* __restrict__ ci, int32_t* __restrict__ dpos,
                                 int* out, unsigned long long* lower) {
   __shared__ unsigned long long red[256 / 64];
   unsigned long long below = 0;
-  int bad = 0, len = 0, side = 0;
+  int bad = 0, len = 0, side = 0, reach = 0;
   for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * 256) {
     const int p0 = rp[i], pe = rp[i + 1];
@@ -124,6 +125,11 @@ __global__ void ilu_rows_kernel(int64_t n, const int32_t* __restrict__ rp,
     }
     dpos[i] = d;
     below += (unsigned long long)(d - p0);
+    if (pe > p0) {  // ascending, or to be sorted
+      const int lo = (int)i - ci[p0], hi = ci[pe - 1] - (int)i;
+      reach = lo > reach ? lo : reach;
+      reach = hi > reach ? hi : reach;
+    }
     len = pe - p0 > len ? pe - p0 : len;
     side = d - p0 > side ? d - p0 : side;
     side = pe - d - 1 > side ? pe - d - 1 : side;
@@ -134,6 +140,8 @@ __global__ void ilu_rows_kernel(int64_t n, const int32_t* __restrict__ rp,
     len = other > len ? other : len;
     const int os = __shfl_xor(side, o, 64);
     side = os > side ? os : side;
+    const int far = __shfl_xor(reach, o, 64);
+    reach = far > reach ? far : reach;
     bad |= __shfl_xor(bad, o, 64);
   }
   if (threadIdx.x == 0) atomicAdd(lower, below);
@@ -141,6 +149,7 @@ __global__ void ilu_rows_kernel(int64_t n, const int32_t* __restrict__ rp,
     if (bad) atomicOr(out, bad);
     atomicMax(out + 1, len);
     atomicMax(out + 4, side);
+    atomicMax(out + 5, reach);
   }
 }
 
@@ -320,29 +329,42 @@ const float* spk_precond_s::inv_diag32() {
 }
 
 // Where a tile's chain of steps (2,048 rows: 32 and more) is longer than the
-// levels: up to 4 levels anywhere; beyond, from three tiles to 2^20 rows, up
-// to 24 levels, 64 where they are launched one by one.  One application (both
+// levels, and its rows wait for other tiles': up to 4 levels anywhere; beyond,
+// from three tiles to 2^20 rows, up to 32 levels (24 of long rows), 64 where
+// they are launched one by one; not where rows reach less far than a tile.  One
+// application (both
 // triangles, FP64) in tiles / as below: two colours of a 5-point stencil 100^2
 // 0.077 / 0.030 ms, 1000^2 0.093 / 0.058; four of a 9-point one 100^2 0.146 /
 // 0.042, 700^2 0.239 / 0.078; stencils in random order 3,600 rows (12 levels)
 // 0.065 / 0.072, 62,500 0.217 / 0.088, 512,000 (20) 0.399 / 0.322, 4.1M (22)
-// 1.03 / 1.44; 27 points 8,000 (49) 0.45 / 0.92, 216,000 (54) 1.94 / 1.77.
+// 1.03 / 1.44; 10 random entries a row, 30,000 rows (31) 0.48 / 0.34; up to 60,
+// 30,000 (26) 0.67 / 1.27;
+// 27 points 8,000 (49) 0.45 / 0.92, 216,000 (54) 1.94 / 1.77;
+// dense blocks of 30 rows, 150,000 (30, within the blocks) 0.29 / 0.72.
 bool spk_precond_s::few_levels() const {
   const int levels = std::max(levels_l, levels_u);
+  if (n <= kTileRows) return levels <= 4;
+  if (reach < kTileRows) return false;
   return levels <= 4 || (n > 2 * kTileRows && n <= (1 << 20) &&
-                         levels <= (n < kLevelLaunchRows ? 24 : 64));
+                         levels <= (n >= kLevelLaunchRows    ? 64
+                                    : max_len <= kTriFactorLen ? 32
+                                                               : 24));
 }
 
-void spk_precond_s::set_schedule(int schedule) {
+void spk_precond_s::choose_sweep(int schedule) {
   const bool launch =
       n >= kLevelLaunchRows && std::max(levels_l, levels_u) <= kLevelLaunchMaxLevels;
   sweep = schedule == SPK_ILU_LEVELS ? kLevels
           : !few_levels() && n < kMaxTileSweepRows ? kTiles
           : schedule == SPK_ILU_SYNC_FREE || !launch ? kWindow
                                                      : kLevels;
+}
+
+void spk_precond_s::set_schedule(int schedule, const int32_t* lvl) {
+  choose_sweep(schedule);
   if (sweep == kTiles) return;
   build_factors();
-  build_levels();
+  build_levels(lvl);
   if (sweep == kWindow) build_windows();
 }
 
@@ -364,7 +386,7 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
   if (nnz) SPK_HIP_TRY(hipMemcpyAsync(ci.p, A.ci.p, nnz * 4, hipMemcpyDeviceToDevice, s));
   DevBuf<double> ordered;  // the values, where the rows had to be sorted
   hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, s, sweep_error.p, kErrorWords);
-  int h[5];
+  int h[6];
   for (bool sorted = false;;) {
     hipLaunchKernelGGL(clear_words_kernel, dim3(1), dim3(256), 0, s, ticket.p,
                        kCount + 6);
@@ -384,36 +406,51 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
   std::memcpy(&below, h + 2, sizeof(below));
   nnz_l = (int64_t)below + n;
   nnz_u = nnz - (int64_t)below;
+  reach = h[5];
   const TriPattern P = pattern();
-  {
-    DevBuf<int32_t> lvl;
-    int count[2];
-    find_levels(lvl, count);
-    levels_l = lower.levels = count[0];
-    levels_u = upper.levels = count[1];
-    tri_layout(P, true, lvl.p, lower);
-    tri_layout(P, false, lvl.p + n, upper);
-  }
+  max_len = h[1];
+  // Long rows, or a column twice: the factorization by levels.  Their levels
+  // come from the host, and those of small factors with more than four entries
+  // on a side: a dependency takes the device a round trip, the host a few
+  // nanoseconds (a chain of 100,000 rows with two of 4,096 entries 80 / 1 ms,
+  // 27 points 20^3 1.84 / 0.4).
+  const bool long_rows = max_len > kTriFactorLen || (h[0] & 8) != 0;
+  DevBuf<int32_t> lvl;
+  int count[2];
+  find_levels(lvl, count, long_rows || (h[4] > kBatch && nnz <= (1 << 20)));
+  levels_l = count[0];
+  levels_u = count[1];
+  choose_sweep(SPK_ILU_AUTO);
+  const bool tiles = sweep == kTiles;
+  if (tiles) tri_layouts(P, lvl.p, lower, upper);
   const double* in = ordered.p ? ordered.p : A.v64.p;
-  bool tiled = h[1] <= kTriFactorLen && (h[0] & 8) == 0;
+  // A tile works on one step at a time, the launches on a whole level: rows of
+  // more than four entries on a side, a row's elimination being hundreds of
+  // loads one after the other, take the tiles where those have fewer steps by
+  // a third.  Set-up in tiles / by levels: 20 random entries a row, 20,000 rows
+  // (54 levels) 28.8 / 13.4 ms, 27 points 20^3 natural 15.3 / 13.2, 40^3
+  // natural 29 / 39, 64^3 natural 47 / 79.
+  bool tiled = tiles && !long_rows &&
+               (h[4] <= kBatch ||
+                2 * (int64_t)levels_l * lower.tiles > 3 * (int64_t)lower.nsteps);
   for (;;) {
     if (tiled)
       tri_factor(P, lower, in, w, modified, h[1], h[4], ticket.p, sweep_error.p);
-    else  // long rows, or a column twice
-      factor_by_levels(in, modified);
-    tri_values(P, true, w.p, lower);
-    tri_values(P, false, w.p, upper);
-    if (!sweep_errors() || !tiled) break;
+    else
+      factor_by_levels(in, modified, lvl.p);
+    if (tiles) tri_values(P, w.p, lower, upper);
+    if (!tiled || !sweep_errors()) break;
     tiled = false;  // a wait expired: again, without waits
   }
-  set_schedule(SPK_ILU_AUTO);
+  set_schedule(SPK_ILU_AUTO, lvl.p);
+  SPK_HIP_TRY(hipStreamSynchronize(s));
 }
 
 // One launch per dependency level, a thread per row.
-void spk_precond_s::factor_by_levels(const double* in, bool modified) {
+void spk_precond_s::factor_by_levels(const double* in, bool modified, const int32_t* lvl) {
   hipStream_t s = stream();
   SPK_HIP_TRY(hipMemcpyAsync(w.p, in, nnz * 8, hipMemcpyDeviceToDevice, s));
-  build_levels();
+  build_levels(lvl);
   for (size_t l = 0; l + 1 < lvl_ptr_l.size(); ++l) {
     const int cnt = lvl_ptr_l[l + 1] - lvl_ptr_l[l];
     hipLaunchKernelGGL(ilu_factor_level_kernel, dim3(blocks_for(cnt)), dim3(256), 0, s,
@@ -423,10 +460,11 @@ void spk_precond_s::factor_by_levels(const double* in, bool modified) {
   SPK_HIP_TRY(hipGetLastError());
 }
 
-// tri_levels, on the host where a wait of it expired
-void spk_precond_s::find_levels(DevBuf<int32_t>& lvl, int count[2]) {
-  if (tri_levels(pattern(), lvl, count)) return;
+// tri_levels, or the same on the host (also where a wait of it expired)
+void spk_precond_s::find_levels(DevBuf<int32_t>& lvl, int count[2], bool host) {
+  if (!host && tri_levels(pattern(), lvl, count)) return;
   hipStream_t s = stream();
+  lvl.reserve((size_t)(2 * n));
   std::vector<int32_t> hrp((size_t)n + 1), hd((size_t)n), hc((size_t)nnz), l((size_t)(2 * n));
   SPK_HIP_TRY(hipMemcpyAsync(hrp.data(), rp.p, (n + 1) * 4, hipMemcpyDeviceToHost, s));
   SPK_HIP_TRY(hipMemcpyAsync(hd.data(), dpos.p, n * 4, hipMemcpyDeviceToHost, s));
@@ -609,14 +647,17 @@ void spk_precond_s::build_factors() {
   SPK_HIP_TRY(hipGetLastError());
 }
 
-void spk_precond_s::build_levels() {
+void spk_precond_s::build_levels(const int32_t* lvl) {
   if (lvl_rows_l.p) return;
   hipStream_t s = stream();
-  DevBuf<int32_t> lvl;
-  int count[2];
-  find_levels(lvl, count);
+  DevBuf<int32_t> own;
+  if (!lvl) {
+    int count[2];
+    find_levels(own, count, false);
+    lvl = own.p;
+  }
   std::vector<int32_t> h((size_t)(2 * n));
-  SPK_HIP_TRY(hipMemcpyAsync(h.data(), lvl.p, 8 * n, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipMemcpyAsync(h.data(), lvl, 8 * n, hipMemcpyDeviceToHost, s));
   SPK_HIP_TRY(hipStreamSynchronize(s));
   std::vector<int32_t> rows_l, rows_u;
   lvl_ptr_l = group_levels({h.begin(), h.begin() + n}, rows_l);
@@ -625,36 +666,43 @@ void spk_precond_s::build_levels() {
   SPK_HIP_TRY(hipMemcpyAsync(l.p, rows_l.data(), n * 4, hipMemcpyHostToDevice, s));
   SPK_HIP_TRY(hipMemcpyAsync(u.p, rows_u.data(), n * 4, hipMemcpyHostToDevice, s));
   SPK_HIP_TRY(hipStreamSynchronize(s));
+  if (sweep == kWindow) {
+    pad_order(rows_u, lvl_ptr_u, sweep_rows_u, &sweep_len_u, &sweep_grid_u);
+    pad_order(rows_l, lvl_ptr_l, sweep_rows_l, &sweep_len_l, &sweep_grid_l);
+  }
   lvl_rows_l = std::move(l);
   lvl_rows_u = std::move(u);
 }
 
-// the padded orders, and grids of about four levels of threads
+// a padded order, and a grid of about four levels of threads
+void spk_precond_s::pad_order(const std::vector<int32_t>& rows,
+                              const std::vector<int32_t>& ptr, DevBuf<int32_t>& out,
+                              int64_t* len, unsigned* grid) {
+  hipStream_t s = stream();
+  const std::vector<int32_t> padded = pad_levels(rows, ptr);
+  SPK_REQUIRE(padded.size() < (size_t)INT32_MAX, SPK_INVALID_ARGUMENT,
+              "too many rows for the sweep order");
+  DevBuf<int32_t> d(padded.size());
+  SPK_HIP_TRY(hipMemcpyAsync(d.p, padded.data(), padded.size() * 4, hipMemcpyHostToDevice, s));
+  SPK_HIP_TRY(hipStreamSynchronize(s));
+  *len = (int64_t)padded.size();
+  const int64_t levels = (int64_t)ptr.size() - 1;
+  const int64_t w = levels > 0 ? *len / levels : 64;
+  const int64_t cap = std::max<int64_t>(4, 4 * ctx().num_cus);
+  const int64_t g = std::max<int64_t>(4, std::min((4 * w + 255) / 256, cap));
+  *grid = (unsigned)std::min<int64_t>(g, blocks_for(std::max<int64_t>(*len, 1)));
+  out = std::move(d);
+}
+
 void spk_precond_s::build_windows() {
   if (sweep_rows_l.p) return;
   hipStream_t s = stream();
-  auto pad = [&](const DevBuf<int32_t>& rows, const std::vector<int32_t>& ptr,
-                 DevBuf<int32_t>& out, int64_t* len, unsigned* grid) {
-    std::vector<int32_t> h((size_t)n);
-    SPK_HIP_TRY(hipMemcpyAsync(h.data(), rows.p, n * 4, hipMemcpyDeviceToHost, s));
-    SPK_HIP_TRY(hipStreamSynchronize(s));
-    const std::vector<int32_t> padded = pad_levels(h, ptr);
-    SPK_REQUIRE(padded.size() < (size_t)INT32_MAX, SPK_INVALID_ARGUMENT,
-                "too many rows for the sweep order");
-    DevBuf<int32_t> d(padded.size());
-    SPK_HIP_TRY(hipMemcpyAsync(d.p, padded.data(), padded.size() * 4, hipMemcpyHostToDevice,
-                               s));
-    SPK_HIP_TRY(hipStreamSynchronize(s));
-    *len = (int64_t)padded.size();
-    const int64_t levels = (int64_t)ptr.size() - 1;
-    const int64_t w = levels > 0 ? *len / levels : 64;
-    const int64_t cap = std::max<int64_t>(4, 4 * ctx().num_cus);
-    const int64_t g = std::max<int64_t>(4, std::min((4 * w + 255) / 256, cap));
-    *grid = (unsigned)std::min<int64_t>(g, blocks_for(std::max<int64_t>(*len, 1)));
-    out = std::move(d);
-  };
-  pad(lvl_rows_u, lvl_ptr_u, sweep_rows_u, &sweep_len_u, &sweep_grid_u);
-  pad(lvl_rows_l, lvl_ptr_l, sweep_rows_l, &sweep_len_l, &sweep_grid_l);
+  std::vector<int32_t> l((size_t)n), u((size_t)n);
+  SPK_HIP_TRY(hipMemcpyAsync(l.data(), lvl_rows_l.p, n * 4, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipMemcpyAsync(u.data(), lvl_rows_u.p, n * 4, hipMemcpyDeviceToHost, s));
+  SPK_HIP_TRY(hipStreamSynchronize(s));
+  pad_order(u, lvl_ptr_u, sweep_rows_u, &sweep_len_u, &sweep_grid_u);
+  pad_order(l, lvl_ptr_l, sweep_rows_l, &sweep_len_l, &sweep_grid_l);
 }
 
 // strict part of one factor row: L drops its last entry (the unit

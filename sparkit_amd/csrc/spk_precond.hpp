@@ -35,6 +35,8 @@ struct spk_precond_s {
   spk::DevBuf<double> w;
   int64_t nnz = 0, nnz_l = 0, nnz_u = 0;
   int levels_l = 0, levels_u = 0;
+  int max_len = 0;  // the longest row
+  int reach = 0;    // the farthest column's distance from its row
   spk::TriTiles lower, upper;
   spk::DevBuf<int> ticket;  // of the forward and of the backward sweep
   spk_csr_s* L = nullptr;
@@ -52,17 +54,21 @@ struct spk_precond_s {
   unsigned sweep_grid_l = 1, sweep_grid_u = 1;  // persistent window grids
   spk::TriPattern pattern() const { return {n, rp.p, ci.p, dpos.p}; }
   bool few_levels() const;
+  void choose_sweep(int schedule);
   // chooses for SPK_ILU_AUTO (0), _LEVELS (1) or _SYNC_FREE (2) and makes what
   // the sweeps need
-  void set_schedule(int schedule);
+  void set_schedule(int schedule, const int32_t* lvl = nullptr);
   void factor(const spk_csr_s& A, bool modified);
-  void factor_by_levels(const double* in, bool modified);
-  void find_levels(spk::DevBuf<int32_t>& lvl, int count[2]);
+  // lvl: both triangles' levels, where they are at hand (else null)
+  void factor_by_levels(const double* in, bool modified, const int32_t* lvl);
+  void find_levels(spk::DevBuf<int32_t>& lvl, int count[2], bool host);
   void sort_rows(const spk_csr_s& A, spk::DevBuf<double>& values);
   // the L and U stores, the level lists
   void build_factors();
-  void build_levels();
+  void build_levels(const int32_t* lvl = nullptr);
   void build_windows();
+  void pad_order(const std::vector<int32_t>& rows, const std::vector<int32_t>& ptr,
+                 spk::DevBuf<int32_t>& out, int64_t* len, unsigned* grid);
   // Approximate apply (jac_sweeps > 0): each triangular solve is replaced
   // by jac_sweeps Jacobi iterations from the diagonal-scaled right-hand
   // side, y <- r - L_s y and z <- (y - U_s z) / d_U, with L_s, U_s the

@@ -19,18 +19,23 @@ __device__ __forceinline__ void beat(int* ticket) {
 }
 
 // A bounded wait, for a whole wavefront: false once the beat has stood still
-// for `ticks` of the 100 MHz clock (looked at every 256 polls).  A wait that
-// lasts sleeps between its polls, up to 3 us: polls by every waiting wavefront
-// keep the memory from those that work.
+// for `ticks` of the 100 MHz clock (looked at every kLook polls).  With kSleep a
+// wait that lasts sleeps between its polls, up to 3 us: 20 addresses a lane of
+// every waiting wavefront keep the memory from those that work.  The sweeps
+// poll what is missing only, in LDS where they can, and do not sleep: a tile
+// of a narrow grid follows the one before it by 30 us (40 x 20,000 rows: 14.9
+// ms an application, 18.7 with the sleep and a look every 256 polls).
+template <unsigned kLook, bool kSleep>
 struct Wait {
   unsigned polls = 0;
   int seen = 0;
   unsigned long long since = 0;
   __device__ bool again(const int* ticket, unsigned long long ticks) {
     ++polls;
-    for (unsigned k = polls >> 6 < 16u ? polls >> 6 : 16u; k > 0; --k)
-      __builtin_amdgcn_s_sleep(8);
-    if ((polls & 255u) != 0) return true;
+    if (kSleep)
+      for (unsigned k = polls >> 6 < 16u ? polls >> 6 : 16u; k > 0; --k)
+        __builtin_amdgcn_s_sleep(8);
+    if ((polls & (kLook - 1)) != 0) return true;
     const int b =
         __hip_atomic_load(ticket + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned long long now = wall_clock64();
@@ -41,6 +46,8 @@ struct Wait {
     return now - since < ticks;
   }
 };
+using BuildWait = Wait<256, true>;
+using SweepWait = Wait<4096, false>;
 constexpr unsigned long long kWaitTicks = 1000000000ull;  // 10 s
 unsigned long long g_wait_ticks = kWaitTicks;
 __device__ __forceinline__ int take_tile(int* ticket) {
@@ -111,7 +118,7 @@ __global__ __launch_bounds__(kLevelBlock) void tri_level_kernel(
 #pragma unroll
   for (int u = 0; u < kLevelRows; ++u)
     if (p[u] < pe[u]) c[u] = P.ci[p[u]];
-  Wait w;
+  BuildWait w;
   unsigned moves = 0;
   while (__any(left > 0)) {
     int l[kLevelRows];
@@ -148,7 +155,7 @@ __global__ __launch_bounds__(kLevelBlock) void tri_level_kernel(
 #pragma unroll
     for (int u = 0; u < kLevelRows; ++u) moved = moved || l[u] >= 0;
     if (__any(moved)) {
-      w = Wait{};
+      w = BuildWait{};
       if ((++moves & 255u) == 0) beat(tk);
       continue;
     }
@@ -174,13 +181,28 @@ __device__ __forceinline__ int length_class(int len) {
   return len <= 4 ? 0 : 30 - __clz(len - 1);
 }
 
-// One block per tile: its rows sorted by (level, length, row), the steps'
-// {position, batches} and their number and groups.
-__global__ __launch_bounds__(256) void tri_order_kernel(
-    TriPattern P, bool lower, const int32_t* __restrict__ lvl, int32_t* __restrict__ order,
-    int2* __restrict__ step, int* __restrict__ nsteps, int* __restrict__ nent) {
+// What the construction of both triangles works on (0: lower, 1: upper).
+struct TriBuild {
+  int tiles;
+  const int32_t* lvl[2];
+  int32_t* rows[2];
+  int2* step[2];
+  int* first[2];  // [tiles + 1]
+  int* ent[2];    // [tiles + 1]
+  int4* steps[2];
+  int4* cols[2];
+};
+
+// One block per tile of either triangle (blocks [0, tiles): lower): its rows
+// sorted by (level, length, row), the steps' {position, batches} and their
+// number and groups.
+__global__ __launch_bounds__(256) void tri_order_kernel(TriPattern P, TriBuild B) {
   __shared__ unsigned long long key[kTileRows];
-  const int tile = blockIdx.x, base = tile * kTileRows;
+  const bool lower = blockIdx.x < (unsigned)B.tiles;
+  const int k2 = lower ? 0 : 1, tile = (int)blockIdx.x - k2 * B.tiles, base = tile * kTileRows;
+  const int32_t* lvl = B.lvl[k2];
+  int32_t* order = B.rows[k2];
+  int2* step = B.step[k2];
   const int rows = (int)(P.n - base < kTileRows ? P.n - base : kTileRows);
   for (int k = threadIdx.x; k < kTileRows; k += 256) {
     unsigned long long q = ~0ull;
@@ -252,15 +274,17 @@ __global__ __launch_bounds__(256) void tri_order_kernel(
   }
   for (int o = 32; o > 0; o >>= 1) ent += __shfl_xor(ent, o, 64);
   if (lane == 0) {
-    nsteps[tile] = count;
-    nent[tile] = ent;
+    B.first[k2][tile] = count;
+    B.ent[k2][tile] = ent;
   }
 }
 
-// exclusive sums of a[0..m-1] and b[0..m-1] in place, the totals in a[m],
-// b[m]; one block
-__global__ __launch_bounds__(1024) void tri_scan_kernel(int m, int* a, int* b) {
+// exclusive sums of each triangle's steps and groups in place, the totals
+// behind them and in total[4]; one block a triangle
+__global__ __launch_bounds__(1024) void tri_scan_kernel(TriBuild B, int* total) {
   __shared__ int sa[1024], sb[1024];
+  const int m = B.tiles;
+  int *a = B.first[blockIdx.x], *b = B.ent[blockIdx.x];
   int ca = 0, cb = 0;
   for (int g = 0; g < m; g += 1024) {
     const int k = g + (int)threadIdx.x;
@@ -285,17 +309,20 @@ __global__ __launch_bounds__(1024) void tri_scan_kernel(int m, int* a, int* b) {
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    a[m] = ca;
-    b[m] = cb;
+    a[m] = total[2 * blockIdx.x] = ca;
+    b[m] = total[2 * blockIdx.x + 1] = cb;
   }
 }
 
-// One block per tile: the step headers and the column codes.
-__global__ __launch_bounds__(256) void tri_fill_kernel(
-    TriPattern P, bool lower, const int32_t* __restrict__ order,
-    const int2* __restrict__ step, const int* __restrict__ first,
-    const int* __restrict__ ent, int4* __restrict__ steps, int4* __restrict__ cols) {
-  const int tile = blockIdx.x, base = tile * kTileRows;
+// One block per tile of either triangle: the step headers and the column
+// codes.
+__global__ __launch_bounds__(256) void tri_fill_kernel(TriPattern P, TriBuild B) {
+  const bool lower = blockIdx.x < (unsigned)B.tiles;
+  const int k2 = lower ? 0 : 1, tile = (int)blockIdx.x - k2 * B.tiles, base = tile * kTileRows;
+  const int32_t* order = B.rows[k2];
+  const int2* step = B.step[k2];
+  const int *first = B.first[k2], *ent = B.ent[k2];
+  int4 *steps = B.steps[k2], *cols = B.cols[k2];
   const int gbase = tile / kGroupTiles * kGroupRows;
   const int rows = (int)(P.n - base < kTileRows ? P.n - base : kTileRows);
   const int s0 = first[tile], count = first[tile + 1] - s0;
@@ -350,13 +377,23 @@ __global__ __launch_bounds__(256) void tri_fill_kernel(
   }
 }
 
-// One wavefront per step: the values in the layout's order.
-__global__ __launch_bounds__(256) void tri_value_kernel(
-    TriPattern P, bool lower, int nsteps, const int32_t* __restrict__ order,
-    const int4* __restrict__ steps, const double* __restrict__ w, double* __restrict__ v,
-    double* __restrict__ d) {
-  const int q = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (q >= nsteps) return;
+// One wavefront per step of either triangle: the values in the layout's order.
+struct TriValues {
+  int nsteps[2];
+  const int32_t* rows[2];
+  const int4* steps[2];
+  double* v[2];
+  double* d;
+};
+__global__ __launch_bounds__(256) void tri_value_kernel(TriPattern P, TriValues B,
+                                                        const double* __restrict__ w) {
+  const int at = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const bool lower = at < B.nsteps[0];
+  const int k2 = lower ? 0 : 1, q = at - k2 * B.nsteps[0];
+  if (q >= B.nsteps[k2]) return;
+  const int32_t* order = B.rows[k2];
+  const int4* steps = B.steps[k2];
+  double *v = B.v[k2], *d = B.d;
   const int4 h = steps[q];
   if (lane >= h.y) return;
   const int i = order[h.x + lane], dp = P.dpos[i];
@@ -550,7 +587,7 @@ __global__ __launch_bounds__(64 * kGroupTiles) void tri_sweep_kernel(
       all = all && is_ready(xv[k]);
     }
     if (!__all(all)) {
-      Wait w;
+      SweepWait w;
       while (!dead && !__all(all)) {
         all = true;
 #pragma unroll
@@ -666,7 +703,7 @@ __global__ __launch_bounds__(64) void tri_factor_kernel(TriPattern P, TriView<do
       const int z0 = has ? P.dpos[k] + 1 : 0, z1 = has ? P.rp[k + 1] : 0;
       double d = 1.0;
       bool ok = !has;
-      Wait wt;
+      BuildWait wt;
       for (;;) {
         if (!ok) ok = load_ready(pivot + k, &d);
         if (__all(ok)) break;
@@ -814,7 +851,7 @@ __global__ __launch_bounds__(64) void tri_factor_short_kernel(
     for (int e = 0; e < kShort; ++e) buf[e * 64 + lane] = g.v[e];
     load_values(ring[(decltype(slot)::value + 1) % 4]);
     load_program(ring[(decltype(slot)::value + 2) % 4], q + 2);
-    Wait wt;
+    BuildWait wt;
     for (;;) {
       bool all = true;
 #pragma unroll
@@ -926,7 +963,8 @@ bool tri_levels(const TriPattern& P, DevBuf<int32_t>& lvl, int levels[2]) {
   if (P.n == 0) return true;
   hipStream_t s = stream();
   constexpr int kMax = 2 * kTriTicketWords;
-  DevBuf<int> st(kMax + 4);  // two tickets, two maxima, the error word
+  // two tickets, two maxima, the error word
+  DevBuf<int> st(kMax + 4);
   fill_words(st, 0, s);
   fill_words(lvl, ~0ull, s);
   const int tiles = tile_count(P.n);
@@ -941,42 +979,63 @@ bool tri_levels(const TriPattern& P, DevBuf<int32_t>& lvl, int levels[2]) {
   return h[2] == 0;
 }
 
-void tri_layout(const TriPattern& P, bool lower, const int32_t* lvl, TriTiles& T) {
+void tri_layouts(const TriPattern& P, const int32_t* lvl, TriTiles& lower, TriTiles& upper) {
   hipStream_t s = stream();
-  T.n = P.n;
-  T.tiles = tile_count(P.n);
+  const size_t m = (size_t)tile_count(P.n);
+  TriTiles* T[2] = {&lower, &upper};
+  for (TriTiles* t : T) {
+    t->n = P.n;
+    t->tiles = (int)m;
+  }
   if (P.n == 0) return;
-  const size_t m = (size_t)T.tiles;
-  T.rows.alloc((size_t)P.n);
-  T.first.alloc(m + 1);
-  DevBuf<int> ent(m + 1);
-  DevBuf<int2> step((size_t)P.n);
-  hipLaunchKernelGGL(tri_order_kernel, dim3(T.tiles), dim3(256), 0, s, P, lower, lvl,
-                     T.rows.p, step.p, T.first.p, ent.p);
-  hipLaunchKernelGGL(tri_scan_kernel, dim3(1), dim3(1024), 0, s, T.tiles, T.first.p, ent.p);
+  DevBuf<int> ent(2 * (m + 1) + 4);  // and the totals
+  DevBuf<int2> step((size_t)(2 * P.n));
+  int* total = ent.p + 2 * (m + 1);
+  TriBuild B{};
+  B.tiles = (int)m;
+  for (int k = 0; k < 2; ++k) {
+    T[k]->rows.alloc((size_t)P.n);
+    T[k]->first.alloc(m + 1);
+    B.lvl[k] = lvl + k * P.n;
+    B.rows[k] = T[k]->rows.p;
+    B.step[k] = step.p + k * P.n;
+    B.first[k] = T[k]->first.p;
+    B.ent[k] = ent.p + k * (m + 1);
+  }
+  hipLaunchKernelGGL(tri_order_kernel, dim3(2 * (unsigned)m), dim3(256), 0, s, P, B);
+  hipLaunchKernelGGL(tri_scan_kernel, dim3(2), dim3(1024), 0, s, B, total);
   SPK_HIP_TRY(hipGetLastError());
-  int h[2];
-  SPK_HIP_TRY(hipMemcpyAsync(h, T.first.p + m, 4, hipMemcpyDeviceToHost, s));
-  SPK_HIP_TRY(hipMemcpyAsync(h + 1, ent.p + m, 4, hipMemcpyDeviceToHost, s));
+  int h[4];
+  SPK_HIP_TRY(hipMemcpyAsync(h, total, sizeof(h), hipMemcpyDeviceToHost, s));
   SPK_HIP_TRY(hipStreamSynchronize(s));
-  T.nsteps = h[0];
-  T.groups = (int64_t)(unsigned)h[1];
-  T.steps.alloc((size_t)T.nsteps);
-  T.cols.alloc((size_t)T.groups);
-  hipLaunchKernelGGL(tri_fill_kernel, dim3(T.tiles), dim3(256), 0, s, P, lower,
-                     (const int32_t*)T.rows.p, (const int2*)step.p, (const int*)T.first.p,
-                     (const int*)ent.p, T.steps.p, T.cols.p);
+  for (int k = 0; k < 2; ++k) {
+    T[k]->nsteps = h[2 * k];
+    T[k]->groups = (int64_t)(unsigned)h[2 * k + 1];
+    T[k]->steps.alloc((size_t)T[k]->nsteps);
+    T[k]->cols.alloc((size_t)T[k]->groups);
+    B.steps[k] = T[k]->steps.p;
+    B.cols[k] = T[k]->cols.p;
+  }
+  hipLaunchKernelGGL(tri_fill_kernel, dim3(2 * (unsigned)m), dim3(256), 0, s, P, B);
   SPK_HIP_TRY(hipGetLastError());
-  SPK_HIP_TRY(hipStreamSynchronize(s));  // the scratch ends here
 }
 
-void tri_values(const TriPattern& P, bool lower, const double* w, TriTiles& T) {
+void tri_values(const TriPattern& P, const double* w, TriTiles& lower, TriTiles& upper) {
   if (P.n == 0) return;
-  T.v64.alloc((size_t)T.groups * kBatch);
-  if (!lower) T.d64.alloc((size_t)P.n);
-  hipLaunchKernelGGL(tri_value_kernel, dim3((T.nsteps + 3) / 4), dim3(256), 0, stream(), P,
-                     lower, T.nsteps, (const int32_t*)T.rows.p, (const int4*)T.steps.p, w,
-                     T.v64.p, T.d64.p);
+  TriTiles* T[2] = {&lower, &upper};
+  TriValues B{};
+  if (!upper.d64.p) upper.d64.alloc((size_t)P.n);
+  for (int k = 0; k < 2; ++k) {
+    if (!T[k]->v64.p) T[k]->v64.alloc((size_t)T[k]->groups * kBatch);
+    B.nsteps[k] = T[k]->nsteps;
+    B.rows[k] = T[k]->rows.p;
+    B.steps[k] = T[k]->steps.p;
+    B.v[k] = T[k]->v64.p;
+  }
+  B.d = upper.d64.p;
+  const int64_t waves = (int64_t)lower.nsteps + upper.nsteps;
+  hipLaunchKernelGGL(tri_value_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
+                     stream(), P, B, w);
   SPK_HIP_TRY(hipGetLastError());
 }
 
@@ -994,7 +1053,6 @@ void tri_factor(const TriPattern& P, const TriTiles& lower, const double* in, De
                        (const RowProgram*)prog.p, in, f.p, modified ? 1 : 0, ticket, error,
                        g_wait_ticks);
     SPK_HIP_TRY(hipGetLastError());
-    SPK_HIP_TRY(hipStreamSynchronize(s));  // the programs end here
     return;
   }
   DevBuf<double> pivot((size_t)P.n);
@@ -1006,7 +1064,6 @@ void tri_factor(const TriPattern& P, const TriTiles& lower, const double* in, De
                      (size_t)max_len * 64 * (sizeof(double) + sizeof(int)), s, P, v, f.p,
                      pivot.p, max_len, modified ? 1 : 0, ticket, error, g_wait_ticks);
   SPK_HIP_TRY(hipGetLastError());
-  SPK_HIP_TRY(hipStreamSynchronize(s));  // the pivots end here
 }
 
 template <typename T, bool LOWER>

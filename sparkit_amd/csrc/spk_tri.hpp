@@ -50,7 +50,7 @@ struct TriView {
 // One triangle of a factor.
 struct TriTiles {
   int64_t n = 0, groups = 0;
-  int tiles = 0, nsteps = 0, levels = 0;
+  int tiles = 0, nsteps = 0;
   DevBuf<int32_t> rows, first;
   DevBuf<int4> steps, cols;
   DevBuf<double> v64, d64;
@@ -79,10 +79,12 @@ constexpr int kTriTicketWords = 4;
 // diagonal, lvl[n..2n-1] above), and the number of levels of each; false if a
 // bounded wait expired.
 bool tri_levels(const TriPattern& P, DevBuf<int32_t>& lvl, int levels[2]);
-// Order and steps of one triangle from its levels (T.levels is set).
-void tri_layout(const TriPattern& P, bool lower, const int32_t* lvl, TriTiles& T);
-// Fills the values from w (one per entry of the pattern).
-void tri_values(const TriPattern& P, bool lower, const double* w, TriTiles& T);
+// Order and steps of both triangles from their levels.  (What is freed here and
+// below while kernels that use it are queued is handed out again only after
+// them, see DevBuf.)
+void tri_layouts(const TriPattern& P, const int32_t* lvl, TriTiles& lower, TriTiles& upper);
+// Fills both triangles' values from w (one per entry of the pattern).
+void tri_values(const TriPattern& P, const double* w, TriTiles& lower, TriTiles& upper);
 // The IKJ factorization (ilu.hpp:72-115) of the values `in` into f (one per
 // entry of the pattern), rows in the lower triangle's tile order.  max_len:
 // the longest row, at most kTriFactorLen; max_side: the most entries a row
