@@ -71,9 +71,10 @@ spk_status spk_set_exchange_polls(uint32_t polls);
 
 /* The ILU(0) construction and triangular sweeps that run in one launch wait
  * for each other's rows.  A wait is given up when nothing of its launch has
- * got on for this long, in ticks of 10 ns (0: the default, 10 s; 1: after 512
- * polls, whatever has got on): a sweep then fails with SPK_HIP_ERROR, the
- * construction goes on without waits.  For tests. */
+ * got on for this long, in ticks of 10 ns (0: the default, 10 s for a sweep and
+ * 1 s for the construction; 1: once it lasts, whatever has got on): a sweep
+ * then fails with SPK_HIP_ERROR, the construction goes on without waits.  For
+ * tests. */
 spk_status spk_set_sweep_wait(uint64_t ticks);
 
 /* Device memory from a pool of at most 2 GiB of freed blocks, given back by
@@ -286,7 +287,12 @@ spk_status spk_convert(int64_t n, int dtype_src, const void* d_src,
 spk_status spk_precond_create_jacobi(spk_csr A, spk_precond* out);
 /* ilu0(A) / milu0(A) (ilu.hpp:35-168): factors on A's pattern, computed on
  * the device by IKJ rows in dependency order; L has its unit diagonal last,
- * U its diagonal first (ilu.hpp:123-141).  SPK_INVALID_ARGUMENT for a
+ * U its diagonal first (ilu.hpp:123-141).  Rows that list their columns in
+ * another order are factored, and downloaded, in ascending order (stable).
+ * Where a row repeats its diagonal entry the first one is the pivot and the
+ * others stay beside it in U: the factors, spk_ilu0_forward and the
+ * Jacobi-sweep apply are defined, the backward solve and so the exact apply
+ * are not (SPK_INVALID_ARGUMENT from those).  SPK_INVALID_ARGUMENT for a
  * non-square matrix or a missing diagonal. */
 spk_status spk_precond_create_ilu0(spk_csr A, int modified, spk_precond* out);
 /* Schedule of the ILU(0) triangular sweeps (no reference counterpart; the

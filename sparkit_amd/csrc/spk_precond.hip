@@ -354,7 +354,7 @@ bool spk_precond_s::few_levels() const {
 void spk_precond_s::choose_sweep(int schedule) {
   const bool launch =
       n >= kLevelLaunchRows && std::max(levels_l, levels_u) <= kLevelLaunchMaxLevels;
-  sweep = schedule == SPK_ILU_LEVELS ? kLevels
+  sweep = schedule == SPK_ILU_LEVELS || twice ? kLevels
           : !few_levels() && n < kMaxTileSweepRows ? kTiles
           : schedule == SPK_ILU_SYNC_FREE || !launch ? kWindow
                                                      : kLevels;
@@ -397,7 +397,6 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
     SPK_HIP_TRY(hipMemcpyAsync(h, ticket.p + kCount, sizeof(h), hipMemcpyDeviceToHost, s));
     SPK_HIP_TRY(hipStreamSynchronize(s));
     SPK_REQUIRE((h[0] & 1) == 0, SPK_INVALID_ARGUMENT, "ilu0: missing diagonal entry");
-    SPK_REQUIRE((h[0] & 4) == 0, SPK_INVALID_ARGUMENT, "ilu0: repeated diagonal entry");
     if ((h[0] & 2) == 0 || sorted) break;
     sort_rows(A, ordered);  // a caller's CSR rows in another order than ascending
     sorted = true;
@@ -409,12 +408,13 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
   reach = h[5];
   const TriPattern P = pattern();
   max_len = h[1];
+  twice = (h[0] & 4) != 0;
   // Long rows, or a column twice: the factorization by levels.  Their levels
   // come from the host, and those of small factors with more than four entries
   // on a side: a dependency takes the device a round trip, the host a few
   // nanoseconds (a chain of 100,000 rows with two of 4,096 entries 80 / 1 ms,
   // 27 points 20^3 1.84 / 0.4).
-  const bool long_rows = max_len > kTriFactorLen || (h[0] & 8) != 0;
+  const bool long_rows = max_len > kTriFactorLen || (h[0] & 12) != 0;
   DevBuf<int32_t> lvl;
   int count[2];
   find_levels(lvl, count, long_rows || (h[4] > kBatch && nnz <= (1 << 20)));
@@ -460,9 +460,10 @@ void spk_precond_s::factor_by_levels(const double* in, bool modified, const int3
   SPK_HIP_TRY(hipGetLastError());
 }
 
-// tri_levels, or the same on the host (also where a wait of it expired)
+// tri_levels, or the same on the host (also where a wait of it expired, or where
+// a row would wait for itself)
 void spk_precond_s::find_levels(DevBuf<int32_t>& lvl, int count[2], bool host) {
-  if (!host && tri_levels(pattern(), lvl, count)) return;
+  if (!host && !twice && tri_levels(pattern(), lvl, count)) return;
   hipStream_t s = stream();
   lvl.reserve((size_t)(2 * n));
   std::vector<int32_t> hrp((size_t)n + 1), hd((size_t)n), hc((size_t)nnz), l((size_t)(2 * n));
@@ -473,7 +474,8 @@ void spk_precond_s::find_levels(DevBuf<int32_t>& lvl, int count[2], bool host) {
   count[0] = count[1] = 0;
   auto row = [&](int64_t i, int64_t p, int64_t pe, int32_t* out, int* most) {
     int32_t v = 0;
-    for (; p < pe; ++p) v = std::max(v, out[hc[(size_t)p]] + 1);
+    for (; p < pe; ++p)
+      if (hc[(size_t)p] != i) v = std::max(v, out[hc[(size_t)p]] + 1);
     out[i] = v;
     *most = std::max(*most, v + 1);
   };
@@ -609,8 +611,15 @@ void spk_precond_s::forward(const T* b, T* x) {
   one_launch<T, true>((T*)b, x, false, nullptr);
 }
 
+void spk_precond_s::require_backward() const {
+  SPK_REQUIRE(!twice, SPK_INVALID_ARGUMENT,
+              "ilu0: a row repeats its diagonal entry, its backward solve would read its "
+              "own result");
+}
+
 template <typename T>
 void spk_precond_s::backward(const T* b, T* x) {
+  require_backward();
   if (sweep == kLevels) {
     level_sweep<T, false>(b, x);
     return;
@@ -884,6 +893,7 @@ void spk_precond_s::apply(const T* in, T* out) {
         jacobi_apply(in, out);
         break;
       }
+      require_backward();
       T* y = tmp<T>();
       if (sweep == kLevels) {  // no waiting
         level_sweep<T, true>(in, y);

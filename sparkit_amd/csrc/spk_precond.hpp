@@ -35,6 +35,7 @@ struct spk_precond_s {
   spk::DevBuf<double> w;
   int64_t nnz = 0, nnz_l = 0, nnz_u = 0;
   int levels_l = 0, levels_u = 0;
+  bool twice = false;  // some row has its diagonal twice: the first one counts
   int max_len = 0;  // the longest row
   int reach = 0;    // the farthest column's distance from its row
   spk::TriTiles lower, upper;
@@ -117,6 +118,8 @@ struct spk_precond_s {
   T* tmp();
   template <typename T, bool LOWER>
   void level_sweep(const T* b, T* x);
+  // throws where a backward solve has no meaning
+  void require_backward() const;
   // x = L^-1 b or U^-1 b in one launch; reset_b and mark as tri_sweep's
   template <typename T, bool LOWER>
   void one_launch(T* b, T* x, bool reset_b, T* mark);

@@ -49,7 +49,11 @@ struct Wait {
 using BuildWait = Wait<256, true>;
 using SweepWait = Wait<4096, false>;
 constexpr unsigned long long kWaitTicks = 1000000000ull;  // 10 s
-unsigned long long g_wait_ticks = kWaitTicks;
+constexpr unsigned long long kBuildTicks = 100000000ull;  // the construction: 1 s,
+                                                          // it goes on without waits
+unsigned long long g_wait_ticks = 0;  // 0: these
+unsigned long long sweep_ticks() { return g_wait_ticks ? g_wait_ticks : kWaitTicks; }
+unsigned long long build_ticks() { return g_wait_ticks ? g_wait_ticks : kBuildTicks; }
 __device__ __forceinline__ int take_tile(int* ticket) {
   int t = 0;
   if ((threadIdx.x & 63) == 0)
@@ -955,7 +959,7 @@ TriView<float> TriTiles::view<float>() {
   return {n, tiles, rows.p, first.p, steps.p, cols.p, v32.p, d32.p};
 }
 
-void set_tri_wait(unsigned long long ticks) { g_wait_ticks = ticks ? ticks : kWaitTicks; }
+void set_tri_wait(unsigned long long ticks) { g_wait_ticks = ticks; }
 
 bool tri_levels(const TriPattern& P, DevBuf<int32_t>& lvl, int levels[2]) {
   levels[0] = levels[1] = 0;
@@ -969,7 +973,7 @@ bool tri_levels(const TriPattern& P, DevBuf<int32_t>& lvl, int levels[2]) {
   fill_words(lvl, ~0ull, s);
   const int tiles = tile_count(P.n);
   hipLaunchKernelGGL(tri_level_kernel, dim3(2 * tiles), dim3(kLevelBlock), 0, s, P, tiles,
-                     lvl.p, st.p, st.p + kMax, st.p + kMax + 2, g_wait_ticks);
+                     lvl.p, st.p, st.p + kMax, st.p + kMax + 2, build_ticks());
   SPK_HIP_TRY(hipGetLastError());
   int h[3];
   SPK_HIP_TRY(hipMemcpyAsync(h, st.p + kMax, sizeof(h), hipMemcpyDeviceToHost, s));
@@ -1051,7 +1055,7 @@ void tri_factor(const TriPattern& P, const TriTiles& lower, const double* in, De
     hipLaunchKernelGGL(tri_factor_short_kernel, dim3(lower.tiles), dim3(64), 0, s,
                        lower.tiles, (const int32_t*)lower.first.p, (const int4*)lower.steps.p,
                        (const RowProgram*)prog.p, in, f.p, modified ? 1 : 0, ticket, error,
-                       g_wait_ticks);
+                       build_ticks());
     SPK_HIP_TRY(hipGetLastError());
     return;
   }
@@ -1062,7 +1066,7 @@ void tri_factor(const TriPattern& P, const TriTiles& lower, const double* in, De
                     nullptr, nullptr, nullptr};
   hipLaunchKernelGGL(tri_factor_kernel, dim3(lower.tiles), dim3(64),
                      (size_t)max_len * 64 * (sizeof(double) + sizeof(int)), s, P, v, f.p,
-                     pivot.p, max_len, modified ? 1 : 0, ticket, error, g_wait_ticks);
+                     pivot.p, max_len, modified ? 1 : 0, ticket, error, build_ticks());
   SPK_HIP_TRY(hipGetLastError());
 }
 
@@ -1073,13 +1077,13 @@ void tri_sweep(TriTiles& A, T* b, T* x, bool reset_b, T* mark, int* ticket, int*
   const dim3 grid((A.tiles + kGroupTiles - 1) / kGroupTiles), block(64 * kGroupTiles);
   if (reset_b)
     hipLaunchKernelGGL((tri_sweep_kernel<T, LOWER, kReset>), grid, block, 0, s,
-                       A.view<T>(), b, x, mark, ticket, error, g_wait_ticks);
+                       A.view<T>(), b, x, mark, ticket, error, sweep_ticks());
   else if (mark)
     hipLaunchKernelGGL((tri_sweep_kernel<T, LOWER, kMark>), grid, block, 0, s, A.view<T>(),
-                       b, x, mark, ticket, error, g_wait_ticks);
+                       b, x, mark, ticket, error, sweep_ticks());
   else
     hipLaunchKernelGGL((tri_sweep_kernel<T, LOWER, kPlain>), grid, block, 0, s,
-                       A.view<T>(), b, x, mark, ticket, error, g_wait_ticks);
+                       A.view<T>(), b, x, mark, ticket, error, sweep_ticks());
   SPK_HIP_TRY(hipGetLastError());
 }
 template void tri_sweep<double, true>(TriTiles&, double*, double*, bool, double*, int*, int*, hipStream_t);

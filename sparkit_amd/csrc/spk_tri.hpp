@@ -70,7 +70,7 @@ struct TriPattern {
 };
 
 // How long a wait may see no tile of its launch get on, in ticks of the 100
-// MHz clock (0: the default, 10 s; 1: every wait that lasts is given up, tiles
+// MHz clock (0: the default, 10 s, of the construction 1 s; 1: every wait that lasts is given up, tiles
 // that get on or not); for tests.
 void set_tri_wait(unsigned long long ticks);
 // Words of what is `ticket` below, zero before the first launch.

@@ -221,3 +221,75 @@ def test_few_levels(O, spk, order, points, nx, ny):
         for _ in range(2):
             F.apply(rd, z)
             assert np.array_equal(z.numpy(), z_ref)
+
+
+def _ikj(rp, ci, v, modified):
+    """ilu0 of rows that may repeat columns: the first diagonal is the pivot."""
+    n, w = len(rp) - 1, np.array(v)
+    dp = [rp[i] + list(ci[rp[i]:rp[i + 1]]).index(i) for i in range(n)]
+    for i in range(n):
+        dropped = 0.0
+        for p in range(rp[i], rp[i + 1]):
+            k = ci[p]
+            if k >= i:
+                break
+            w[p] = w[p] / w[dp[k]]
+            pi = p + 1
+            for q in range(dp[k] + 1, rp[k + 1]):
+                while pi < rp[i + 1] and ci[pi] < ci[q]:
+                    pi += 1
+                if pi < rp[i + 1] and ci[pi] == ci[q]:
+                    w[pi] = w[pi] - w[p] * w[q]
+                elif modified:
+                    dropped = dropped + w[p] * w[q]
+        if modified:
+            w[dp[i]] = w[dp[i]] - dropped
+    return w, dp
+
+
+@pytest.mark.parametrize("modified", [False, True])
+def test_repeated_diagonal(O, spk, modified):
+    """Rows 5, 50 and 300 have their diagonal twice: factors, forward sweep
+    and Jacobi sweeps as ever; the backward solve is refused, on every
+    schedule, and at once."""
+    A = _banded(O, 400, (-20, -1, 1, 20))
+    twice = [5, 50, 300]
+    rp, ci, v = [0], [], []
+    for i in range(A.nrows):
+        s = slice(A.row_ptr[i], A.row_ptr[i + 1])
+        for c, x in zip(A.col_ind[s], A.vals[s]):
+            ci += [c, c] if c == i and i in twice else [c]
+            v += [x, 0.25] if c == i and i in twice else [x]
+        rp.append(len(ci))
+    rp, ci, v = np.array(rp), np.array(ci), np.array(v)
+    F = (spk.milu0 if modified else spk.ilu0)(
+        spk.CsrMatrix.from_host(A.nrows, A.nrows, rp, ci, v))
+    w, dp = _ikj(rp, ci, v, modified)
+    (lrp, lci, lv), (urp, uci, uv) = F.factors()
+    for i in range(A.nrows):
+        assert np.array_equal(lv[lrp[i]:lrp[i + 1] - 1], w[rp[i]:dp[i]])
+        assert np.array_equal(uv[urp[i]:urp[i + 1]], w[dp[i]:rp[i + 1]])
+        assert np.array_equal(uci[urp[i]:urp[i + 1]], ci[dp[i]:rp[i + 1]])
+    r = O.uniform_pm1(3, A.nrows)
+    rd, y = spk.DeviceVector.from_numpy(r), spk.DeviceVector.zeros(A.nrows)
+    for schedule in ("auto", "sync-free", "levels"):
+        F.schedule = schedule
+        F.forward(rd, y)
+        x = np.array(r)
+        for i in range(A.nrows):
+            for p in range(lrp[i], lrp[i + 1] - 1):
+                x[i] = x[i] - lv[p] * x[lci[p]]
+        assert np.array_equal(y.numpy(), x)
+        for call in (F.apply, F.backward):
+            with pytest.raises(spk.InvalidArgument, match="diagonal"):
+                call(rd, y)
+    F.jacobi_sweeps = 1
+    F.apply(rd, y)
+    d = uv[urp[:-1]]
+    low, up = np.array(r), np.zeros(A.nrows)
+    for i in range(A.nrows):
+        low[i] -= lv[lrp[i]:lrp[i + 1] - 1] @ r[lci[lrp[i]:lrp[i + 1] - 1]]
+    for i in range(A.nrows):
+        p = slice(urp[i] + 1, urp[i + 1])
+        up[i] = (low[i] - uv[p] @ (low / d)[uci[p]]) / d[i]
+    assert np.allclose(y.numpy(), up, rtol=1e-13, atol=1e-14)
