@@ -97,7 +97,11 @@ class Pool {
   hipError_t get(void** p, size_t bytes) {
     const size_t size = rounded(bytes);
     std::lock_guard<std::mutex> lk(m_);
-    if (!open()) return hipMalloc(p, bytes);
+    if (!open()) {
+      const hipError_t e = hipMalloc(p, bytes);
+      if (e == hipSuccess) owned_.erase(*p);
+      return e;
+    }
     Size& c = sizes_[size];
     c.used = ++uses_;
     if (c.ready.empty() && c.idle.size() >= idle_limit(size)) {
@@ -135,7 +139,7 @@ class Pool {
     if (it == owned_.end()) return kForeign;
     if (it->second.kept) return kFreed;
     const size_t size = it->second.size;
-    if (!open()) {
+    if (!open() || !still_ours(p, size)) {
       owned_.erase(it);
       return kForeign;
     }
@@ -194,6 +198,17 @@ class Pool {
       return false;
     }
     return dev == g_ctx.device && st == hipStreamCaptureStatusNone;
+  }
+  // A caller may have given a block of the pool back by hipFree; its address is
+  // then whatever was allocated there since.
+  static bool still_ours(void* p, size_t size) {
+    hipDeviceptr_t base = nullptr;
+    size_t bytes = 0;
+    if (hipMemGetAddressRange(&base, &bytes, (hipDeviceptr_t)p) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    return base == (hipDeviceptr_t)p && bytes == size;
   }
   void drop(void* p) {
     owned_.erase(p);

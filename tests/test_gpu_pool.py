@@ -126,3 +126,34 @@ def test_a_second_free_is_refused(spk):
             _lib.call("spk_free", p)
         vs = [spk.DeviceVector(nbytes // 8) for _ in range(40)]
         assert len({v.ptr.value for v in vs}) == 40
+
+
+@pytest.mark.parametrize("nbytes", [4096, 1 << 20])
+def test_a_block_given_back_by_hipfree(spk, nbytes):
+    """spk_malloc's memory given to hipFree, its address taken by a smaller
+    hipMalloc, and that given to spk_free: it goes to hipFree, and no vector
+    of the old size gets it."""
+    import ctypes as C
+
+    from sparkit_amd import _lib
+    hip = C.CDLL("libamdhip64.so")
+    p, q = C.c_void_p(), C.c_void_p()
+    held, met = [], False
+    for _ in range(60):  # until hipMalloc returns an address of the pool's
+        _lib.call("spk_malloc", C.byref(p), nbytes)
+        assert hip.hipFree(p) == 0
+        assert hip.hipMalloc(C.byref(q), C.c_size_t(nbytes // 4)) == 0
+        if q.value == p.value:
+            met = True
+            break
+        held.append(q.value)
+    for h in held:
+        assert hip.hipFree(C.c_void_p(h)) == 0
+    print("address met again:", met, flush=True)
+    if met:
+        _lib.call("spk_free", q)
+        vs = [spk.DeviceVector.from_numpy(np.full(nbytes // 8, float(k))) for k in range(40)]
+        for k, v in enumerate(vs):
+            assert (v.numpy() == k).all()
+        spans = sorted((v.ptr.value, v.ptr.value + nbytes) for v in vs)
+        assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
