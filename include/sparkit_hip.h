@@ -78,12 +78,16 @@ spk_status spk_set_exchange_polls(uint32_t polls);
 spk_status spk_set_sweep_wait(uint64_t ticks);
 
 /* Device memory from a pool of at most 2 GiB of freed blocks, given back by
- * spk_finalize and when an allocation would fail.  Freed memory is handed out
+ * spk_release_memory, by spk_finalize and when an allocation of the library's
+ * would fail; another allocator of the process that runs short has to have
+ * spk_release_memory called.  The first allocations of a size cost what
+ * hipMalloc does, later ones less.  Freed memory is handed out
  * again only after all work on the device queued before the spk_free has
  * ended, on any stream; spk_free itself does not wait.  spk_free also takes
  * memory from hipMalloc (and then waits as hipFree does). */
 spk_status spk_malloc(void** dptr, size_t bytes);
 spk_status spk_free(void* dptr);
+spk_status spk_release_memory(void);
 spk_status spk_memcpy_htod(void* dst, const void* src, size_t bytes);
 spk_status spk_memcpy_dtoh(void* dst, const void* src, size_t bytes);
 spk_status spk_memcpy_dtod(void* dst, const void* src, size_t bytes);

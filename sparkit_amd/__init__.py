@@ -34,7 +34,7 @@ from ._lib import (F32, F64, BREAKDOWN, ORTHO_CGS1, ORTHO_CGS2, ORTHO_MGS,
                    LogicError, ReadError, SpkError, call, load)
 
 __all__ = [
-    "init", "synchronize", "DeviceVector", "CsrMatrix", "Preconditioner",
+    "init", "synchronize", "release_memory", "DeviceVector", "CsrMatrix", "Preconditioner",
     "identity", "jacobi", "ilu0", "milu0", "spai", "multiply",
     "extract_diagonal", "jacobi_apply", "ilu_apply", "CGConfig",
     "GmresConfig", "FgmresConfig", "BicgstabConfig", "Summary",
@@ -65,6 +65,12 @@ def init(device: int = 0):
 
 def synchronize():
     call("spk_synchronize")
+
+
+def release_memory():
+    """Gives the freed device memory that the library keeps back to the device,
+    for other allocators of the process."""
+    call("spk_release_memory")
 
 
 def device_info():

@@ -136,6 +136,7 @@ _SIGS = {
     "spk_set_sweep_wait": ([C.c_uint64], None),
     "spk_malloc": ([C.POINTER(vp), C.c_size_t], None),
     "spk_free": ([vp], None),
+    "spk_release_memory": ([], None),
     "spk_memcpy_htod": ([vp, vp, C.c_size_t], None),
     "spk_memcpy_dtoh": ([vp, vp, C.c_size_t], None),
     "spk_memcpy_dtod": ([vp, vp, C.c_size_t], None),

@@ -470,6 +470,13 @@ spk_status spk_free(void* dptr) {
   });
 }
 
+spk_status spk_release_memory(void) {
+  return guarded([&] {
+    ctx();
+    pool().drain();
+  });
+}
+
 spk_status spk_memcpy_htod(void* dst, const void* src, size_t bytes) {
   return guarded([&] {
     SPK_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream()));

@@ -157,3 +157,24 @@ def test_a_block_given_back_by_hipfree(spk, nbytes):
             assert (v.numpy() == k).all()
         spans = sorted((v.ptr.value, v.ptr.value + nbytes) for v in vs)
         assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
+
+
+def test_release_memory(spk):
+    """What the pool keeps goes back to the device; what is in use stays."""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so")
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+    keep = spk.DeviceVector.from_numpy(np.arange(1 << 20, dtype=np.float64))
+    big = [spk.DeviceVector.zeros(1 << 24) for _ in range(8)]  # 1 GiB
+    del big
+    spk.synchronize()
+    before = free()
+    spk.release_memory()
+    assert free() - before >= 1 << 30
+    spk.release_memory()  # nothing left to give
+    assert np.array_equal(keep.numpy(), np.arange(1 << 20, dtype=np.float64))
+    assert (spk.DeviceVector.from_numpy(np.full(1 << 20, 2.0)).numpy() == 2.0).all()
