@@ -537,18 +537,25 @@ struct spk_batch_s {
   DevBuf<int32_t> iters, outer, conv;
   DevBuf<double> relres;
   spk_batch_tuning tuning{512, 2, kSmallSystem, 0};
-  // The launch shape until a caller sets or tunes another, by the largest
-  // system: a pass over its rows is a few loads per lane at 512 threads up to
-  // kSmallSystem rows, two workgroups a CU; the largest system's solve is the
-  // whole solve's tail, so beyond that it gets 1,024 threads.  p sits in LDS
-  // in both.  (512, 2) / (1024, 1) / 256 threads and p in HBM, ms: 256
-  // systems of 12^2-30^2 0.42 / 0.51 / 0.56, 4,096 of 12^2-40^2 3.4 / 5.9 /
-  // 4.3, 256 of 32^2-96^2 6.4 / 4.75 / 12.9, 256 of 96^2-200^2 79 / 59 / 138;
-  // FP64, 256 of 32^2-96^2: 12.0 / 8.3 / 15.7.
-  static constexpr int kSmallSystem = 2048;
-  static spk_batch_tuning default_tuning(int64_t max_rows) {
-    if (max_rows <= kSmallSystem) return {512, 2, kSmallSystem, 0};
-    return {1024, 1, 16384, 0};
+  // The launch shape until a caller sets or tunes another.  A batch whose
+  // largest system is more than a CU's share of the rows ends with that system
+  // alone: it gets 1,024 threads.  Otherwise a pass over a system's rows is to
+  // be a few loads per lane: 1,024 threads for 1,024 rows on average where some
+  // have more than kSmallSystem, 256 up to kTinySystem, else 512, two
+  // workgroups a CU.  p sits in LDS.  (256, 2) with p in HBM / (256, 2) /
+  // (512, 2) / (1024, 1), ms, FP32: 20,000 systems of 8^2 1.27 / 1.19 / 1.50 /
+  // 3.46, 4,096 of 16^2 and one of 50^2 0.39 / 0.37 / 0.42 / 0.85, 2,000 of
+  // 12^2-40^2 and one of 60^2 0.44 / 0.40 / 0.36 / 0.55, 400 of these and it
+  // 0.33 / 0.32 / 0.24 / 0.19, 4,096 of 12^2-40^2 4.35 / 3.66 / 3.42 / 5.98,
+  // 256 of 32^2-96^2 14.1 / 14.0 / 8.4 / 5.3; FP64 16.6 / 16.7 / 14.2 / 9.1.
+  static constexpr int kSmallSystem = 2048, kTinySystem = 320;
+  static spk_batch_tuning default_tuning(int64_t max_rows, int64_t total, int64_t systems) {
+    const int64_t mean = total / std::max<int64_t>(systems, 1);
+    if (max_rows > kSmallSystem &&
+        (mean >= kSmallSystem / 2 || max_rows * ctx().num_cus > total))
+      return {1024, 1, 16384, 0};
+    if (mean <= kTinySystem) return {256, 2, kSmallSystem, 0};
+    return {512, 2, kSmallSystem, 0};
   }
   // captured graphs, keyed by (b, x, config, tuning, precision)
   struct Key {
@@ -579,7 +586,7 @@ struct spk_batch_s {
       max_rows = std::max(max_rows, h_row[(size_t)k + 1] - h_row[(size_t)k]);
     SPK_REQUIRE(max_rows < ((int64_t)1 << 29), SPK_INVALID_ARGUMENT,
                 "a system of the batch holds 2^29 rows or more");
-    tuning = default_tuning(max_rows);
+    tuning = default_tuning(max_rows, total, K);
     sys_row.alloc((size_t)K + 1);
     SPK_HIP_TRY(hipMemcpyAsync(sys_row.p, h_row.data(), (K + 1) * 8,
                                hipMemcpyHostToDevice, s));

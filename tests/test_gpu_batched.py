@@ -246,3 +246,50 @@ def test_wide_band_system_keeps_32_bit_columns(O, spk):
                           max_iterations=20000, left="jacobi")
             assert abs(it[k] - sr.computed_iterations) <= 2, k
             assert np.linalg.norm(xk - xr) <= 1e-6 * np.linalg.norm(xr)
+
+
+def _poissons(spk, sides):
+    """Systems side by side: 5-point Laplacians of side^2 rows, diagonal 4.5."""
+    r, c, ro = [], [], [0]
+    for s in sides:
+        i = ro[-1] + np.arange(s * s).reshape(s, s)
+        for p, q in ((i, i), (i[1:], i[:-1]), (i[:-1], i[1:]), (i[:, 1:], i[:, :-1]),
+                     (i[:, :-1], i[:, 1:])):
+            r.append(p.ravel())
+            c.append(q.ravel())
+        ro.append(ro[-1] + s * s)
+    r, c = np.concatenate(r), np.concatenate(c)
+    at = np.lexsort((c, r))
+    r, c = r[at], c[at]
+    rp = np.zeros(ro[-1] + 1, np.int64)
+    np.cumsum(np.bincount(r, minlength=ro[-1]), out=rp[1:])
+    v = np.where(r == c, 4.5, -1.0)
+    A = spk.CsrMatrix.from_host(ro[-1], ro[-1], rp, c, v)
+    return spk.BatchedSystems.from_blocks(A, ro), (r, c, v, rp)
+
+
+@pytest.mark.parametrize("sides,shape", [
+    ([8] * 2000, (256, 2, 2048)),              # tiny systems
+    ([17] * 300, (256, 2, 2048)),
+    ([18] * 300, (512, 2, 2048)),              # 324 rows on average
+    ([45] * 40, (512, 2, 2048)),               # 2,025 rows
+    ([46] * 40, (1024, 1, 16384)),             # 2,116
+    ([8] * 12000 + [50], (256, 2, 2048)),      # one large system among tiny ones
+    ([30] * 800 + [50], (512, 2, 2048)),       # among small ones
+    ([30] * 100 + [50], (1024, 1, 16384)),     # it ends last
+    ([8] * 2000 + [130], (1024, 1, 16384)),    # and does not fit LDS in FP64
+])
+def test_default_launch_shape(spk, sides, shape):
+    print("batch", len(sides), max(sides), flush=True)
+    B, (r, c, v, rp) = _poissons(spk, sides)
+    assert B.tuning == shape
+    b = spk.uniform_pm1(4, B.total_rows)
+    x = spk.DeviceVector.zeros(B.total_rows)
+    ro = B.row_offsets()
+    for prec in (spk.F32, spk.F64):
+        s = B.solve(spk.BatchConfig(1e-9, 1e-4, 30, 5000, prec), b, x)
+        assert s["converged"] == len(sides)
+        bh, xh = b.numpy(), x.numpy()
+        res = bh - np.add.reduceat(v * xh[c], rp[:-1])
+        rel = np.sqrt(np.add.reduceat(res * res, ro[:-1]) / np.add.reduceat(bh * bh, ro[:-1]))
+        assert rel.max() < 1e-9
