@@ -258,7 +258,7 @@ struct EntryRows {
 #pragma unroll
     for (int k = 0; k < 5; ++k) own[k] = row[64 * k];
 #pragma unroll
-    for (int k = 1; k < 5; ++k) d = own[k] == (int32_t)i ? k : d;
+    for (int k = 4; k >= 0; --k) d = own[k] == (int32_t)i ? k : d;  // the first
 #pragma unroll
     for (int s = 0; s < kO; ++s) {
       const int k = s - 4 + d;  // at most 8

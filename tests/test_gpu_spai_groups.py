@@ -102,3 +102,41 @@ def test_rejections_keep_their_order(spk):
                        ([ok, wide, bad], "square matrix")):
         with pytest.raises(spk.InvalidArgument, match=what):
             model.train(mats, epochs=1, learning_rate=1e-3, batch_matrices=2)
+
+
+def _merged_loss(rp, ci, v, m):
+    """The loss of M's values m on A's entries, rows merged list by list (a
+    repeated column is met once per entry)."""
+    n, total = len(rp) - 1, 0.0
+    for i in range(n):
+        heads = [[int(rp[ci[p]]), int(rp[ci[p] + 1]), m[p]] for p in range(rp[i], rp[i + 1])]
+        while any(h[0] < h[1] for h in heads):
+            c = min(ci[h[0]] for h in heads if h[0] < h[1])
+            met = [h for h in heads if h[0] < h[1] and ci[h[0]] == c]
+            res = (1.0 if c == i else 0.0) - sum(h[2] * v[h[0]] for h in met)
+            total += res * res
+            for h in met:
+                h[0] += 1
+    return total / n
+
+
+def test_a_repeated_diagonal_has_the_same_slots_in_training(spk):
+    """Training and prediction read their rows in two forms; both take the
+    first of two diagonal entries as the row's."""
+    A = band(150, 9, keep=1.0)
+    rp, ci, v = [0], [], []
+    for i in range(150):
+        for p in range(A.indptr[i], A.indptr[i + 1]):
+            again = A.indices[p] == i and i % 7 == 3 and A.indptr[i + 1] - p < 5
+            ci += [A.indices[p]] * (2 if again else 1)
+            v += [A.data[p], 0.75 * A.data[p]][:2 if again else 1]
+        rp.append(len(ci))
+    rp, ci, v = np.array(rp), np.array(ci), np.array(v)
+    Ad = spk.CsrMatrix.from_host(150, 150, rp, ci, v)
+    model = spk.SpaiModel(4)
+    model.params = rand_params(5)
+    m = model.predict(Ad).download()[2]
+    loss, _ = model.loss_grad(Ad)
+    # the same FP64 values merged in the same order, but for the sum's order
+    ref = _merged_loss(rp, ci, v, m)
+    assert abs(loss - ref) <= 1e-12 * ref
