@@ -91,9 +91,15 @@ struct spk_csr_s {
   spk::DevBuf<int32_t> pat_len;  // [pat_count]
   spk::DevBuf<double> pat_v64;   // [pat_count][max_len]
   spk::DevBuf<float> pat_v32;
+  // From where their kernel is the faster one, by the bytes of the entries it
+  // need not read: 5 points 363^2 FP64 (7.9 MB) 4.27 us with them, 3.94 without,
+  // 400^2 (9.6) 4.28 / 4.90, FP32 400^2 (6.4) 4.39 / 4.17, 512^2 (10.5) 4.27 /
+  // 4.34; 7 points 51^3 FP64 (10.9) 4.41 / 4.44, FP32 (7.3) 4.32 / 4.05.
+  static constexpr int64_t kPatMinBytes = 9 << 20;
   template <typename T>
   bool patterned() const {
-    return pat_count > 0 && !(std::is_same<T, float>::value && half32);
+    return pat_count > 0 && nnz * (int64_t)(sizeof(T) + 4) >= kPatMinBytes &&
+           !(std::is_same<T, float>::value && half32);
   }
   std::vector<int32_t> h_rp;  // host copy of the row offsets
   // Column panels (empty: none).  Panel p holds the entries with columns in
@@ -562,8 +568,8 @@ constexpr int kPatMaxLen = 15;    // entries a row: the row kernel sums such
 constexpr int kPatMax = 255;      // lists a store may have
 constexpr int kPatMaxEntries = 1024;  // and their entries: 12 KB of LDS
 // Below, the row kernel is as fast (its launch and load chain, not its bytes,
-// take the time: 134,784 rows 7-point 4.9 us here with four rows a thread,
-// 5.1 there).
+// take the time), and lists are not looked for; beyond, the entries decide
+// (spk_csr_s::patterned).
 constexpr int64_t kPatMinRows = 1 << 17;
 constexpr int kXcds = 8;
 // Rows a thread: two (262,144 rows 7-point 3.6 us against 5.1 with four,
