@@ -178,3 +178,39 @@ def test_release_memory(spk):
     spk.release_memory()  # nothing left to give
     assert np.array_equal(keep.numpy(), np.arange(1 << 20, dtype=np.float64))
     assert (spk.DeviceVector.from_numpy(np.full(1 << 20, 2.0)).numpy() == 2.0).all()
+
+
+def test_freed_while_another_stream_reads(spk):
+    """A vector freed while work on a second stream is still to read it: what
+    the next owners of its block write does not reach that work."""
+    import ctypes as C
+
+    from sparkit_amd import _lib
+    hip = C.CDLL("libamdhip64.so")
+    stream = C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(stream), 1) == 0  # non-blocking
+    A = spk.poisson_3d(128)
+    u, w = spk.uniform_pm1(1, A.nrows), spk.DeviceVector.zeros(A.nrows)
+    n = 5000
+    for k in range(5):
+        v = spk.DeviceVector.from_numpy(np.full(n, 7.0 + k))
+        out = spk.DeviceVector.zeros(n)
+        spk.synchronize()
+        _lib.call("spk_set_stream", stream)
+        try:
+            for _ in range(300):  # some milliseconds of products, then the read
+                A.spmv(u, w)
+            out.copy_from(v)
+        finally:
+            _lib.call("spk_set_stream", None)
+        at = v.ptr.value
+        del v
+        met = False
+        for _ in range(40):  # until the block comes back, as soon as it may
+            y = spk.DeviceVector.zeros(n)
+            met = met or y.ptr.value == at
+            del y
+        assert met
+        assert hip.hipStreamSynchronize(stream) == 0
+        assert (out.numpy() == 7.0 + k).all()
+    assert hip.hipStreamDestroy(stream) == 0

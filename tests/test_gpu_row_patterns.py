@@ -192,3 +192,31 @@ def test_rectangular_and_small(spk):
     y = spk.DeviceVector.zeros(A.nrows)
     R.spmv(spk.DeviceVector.from_numpy(x), y)
     assert np.array_equal(y.numpy(), _reference(A, x[:A.ncols]))
+
+
+@pytest.mark.parametrize("solver", ["cg", "bicg", "bicgstab", "cgs", "minres", "qmr"])
+@pytest.mark.parametrize("left", [None, "jacobi"])
+def test_solvers(O, spk, solver, left):
+    """Every solver's products, transposed ones too, and the sums in their
+    epilogues, over stores with row patterns; CG at a size whose rows do not
+    fit the registers."""
+    print("patterned", solver, left, flush=True)
+    A = (O.poisson_3d(90, 80, 75) if solver in ("cg", "minres")
+         else O.convdiff_3d(61, 63, 67, 1.0, 0.3, 0.2, 0.1))
+    b = O.uniform_pm1(9, A.nrows)
+    Ad = spk.CsrMatrix.from_oracle(A)
+    bd, x = spk.DeviceVector.from_numpy(b), spk.DeviceVector.zeros(A.nrows)
+    M = spk.jacobi(Ad) if left else spk.identity
+    steps = 8
+    if solver == "cg":
+        s = spk.conjugate_gradient(bd, x, spk.CGConfig(0.0, 100, steps, True), Ad, M)
+        xr, sr = O.cg(A, b, tol=0.0, restart_iterations=100, max_iterations=steps, left=left)
+    else:
+        mats = (Ad, Ad.transpose()) if solver in ("bicg", "qmr") else (Ad,)
+        s = getattr(spk, solver)(bd, x, spk.BicgstabConfig(0.0, steps, True), *mats, M)
+        xr, sr = getattr(O, solver)(A, b, tol=0.0, max_iterations=steps, left=left)
+    assert s.computed_iterations == sr.computed_iterations
+    # the dot products in another order (2^-53 a term), eight steps of a
+    # well-conditioned start
+    assert np.linalg.norm(x.numpy() - xr) <= 1e-11 * np.linalg.norm(xr)
+    assert np.allclose(s.iteration_residuals, sr.iteration_residuals, rtol=1e-11, atol=0)
