@@ -416,23 +416,26 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
   // 27 points 20^3 1.84 / 0.4).
   const bool long_rows = max_len > kTriFactorLen || (h[0] & 12) != 0;
   DevBuf<int32_t> lvl;
-  int count[2];
-  find_levels(lvl, count, long_rows || (h[4] > kBatch && nnz <= (1 << 20)));
-  levels_l = count[0];
-  levels_u = count[1];
-  choose_sweep(SPK_ILU_AUTO);
-  const bool tiles = sweep == kTiles;
-  if (tiles) tri_layouts(P, lvl.p, lower, upper);
+  bool on_host = long_rows || (h[4] > kBatch && nnz <= (1 << 20)), tiles, tiled;
+  auto lay_out = [&] {
+    int count[2];
+    find_levels(lvl, count, on_host);
+    levels_l = count[0];
+    levels_u = count[1];
+    choose_sweep(SPK_ILU_AUTO);
+    tiles = sweep == kTiles;
+    if (tiles) tri_layouts(P, lvl.p, lower, upper);
+  };
+  lay_out();
   const double* in = ordered.p ? ordered.p : A.v64.p;
   // A tile works on one step at a time, the launches on a whole level: rows of
   // more than four entries on a side, a row's elimination being hundreds of
   // loads one after the other, take the tiles where those have fewer steps by
   // a third.  Set-up in tiles / by levels: 20 random entries a row, 20,000 rows
-  // (54 levels) 28.8 / 13.4 ms, 27 points 20^3 natural 15.3 / 13.2, 40^3
+  // (54 levels) 28.8 / 13.1 ms, 27 points 20^3 natural 15.3 / 13.4, 40^3
   // natural 29 / 39, 64^3 natural 47 / 79.
-  bool tiled = tiles && !long_rows &&
-               (h[4] <= kBatch ||
-                2 * (int64_t)levels_l * lower.tiles > 3 * (int64_t)lower.nsteps);
+  tiled = tiles && !long_rows &&
+          (h[4] <= kBatch || 2 * (int64_t)levels_l * lower.tiles > 3 * (int64_t)lower.nsteps);
   for (;;) {
     if (tiled)
       tri_factor(P, lower, in, w, modified, h[1], h[4], ticket.p, sweep_error.p);
@@ -440,7 +443,10 @@ void spk_precond_s::factor(const spk_csr_s& A, bool modified) {
       factor_by_levels(in, modified, lvl.p);
     if (tiles) tri_values(P, w.p, lower, upper);
     if (!tiled || !sweep_errors()) break;
-    tiled = false;  // a wait expired: again, without waits
+    // a wait expired: again, without waits and with nothing that came of them
+    tiled = false;
+    on_host = true;
+    lay_out();
   }
   set_schedule(SPK_ILU_AUTO, lvl.p);
   SPK_HIP_TRY(hipStreamSynchronize(s));

@@ -998,6 +998,7 @@ void tri_layouts(const TriPattern& P, const int32_t* lvl, TriTiles& lower, TriTi
   TriBuild B{};
   B.tiles = (int)m;
   for (int k = 0; k < 2; ++k) {
+    T[k]->v64.release();  // of another layout
     T[k]->rows.alloc((size_t)P.n);
     T[k]->first.alloc(m + 1);
     B.lvl[k] = lvl + k * P.n;
