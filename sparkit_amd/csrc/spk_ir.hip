@@ -391,6 +391,7 @@ void cg_reliable(spk_csr_s* A, spk_precond_s* M, const spk_ir_config* cfg,
             h.rz = 1.0;
             st.upload(h);
             restart(true);
+            ran = h.iters;
             continue;
           }
           ran = h.iters;

@@ -68,6 +68,24 @@ def test_reliable_cg(spk, hindered):
     assert abs(a - h) <= 0.1 * a
 
 
+def test_reliable_cg_budget(spk):
+    """A budget of more than one launch's 4,096 steps, undisturbed and lost: it
+    is charged with the steps that were kept."""
+    from sparkit_amd import _lib
+    A = spk.poisson_2d(300, 200, 0.05)
+    b, J = spk.uniform_pm1(3, A.nrows), spk.jacobi(A)
+    cfg = spk.IrConfig(1e-300, 1, 1e-300, 0, 5000, spk.IR_CG_RELIABLE)  # no update due
+    for polls in (0, 1):
+        _lib.call("spk_set_exchange_polls", polls)
+        try:
+            x = spk.DeviceVector.zeros(A.nrows)
+            s = spk.ir_solve(b, x, cfg, A, J)
+        finally:
+            _lib.call("spk_set_exchange_polls", 0)
+        assert s.inner_iterations == 5000 and not s.converged
+        assert spk.true_relres(A, b, x) < 1e-5  # what FP32 reaches
+
+
 @pytest.mark.parametrize("precond", ["none", "jacobi", "ilu0", "inner cg"])
 def test_gmres(spk, hindered, precond):
     """An inner CG shares the exchange with the outer solver's steps."""
